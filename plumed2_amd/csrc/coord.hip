@@ -92,6 +92,7 @@ struct p2a_coord {
   std::vector<hipEvent_t> ev_pool;
   std::vector<std::pair<hipEvent_t, hipEvent_t>> pending;
   bool has_duplicates = false;  // an absolute index listed twice in one group
+  bool distinct = true;         // no absolute index listed twice in the two groups together
   p2a::PbcHost pbc;
   p2a::PbcArg pbc_stage;
   p2a::DBuf<p2a::PbcArg> pbc_dev;
@@ -115,6 +116,7 @@ struct p2a_coord {
   p2a::DBuf<int> nl_count, nl_start, nl_nbr, nl_cell;
   p2a::DBuf<long long> nl_total;
   bool nl_valid = false;
+  int64_t nl_entries = 0;  // partners listed in nl_nbr
   // per-atom coordination numbers: weights per requested atom; row and
   // environment indices for the FP64 path
   p2a::DBuf<float> wreq;
@@ -556,10 +558,9 @@ static int run_fallback(p2a_coord* c, const double* box9, const double* pos_dev,
     hipLaunchKernelGGL(k_pairmode, dim3(std::max(nblocks, 1)), dim3(256), 0, s, nA, c->spec.pbc, P, c->spec.sw,
                        pos_dev, c->abs_dev.p, deriv_dev, c->partial.p);
   } else {
-    nblocks = grid1(c->natoms, 256);
-    if ((rc = c->partial.reserve(8 * (size_t)std::max(nblocks, 1)))) return rc;
-    hipLaunchKernelGGL(k_allpairs, dim3(std::max(nblocks, 1)), dim3(256), 0, s, nA, nB, c->spec.pbc, P, c->spec.sw,
-                       pos_dev, c->abs_dev.p, deriv_dev, c->partial.p);
+    if ((rc = c->partial.reserve(8 * (size_t)kMaxBlocks64))) return rc;
+    nblocks = launch_pairs64(s, nA, nB, c->spec.pbc, P, c->spec.sw, pos_dev,
+                             c->distinct ? nullptr : (const long long*)c->abs_dev.p, deriv_dev, c->partial.p);
   }
   if ((rc = launch_check("fp64 pair kernel"))) return rc;
   if ((rc = reduce_partials(c, std::max(nblocks, 1), value_dev, virial_dev))) return rc;
@@ -644,8 +645,8 @@ static int run_fallback_nl(p2a_coord* c, bool build, const double* box9, const d
         if ((rc = c->nl_cell.reserve(3 * (size_t)natoms))) return rc;
         hipLaunchKernelGGL(k_nl_cells, dim3(grid1(natoms, 256)), dim3(256), 0, s, natoms, G, pos_dev, c->nl_cell.p);
       }
-      hipLaunchKernelGGL(k_nl_atoms<0>, dim3(grid1(natoms, 256)), dim3(256), 0, s, nA, nB, mode, use_pbc, P, cut2, G,
-                         pos_dev, (const int*)c->nl_cell.p, c->nl_count.p, (const int*)nullptr, (int*)nullptr);
+      launch_nl_atoms<0>(s, nA, nB, mode == P2A_NL_CELLS, use_pbc, P, cut2, G, pos_dev, c->nl_cell.p, c->nl_count.p,
+                         nullptr, nullptr);
       hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(1024), 0, s, natoms, (const int*)c->nl_count.p, c->nl_start.p,
                          c->nl_total.p);
       long long total = 0;
@@ -654,8 +655,9 @@ static int run_fallback_nl(p2a_coord* c, bool build, const double* box9, const d
       std::memcpy(&total, c->host_ro + 40, sizeof(total));
       if (total > INT32_MAX) return fail(P2A_ERR_UNSUPPORTED, "neighbour list too long for the FP64 path");
       if ((rc = c->nl_nbr.reserve(std::max<long long>(total, 1)))) return rc;
-      hipLaunchKernelGGL(k_nl_atoms<1>, dim3(grid1(natoms, 256)), dim3(256), 0, s, nA, nB, mode, use_pbc, P, cut2, G,
-                         pos_dev, (const int*)c->nl_cell.p, (int*)nullptr, (const int*)c->nl_start.p, c->nl_nbr.p);
+      c->nl_entries = total;
+      launch_nl_atoms<1>(s, nA, nB, mode == P2A_NL_CELLS, use_pbc, P, cut2, G, pos_dev, c->nl_cell.p, nullptr,
+                         c->nl_start.p, c->nl_nbr.p);
     }
     if ((rc = launch_check("FP64 neighbour list"))) return rc;
     c->nl_valid = true;
@@ -669,11 +671,10 @@ static int run_fallback_nl(p2a_coord* c, bool build, const double* box9, const d
     hipLaunchKernelGGL(k_pairmode, dim3(std::max(nblocks, 1)), dim3(256), 0, s, nA, c->spec.pbc, P, c->spec.sw,
                        pos_dev, c->abs_dev.p, deriv_dev, c->partial.p, (const int*)c->nl_count.p);
   } else {
-    nblocks = grid1(natoms, 256);
-    if ((rc = c->partial.reserve(8 * (size_t)std::max(nblocks, 1)))) return rc;
-    hipLaunchKernelGGL(k_allpairs, dim3(std::max(nblocks, 1)), dim3(256), 0, s, nA, nB, c->spec.pbc, P, c->spec.sw,
-                       pos_dev, c->abs_dev.p, deriv_dev, c->partial.p, (const int*)c->nl_start.p,
-                       (const int*)c->nl_nbr.p);
+    if ((rc = c->partial.reserve(8 * (size_t)kMaxListBlocks64))) return rc;
+    nblocks = launch_pairs64(s, nA, nB, c->spec.pbc, P, c->spec.sw, pos_dev,
+                             c->distinct ? nullptr : (const long long*)c->abs_dev.p, deriv_dev, c->partial.p,
+                             c->nl_start.p, c->nl_nbr.p, c->nl_entries);
   }
   if ((rc = launch_check("fp64 pair kernel"))) return rc;
   if ((rc = reduce_partials(c, std::max(nblocks, 1), value_dev, virial_dev))) return rc;
@@ -890,21 +891,24 @@ static void collect_profile(p2a_coord* c) {
 // matrix element of (rows[k], j), ContactMatrix::calculateWeight
 // (src/adjmat/ContactMatrix.h:95-121): nothing when |r|^2 < DBL_EPSILON (the
 // diagonal, or two atoms at one place), s(r) zeroed below DBL_EPSILON.  One
-// thread per row, FP64, environment in list order.  An index outside
-// [0, natoms) makes that row NaN instead of being read.
+// wave per row, FP64, the environment over the lanes (a row meets every
+// environment atom, so one thread per row left the chip idle for any but the
+// longest lists).  An index outside [0, natoms) makes that row NaN instead of
+// being read.
 __global__ __launch_bounds__(256) void k_cn_rows(int natoms, int nrows, const int* __restrict__ rows, int nenv,
                                                  const int* __restrict__ env, int use_pbc, PbcArg P, p2a_switch sw,
                                                  const double* __restrict__ pos, double* __restrict__ cn) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int k = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (k >= nrows) return;
   const int i = rows[k];
   if (i < 0 || i >= natoms) {
-    cn[k] = __builtin_nan("");
+    if (lane == 0) cn[k] = __builtin_nan("");
     return;
   }
   const double* xi = pos + 3 * (size_t)i;
   double sum = 0.0;
-  for (int q = 0; q < nenv; q++) {
+  for (int q = lane; q < nenv; q += WAVE) {
     const int j = env[q];
     if (j < 0 || j >= natoms) {
       sum = __builtin_nan("");
@@ -921,16 +925,16 @@ __global__ __launch_bounds__(256) void k_cn_rows(int natoms, int nrows, const in
     if (v < DBL_EPSILON) continue;
     sum += v;
   }
-  cn[k] = sum;
+  sum = wave_sum_d(sum);
+  if (lane == 0) cn[k] = sum;
 }
 
 // Scratch of the allocation-free entry point: the per-workgroup partials of
-// k_allpairs that k_finalize sums (8 doubles per 256-atom workgroup).  Each
+// k_allpairs that k_finalize sums (8 doubles for each of kMaxBlocks64).  Each
 // device holds its own copy for the life of the process; its address is
 // looked up once per device and kept in g_scratch_dev.
 constexpr int kNoAllocMaxAtoms = 1 << 18;
-constexpr int kNoAllocBlocks = kNoAllocMaxAtoms / 256;
-static __device__ __align__(256) double scratch[8 * kNoAllocBlocks];
+static __device__ __align__(256) double scratch[8 * kMaxBlocks64];
 
 constexpr int kMaxDevices = 64;
 static std::mutex g_scratch_mu;
@@ -992,11 +996,19 @@ int p2a_coord_create(p2a_coord** out, int device, const p2a_coord_spec* spec) {
   c->abs.resize(c->natoms);
   for (int64_t i = 0; i < spec->na; i++) c->abs[i] = spec->groupa[i];
   for (int64_t i = 0; i < spec->nb; i++) c->abs[spec->na + i] = spec->groupb[i];
+  std::vector<int64_t> sorted[2];
   for (int gi = 0; gi < 2; gi++) {
-    std::vector<int64_t> v(gi == 0 ? spec->groupa : spec->groupb,
-                           (gi == 0 ? spec->groupa : spec->groupb) + (gi == 0 ? spec->na : spec->nb));
-    std::sort(v.begin(), v.end());
+    const int64_t* g = gi == 0 ? spec->groupa : spec->groupb;
+    std::vector<int64_t>& v = sorted[gi];
+    v.assign(g, g + (gi == 0 ? spec->na : spec->nb));
+    if (!std::is_sorted(v.begin(), v.end())) std::sort(v.begin(), v.end());
     if (std::adjacent_find(v.begin(), v.end()) != v.end()) c->has_duplicates = true;
+  }
+  c->distinct = !c->has_duplicates;
+  for (auto a = sorted[0].begin(), b = sorted[1].begin(); c->distinct && a != sorted[0].end() && b != sorted[1].end();) {
+    if (*a == *b) c->distinct = false;
+    else if (*a < *b) ++a;
+    else ++b;
   }
   int ncu = 0;
   if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && ncu > 0)
@@ -1093,7 +1105,7 @@ int p2a_coord_calculate_noalloc(void* stream, const p2a_switch* sw, const double
   if (nb < 0) return fail(P2A_ERR_ARG, "GROUPB cannot have a negative size");
   if (na + nb > kNoAllocMaxAtoms)
     return fail(P2A_ERR_ARG, "p2a_coord_calculate_noalloc handles at most " + std::to_string(kNoAllocMaxAtoms) +
-                                 " atoms (its scratch holds 8 doubles per 256 atoms)");
+                                 " atoms");
   if (use_pbc && !box9) return fail(P2A_ERR_ARG, "box is required with periodic boundaries");
   int dev = 0;
   P2A_HIP(hipGetDevice(&dev));
@@ -1113,12 +1125,10 @@ int p2a_coord_calculate_noalloc(void* stream, const p2a_switch* sw, const double
     if (h.type == 0) return fail(P2A_ERR_ARG, "the box is singular");
     fill_pbc_arg(h, P);
   }
-  const int natoms = (int)(na + nb);
-  const int nblocks = grid1(natoms, 256);
   hipStream_t s = (hipStream_t)stream;
   // every workgroup writes its 8 partials, so nothing in scratch needs clearing
-  hipLaunchKernelGGL(k_allpairs, dim3(nblocks), dim3(256), 0, s, (int)na, (int)nb, use_pbc ? 1 : 0, P, *sw, pos_dev,
-                     (const long long*)absidx_dev, deriv_dev, part);
+  const int nblocks = launch_pairs64(s, (int)na, (int)nb, use_pbc ? 1 : 0, P, *sw, pos_dev,
+                                     (const long long*)absidx_dev, deriv_dev, part);
   hipLaunchKernelGGL(k_finalize, dim3(1), dim3(128), 0, s, nblocks, (const double*)part, value_dev, virial_dev,
                      (double*)nullptr);
   return launch_check("p2a_coord_calculate_noalloc");
@@ -1260,7 +1270,7 @@ int p2a_coord_rows_device(p2a_coord* c, int64_t step, const double* box9, const 
     P2A_HIP(hipMemcpyAsync(c->cn_rows.p, r.data(), na * sizeof(int), hipMemcpyHostToDevice, c->stream));
     P2A_HIP(hipMemcpyAsync(c->cn_env.p, e.data(), nenv * sizeof(int), hipMemcpyHostToDevice, c->stream));
     if ((rc = upload_pbc(c, box9))) return rc;
-    hipLaunchKernelGGL(k_cn_rows, dim3(grid1((size_t)na, 256)), dim3(256), 0, c->stream, c->natoms, na,
+    hipLaunchKernelGGL(k_cn_rows, dim3(grid1((size_t)na, 4)), dim3(256), 0, c->stream, c->natoms, na,
                        (const int*)c->cn_rows.p, nenv, (const int*)c->cn_env.p, c->spec.pbc ? 1 : 0, c->pbc_stage,
                        c->spec.sw, pos_dev, rows_dev);
     // the host vectors are read by the copies above before they return
@@ -1288,7 +1298,7 @@ int p2a_coordination_numbers_device(void* stream, const p2a_switch* sw, const do
     pbc_setup(box9, h);
     fill_pbc_arg(h, P);
   }
-  hipLaunchKernelGGL(k_cn_rows, dim3(grid1((size_t)nrows, 256)), dim3(256), 0, (hipStream_t)stream, (int)natoms,
+  hipLaunchKernelGGL(k_cn_rows, dim3(grid1((size_t)nrows, 4)), dim3(256), 0, (hipStream_t)stream, (int)natoms,
                      (int)nrows, rows_dev, (int)nenv, env_dev, use_pbc ? 1 : 0, P, *sw, pos_dev, cn_dev);
   return launch_check("coordination numbers");
 }

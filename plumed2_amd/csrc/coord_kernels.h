@@ -2084,81 +2084,252 @@ __global__ __launch_bounds__(256) void k_sys_reduce(int nsys, const int* __restr
 // partners are every atom of the other group (two groups) or of the group,
 // or, with a neighbour list (nbr_start non-null), the atoms nbr[nbr_start[i]
 // .. nbr_start[i+1]) listed for atom i in both directions.
-__global__ void k_allpairs(int nA, int nB, int use_pbc, PbcArg P, p2a_switch sw, const double* __restrict__ pos,
-                           const long long* __restrict__ absidx, double* __restrict__ deriv,
-                           double* __restrict__ partial, const int* __restrict__ nbr_start = nullptr,
-                           const int* __restrict__ nbr = nullptr) {
+
+// minimum image of d = x_q - x_p: PBC 0 none, 1 orthorhombic, 2 any cell
+template <int PBC>
+__device__ __forceinline__ void wrap64(const PbcArg& P, double* d) {
 #pragma clang fp contract(off)
-  const int natoms = nA + nB;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  double cv = 0, v[6] = {0, 0, 0, 0, 0, 0}, f[3] = {0, 0, 0};
-  double np = 0;
-  if (i < natoms) {
-    const bool two = nB > 0;
-    int j0, j1;
-    if (nbr_start) {
-      j0 = nbr_start[i];
-      j1 = nbr_start[i + 1];
-    } else if (two) {
-      if (i < nA) { j0 = nA; j1 = natoms; } else { j0 = 0; j1 = nA; }
-    } else {
-      j0 = 0;
-      j1 = nA;
-    }
-    const double* xi = pos + 3 * (size_t)i;
-    for (int jj = j0; jj < j1; jj++) {
-      const int j = nbr_start ? nbr[jj] : jj;
-      // absidx null: the requested atoms are distinct atoms
-      if (j == i || (absidx && absidx[i] == absidx[j])) continue;
-      const double* xj = pos + 3 * (size_t)j;
-      // the pair is measured once, as the reference lists it: p -> q with p
-      // in GROUPA (two groups) or p < q, d = Pbc::distance(x_p, x_q); atom
-      // i is p ("own") or q.  Measured from q, a pair at half a cell could
-      // take another of its tied images.
-      const bool own = two ? (i < nA) : (i < j);
-      const double* xp = own ? xi : xj;
-      const double* xq = own ? xj : xi;
-      double d[3];
-      if (use_pbc) pbc_distance(P, xp, xq, d);
-      else { d[0] = xq[0] - xp[0]; d[1] = xq[1] - xp[1]; d[2] = xq[2] - xp[2]; }
-      double r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
-      double df;
-      double s = switch_calc_sqr(sw, r2, df);
-      // CoordinationBase: deriv[p] -= df*d, deriv[q] += df*d
-      const double g = own ? -df : df;
-      f[0] += g * d[0];
-      f[1] += g * d[1];
-      f[2] += g * d[2];
-      if (own) {
-        cv += s;
-        if (switch_inside(sw, r2)) np += 1;
-        v[0] -= df * d[0] * d[0];
-        v[1] -= df * d[0] * d[1];
-        v[2] -= df * d[0] * d[2];
-        v[3] -= df * d[1] * d[1];
-        v[4] -= df * d[1] * d[2];
-        v[5] -= df * d[2] * d[2];
-      }
-    }
-    deriv[3 * (size_t)i + 0] = f[0];
-    deriv[3 * (size_t)i + 1] = f[1];
-    deriv[3 * (size_t)i + 2] = f[2];
+  if constexpr (PBC == 1) {
+    for (int i = 0; i < 3; i++) d[i] = pbc1(d[i] * P.inv[4 * i]) * P.box[4 * i];
+  } else if constexpr (PBC == 2) {
+    const double zero[3] = {0.0, 0.0, 0.0};
+    const double v[3] = {d[0], d[1], d[2]};
+    pbc_distance(P, zero, v, d);
   }
-  // block partials: cv, -virial terms are stored as +sum g (x) d for k_finalize
-  double r[8] = {cv, -v[0], -v[1], -v[2], -v[3], -v[4], -v[5], np};
-  const int lane = threadIdx.x & 63;
-  for (int q = 0; q < 8; q++) r[q] = wave_sum(r[q]);
+}
+
+// s and dfunc: SWK = P > 0 for fixedRational<2P> (its exponents unroll), 0 any
+template <int SWK>
+__device__ __forceinline__ double switch64(const p2a_switch& sw, double d2, double& df) {
+#pragma clang fp contract(off)
+  if constexpr (SWK > 0) {
+    // switch_calc_sqr of RATIONAL_FIXED, for d2 inside D_MAX
+    const double rdist = d2 * sw.invr0_2;
+    const double rN = ipow(rdist, SWK - 1);
+    const double r = 1.0 / (1.0 + rN * rdist);
+    double f = -SWK * rN * r * r;
+    f *= 2 * sw.invr0_2;
+    df = f * sw.stretch;
+    return r * sw.stretch + sw.shift;
+  } else {
+    return switch_calc_sqr(sw, d2, df);
+  }
+}
+
+struct Sum64 {
+  double cv, v[6], np;
+};
+
+// the pair (i, j) seen from atom i: f += its derivative; value, virial and
+// count when `own` (the pair is listed as i -> j)
+template <int PBC, int SWK>
+__device__ __forceinline__ void pair64(const PbcArg& P, const p2a_switch& sw, const double* xi, const double* xj,
+                                       bool own, double* f, Sum64& a) {
+#pragma clang fp contract(off)
+  // the pair is measured once, as the reference lists it: p -> q with p in
+  // GROUPA (two groups) or p < q, d = Pbc::distance(x_p, x_q); atom i is p
+  // ("own") or q.  Measured from q, a pair at half a cell could take another
+  // of its tied images.  x_j - x_i changes sign exactly.
+  double d[3] = {xj[0] - xi[0], xj[1] - xi[1], xj[2] - xi[2]};
+  if constexpr (PBC != 0) {
+    if (!own)
+      for (int k = 0; k < 3; k++) d[k] = -d[k];
+    wrap64<PBC>(P, d);
+    if (!own)
+      for (int k = 0; k < 3; k++) d[k] = -d[k];
+  }
+  const double r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+  if (SWK > 0 && !(r2 <= sw.dmax_2)) return;
+  double df;
+  const double s = switch64<SWK>(sw, r2, df);
+  // CoordinationBase: deriv[p] -= df*d, deriv[q] += df*d
+  for (int k = 0; k < 3; k++) f[k] = fma(-df, d[k], f[k]);
+  if (own) {
+    const double g[3] = {df * d[0], df * d[1], df * d[2]};
+    a.cv += s;
+    if (SWK > 0 || switch_inside(sw, r2)) a.np += 1;
+    a.v[0] = fma(g[0], d[0], a.v[0]);
+    a.v[1] = fma(g[0], d[1], a.v[1]);
+    a.v[2] = fma(g[0], d[2], a.v[2]);
+    a.v[3] = fma(g[1], d[1], a.v[3]);
+    a.v[4] = fma(g[1], d[2], a.v[4]);
+    a.v[5] = fma(g[2], d[2], a.v[5]);
+  }
+}
+
+// block partials of a 256-thread workgroup, for the final reduction
+__device__ __forceinline__ void store_partial64(const Sum64& a, double* __restrict__ partial) {
   __shared__ double red[4][8];
-  if (lane == 0)
+  double r[8] = {a.cv, a.v[0], a.v[1], a.v[2], a.v[3], a.v[4], a.v[5], a.np};
+  for (int q = 0; q < 8; q++) r[q] = wave_sum_d(r[q]);
+  if ((threadIdx.x & 63) == 0)
     for (int q = 0; q < 8; q++) red[threadIdx.x >> 6][q] = r[q];
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int q = 0; q < 8; q++) {
-      double t = 0;
-      for (int w = 0; w < (int)(blockDim.x / 64); w++) t += red[w][q];
-      partial[(size_t)blockIdx.x * 8 + q] = t;
+  if (threadIdx.x < 8) {
+    double t = 0;
+    for (int w = 0; w < 4; w++) t += red[w][threadIdx.x];
+    partial[(size_t)blockIdx.x * 8 + threadIdx.x] = t;
+  }
+}
+
+// One side of the all-pairs pass: atoms [i0, i0 + n) against [j0, j0 + m).
+struct Side64 {
+  int i0, n, j0, m;
+  int it;      // atoms a workgroup takes together (1 or kIt64); 0: one per thread
+  int blocks;  // workgroups of this side
+};
+constexpr int kIt64 = 4;
+// At most this many workgroups a launch, so that the partials of any launch
+// fit the rows of the allocation-free entry point.  With more atom groups
+// than that a workgroup takes several in turn.
+constexpr int kMaxBlocks64 = 1024;
+
+// `it` atoms against all partners, the lanes of the workgroup over the partners
+template <int PBC, int SWK, int IT>
+__device__ __forceinline__ void atoms64(const Side64& S, int g, bool two, bool own2, const PbcArg& P,
+                                        const p2a_switch& sw, const double* __restrict__ pos,
+                                        const long long* __restrict__ absidx, double* __restrict__ deriv, Sum64& a) {
+  __shared__ double sf[4][3 * IT];
+  const int ib = S.i0 + g * IT;
+  const int ni = min(IT, S.i0 + S.n - ib);
+  double xi[IT][3], f[IT][3];
+#pragma unroll
+  for (int u = 0; u < IT; u++) {
+    const int i = ib + (u < ni ? u : 0);
+    for (int k = 0; k < 3; k++) {
+      xi[u][k] = pos[3 * (size_t)i + k];
+      f[u][k] = 0.0;
     }
   }
+  for (int j = S.j0 + (int)threadIdx.x; j < S.j0 + S.m; j += 256) {
+    const double xj[3] = {pos[3 * (size_t)j], pos[3 * (size_t)j + 1], pos[3 * (size_t)j + 2]};
+#pragma unroll
+    for (int u = 0; u < IT; u++) {
+      const int i = ib + u;
+      // absidx null: the requested atoms are distinct atoms
+      if (u < ni && j != i && !(absidx && absidx[i] == absidx[j]))
+        pair64<PBC, SWK>(P, sw, xi[u], xj, two ? own2 : i < j, f[u], a);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < IT; u++)
+    for (int k = 0; k < 3; k++) {
+      const double t = wave_sum_d(f[u][k]);
+      if ((threadIdx.x & 63) == 0) sf[threadIdx.x >> 6][3 * u + k] = t;
+    }
+  __syncthreads();
+  const int t = threadIdx.x;
+  if (t < 3 * ni) deriv[3 * (size_t)ib + t] = ((sf[0][t] + sf[1][t]) + sf[2][t]) + sf[3][t];
+  __syncthreads();
+}
+
+// All pairs.  Bound by FP64 VALU issue (about 45 instructions a pair without
+// a cell): the partners of an atom go over the 256 lanes of a workgroup, so
+// that a few hundred atoms already fill the chip, and kIt64 atoms share each
+// loaded partner (24 B at a stride of 24 B: with one atom a load the L1 would
+// be the bound).  Measured, one thread per atom before -> this: 5,001 atoms
+// without a cell 3.24 ms -> 53 us; 100 x 200 atoms in a 3 nm cell 157 -> 4.7 us.
+// A side with few partners keeps one thread per atom (its partners are then
+// uniform loads), see allpairs_sides.
+template <int PBC, int SWK>
+__global__ __launch_bounds__(256) void k_allpairs(Side64 S0, Side64 S1, PbcArg P, p2a_switch sw,
+                                                  const double* __restrict__ pos,
+                                                  const long long* __restrict__ absidx, double* __restrict__ deriv,
+                                                  double* __restrict__ partial) {
+  const bool two = S1.n > 0;
+  const bool first = (int)blockIdx.x < S0.blocks;
+  const Side64 S = first ? S0 : S1;
+  const int b = first ? (int)blockIdx.x : (int)blockIdx.x - S0.blocks;
+  Sum64 a = {0.0, {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, 0.0};
+  if (S.it == 1) {
+    for (int g = b; g < S.n; g += S.blocks) atoms64<PBC, SWK, 1>(S, g, two, first, P, sw, pos, absidx, deriv, a);
+  } else if (S.it == kIt64) {
+    for (int g = b; g * kIt64 < S.n; g += S.blocks)
+      atoms64<PBC, SWK, kIt64>(S, g, two, first, P, sw, pos, absidx, deriv, a);
+  } else {
+    for (int q = b * 256 + (int)threadIdx.x; q < S.n; q += S.blocks * 256) {
+      const int i = S.i0 + q;
+      const double xi[3] = {pos[3 * (size_t)i], pos[3 * (size_t)i + 1], pos[3 * (size_t)i + 2]};
+      double f[3] = {0.0, 0.0, 0.0};
+      for (int j = S.j0; j < S.j0 + S.m; j++) {
+        if (j == i || (absidx && absidx[i] == absidx[j])) continue;
+        const double xj[3] = {pos[3 * (size_t)j], pos[3 * (size_t)j + 1], pos[3 * (size_t)j + 2]};
+        pair64<PBC, SWK>(P, sw, xi, xj, two ? first : i < j, f, a);
+      }
+      for (int k = 0; k < 3; k++) deriv[3 * (size_t)i + k] = f[k];
+    }
+  }
+  store_partial64(a, partial);
+}
+
+// One side of the list pass: atoms [i0, i0 + n), `wide`: a workgroup per
+// atom, else a wave per atom.
+struct ListSide64 {
+  int i0, n, wide, blocks;
+};
+
+// atom i against the listed partners p0, p0 + step, ...: each partner's
+// index and position are loaded ahead of the pair before it
+template <int PBC, int SWK>
+__device__ __forceinline__ void listed64(int i, int p0, int step, bool two, bool own2, const PbcArg& P,
+                                         const p2a_switch& sw, const double* __restrict__ pos,
+                                         const long long* __restrict__ absidx, const int* __restrict__ nbr, int e,
+                                         double* f, Sum64& a) {
+  const double xi[3] = {pos[3 * (size_t)i], pos[3 * (size_t)i + 1], pos[3 * (size_t)i + 2]};
+  int p = p0;
+  int j = p < e ? nbr[p] : 0;
+  int jn = p + step < e ? nbr[p + step] : 0;
+  double x[3] = {pos[3 * (size_t)j], pos[3 * (size_t)j + 1], pos[3 * (size_t)j + 2]};
+  for (; p < e; p += step) {
+    const int jc = j;
+    const double xj[3] = {x[0], x[1], x[2]};
+    j = jn;
+    for (int k = 0; k < 3; k++) x[k] = pos[3 * (size_t)j + k];
+    jn = p + 2 * step < e ? nbr[p + 2 * step] : 0;
+    if (jc != i && !(absidx && absidx[i] == absidx[jc]))
+      pair64<PBC, SWK>(P, sw, xi, xj, two ? own2 : i < jc, f, a);
+  }
+}
+
+// The pairs of a neighbour list.  A list holds tens to thousands of partners:
+// long lists (see list_side64) take a workgroup per atom, the others a wave
+// per atom.  Bound by the latency of partner index -> position, hence the
+// loads ahead.  Measured at 700 x 5,300 atoms with 3,100 / 410 partners
+// listed: one thread per atom 3.61 ms, now 22 us.
+template <int PBC, int SWK>
+__global__ __launch_bounds__(256) void k_listpairs(ListSide64 S0, ListSide64 S1, PbcArg P, p2a_switch sw,
+                                                   const double* __restrict__ pos,
+                                                   const long long* __restrict__ absidx, double* __restrict__ deriv,
+                                                   double* __restrict__ partial, const int* __restrict__ nbr_start,
+                                                   const int* __restrict__ nbr) {
+  __shared__ double sf[4][3];
+  const bool two = S1.n > 0;
+  const bool first = (int)blockIdx.x < S0.blocks;
+  const ListSide64 S = first ? S0 : S1;
+  const int b = first ? (int)blockIdx.x : (int)blockIdx.x - S0.blocks;
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  Sum64 a = {0.0, {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, 0.0};
+  const int per = S.wide ? 1 : 4;
+  for (int g = b * per; g < S.n; g += S.blocks * per) {
+    const int q = S.wide ? g : g + w;
+    double f[3] = {0.0, 0.0, 0.0};
+    if (q < S.n) {
+      const int i = S.i0 + q;
+      const int p0 = nbr_start[i] + (S.wide ? t : lane), e = nbr_start[i + 1];
+      listed64<PBC, SWK>(i, p0, S.wide ? 256 : WAVE, two, first, P, sw, pos, absidx, nbr, e, f, a);
+    }
+    for (int k = 0; k < 3; k++) f[k] = wave_sum_d(f[k]);
+    if (!S.wide) {
+      if (q < S.n && lane < 3) deriv[3 * (size_t)(S.i0 + q) + lane] = lane == 0 ? f[0] : (lane == 1 ? f[1] : f[2]);
+      continue;
+    }
+    if (lane == 0)
+      for (int k = 0; k < 3; k++) sf[w][k] = f[k];
+    __syncthreads();
+    if (t < 3) deriv[3 * (size_t)(S.i0 + q) + t] = ((sf[0][t] + sf[1][t]) + sf[2][t]) + sf[3][t];
+    __syncthreads();
+  }
+  store_partial64(a, partial);
 }
 
 // PAIR: the k-th atom of GROUPA with the k-th of GROUPB
@@ -2263,25 +2434,6 @@ __device__ __forceinline__ bool grid_adjacent(const CellGrid& G, const int* a, c
   return true;
 }
 
-// pair (p,q) as the reference lists it: GROUPA atom first with two groups,
-// the lower index first in one group
-__device__ __forceinline__ bool nl_member(int mode, int p, int q, int use_pbc, const PbcArg& P, double cut2,
-                                          const CellGrid& G, const double* __restrict__ pos,
-                                          const int* __restrict__ cellof) {
-#pragma clang fp contract(off)
-  if (mode == P2A_NL_CELLS) {
-    const int a[3] = {cellof[3 * p], cellof[3 * p + 1], cellof[3 * p + 2]};
-    const int b[3] = {cellof[3 * q], cellof[3 * q + 1], cellof[3 * q + 2]};
-    return grid_adjacent(G, a, b);
-  }
-  const double* xa = pos + 3 * (size_t)p;
-  const double* xb = pos + 3 * (size_t)q;
-  double d[3];
-  if (use_pbc) pbc_distance(P, xa, xb, d);
-  else { d[0] = xb[0] - xa[0]; d[1] = xb[1] - xa[1]; d[2] = xb[2] - xa[2]; }
-  return d[0] * d[0] + d[1] * d[1] + d[2] * d[2] <= cut2;
-}
-
 __global__ void k_nl_cells(int natoms, CellGrid G, const double* __restrict__ pos, int* __restrict__ cellof) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= natoms) return;
@@ -2293,37 +2445,98 @@ __global__ void k_nl_cells(int natoms, CellGrid G, const double* __restrict__ po
 }
 
 // FILL = 0: count[i] = listed partners of atom i; FILL = 1: write them, in
-// index order, from start[i]
-template <int FILL>
-__global__ void k_nl_atoms(int nA, int nB, int mode, int use_pbc, PbcArg P, double cut2, CellGrid G,
-                           const double* __restrict__ pos, const int* __restrict__ cellof,
-                           int* __restrict__ count, const int* __restrict__ start, int* __restrict__ nbr) {
+// index order, from start[i].  CELLS: the stencil of link cells, else
+// |d|^2 <= cut2.  One wave per atom; four chunks of 64 candidates a trip,
+// whose loads go out together (the candidates' latency is the bound), and a
+// ballot places the listed ones in index order.  Measured at 700 x 5,300
+// atoms: one thread per atom 1.81 ms (count) and 2.21 ms (fill), now 18 and 29 us.
+template <int FILL, bool CELLS, int PBC>
+__global__ __launch_bounds__(256) void k_nl_atoms(int nA, int nB, PbcArg P, double cut2, CellGrid G,
+                                                  const double* __restrict__ pos,
+                                                  const int* __restrict__ cellof, int* __restrict__ count,
+                                                  const int* __restrict__ start, int* __restrict__ nbr) {
+#pragma clang fp contract(off)
+  constexpr int U = 4;
   const int natoms = nA + nB;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (i >= natoms) return;
   const bool two = nB > 0;
   const int j0 = two ? (i < nA ? nA : 0) : 0;
   const int j1 = two ? (i < nA ? natoms : nA) : nA;
+  double xi[3] = {0.0, 0.0, 0.0};
+  int ci[3] = {0, 0, 0};
+  for (int k = 0; k < 3; k++) {
+    if constexpr (CELLS) ci[k] = cellof[3 * i + k];
+    else xi[k] = pos[3 * (size_t)i + k];
+  }
   int n = 0;
   const int base = FILL ? start[i] : 0;
-  for (int j = j0; j < j1; j++) {
-    if (!two && j == i) continue;
-    const int p = two ? (i < nA ? i : j) : min(i, j);
-    const int q = two ? (i < nA ? j : i) : max(i, j);
-    if (nl_member(mode, p, q, use_pbc, P, cut2, G, pos, cellof)) {
-      if (FILL) nbr[base + n] = j;
-      n++;
+  for (int jb = j0; jb < j1; jb += U * WAVE) {
+    double x[U][3];
+    int c[U][3];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int j = min(jb + u * WAVE + lane, j1 - 1);
+      for (int k = 0; k < 3; k++) {
+        if constexpr (CELLS) c[u][k] = cellof[3 * j + k];
+        else x[u][k] = pos[3 * (size_t)j + k];
+      }
+    }
+    bool in[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int j = jb + u * WAVE + lane;
+      // the pair (p, q) as the reference lists it: GROUPA atom first with two
+      // groups, the lower index first in one group
+      const bool own = two ? i < nA : i < j;
+      if constexpr (CELLS) {
+        in[u] = own ? grid_adjacent(G, ci, c[u]) : grid_adjacent(G, c[u], ci);
+      } else {
+        double d[3];
+        for (int k = 0; k < 3; k++) d[k] = own ? x[u][k] - xi[k] : xi[k] - x[u][k];
+        wrap64<PBC>(P, d);
+        in[u] = d[0] * d[0] + d[1] * d[1] + d[2] * d[2] <= cut2;
+      }
+      in[u] = in[u] && j < j1 && (two || j != i);
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const unsigned long long m = __ballot(in[u]);
+      if (FILL && in[u]) nbr[base + n + bits_below(m)] = jb + u * WAVE + lane;
+      n += __popcll(m);
     }
   }
-  if (!FILL) count[i] = n;
+  if (!FILL && lane == 0) count[i] = n;
+}
+
+template <int FILL>
+inline void launch_nl_atoms(hipStream_t s, int nA, int nB, bool cells, int use_pbc, const PbcArg& P, double cut2,
+                            const CellGrid& G, const double* pos, const int* cellof, int* count, const int* start,
+                            int* nbr) {
+  const dim3 grid((unsigned)((nA + nB + 3) / 4));
+#define P2A_NL(C, PBC)                                                                                      \
+  hipLaunchKernelGGL((k_nl_atoms<FILL, C, PBC>), grid, dim3(256), 0, s, nA, nB, P, cut2, G, pos, cellof, count, start, nbr)
+  const int pbc = use_pbc ? P.type : 0;
+  if (cells) P2A_NL(true, 0);
+  else if (pbc == 0) P2A_NL(false, 0);
+  else if (pbc == 1) P2A_NL(false, 1);
+  else P2A_NL(false, 2);
+#undef P2A_NL
 }
 
 // PAIR with a list: keep[k] = pair k within NL_CUTOFF (classic branch)
 __global__ void k_nl_pairs_keep(int nA, int use_pbc, PbcArg P, double cut2, const double* __restrict__ pos,
                                 int* __restrict__ keep) {
+#pragma clang fp contract(off)
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nA) return;
-  keep[i] = nl_member(P2A_NL_CLASSIC, i, nA + i, use_pbc, P, cut2, CellGrid{}, pos, nullptr) ? 1 : 0;
+  const double* xa = pos + 3 * (size_t)i;
+  const double* xb = pos + 3 * (size_t)(nA + i);
+  double d[3];
+  if (use_pbc) pbc_distance(P, xa, xb, d);
+  else { d[0] = xb[0] - xa[0]; d[1] = xb[1] - xa[1]; d[2] = xb[2] - xa[2]; }
+  keep[i] = d[0] * d[0] + d[1] * d[1] + d[2] * d[2] <= cut2 ? 1 : 0;
 }
 
 // exclusive scan of n counts in one workgroup of 1024 threads (contiguous
@@ -2403,6 +2616,82 @@ inline void sys_columns(const double* box9, int n, SysArg& S) {
     S.ncx = std::max(1, S.ncx / 2);
     S.ncy = std::max(1, S.ncy / 2);
   }
+}
+
+// How one side of the all-pairs pass goes over the chip: many atoms with at
+// most 64 partners (a solvent against one ion), or more atoms than fill the
+// chip as threads: one thread per atom; up to 1,024 atoms: one atom per
+// workgroup; above: kIt64 atoms per workgroup share each partner.
+inline Side64 side64(int i0, int n, int j0, int m, int max_blocks) {
+  Side64 S = {i0, n, j0, m, 0, 0};
+  if (n == 0) return S;
+  S.it = ((m <= 64 && n > 4096) || n >= (1 << 18)) ? 0 : (n <= 1024 ? 1 : kIt64);
+  const int per = S.it == 0 ? 256 : S.it;
+  S.blocks = std::max(1, std::min(grid1((size_t)n, per), max_blocks));
+  return S;
+}
+
+// Side of a list pass over `entries` listed partners: a workgroup per atom
+// from 512 partners an atom on (two trips of a workgroup), and for so few
+// atoms that waves would leave the chip idle.
+constexpr int kMaxListBlocks64 = 4096;
+inline ListSide64 list_side64(int i0, int n, int64_t entries) {
+  ListSide64 S = {i0, n, 0, 0};
+  if (n == 0) return S;
+  S.wide = entries >= 512 * (int64_t)n || (n < 1024 && entries >= 128 * (int64_t)n);
+  S.blocks = std::min(grid1((size_t)n, S.wide ? 1 : 4), kMaxListBlocks64 / 2);
+  return S;
+}
+
+// the switch of the FP64 pair kernels that unrolls (0: evaluated generically)
+inline int switch64_kind(const p2a_switch& sw) {
+  return sw.type == P2A_SW_RATIONAL_FIXED && (sw.nn == 6 || sw.nn == 8) ? sw.nn / 2 : 0;
+}
+
+// FP64 pass over every pair (at most kMaxBlocks64 rows of `partial`), or over
+// the list nbr_start / nbr of nbr_total partners (at most kMaxListBlocks64
+// rows); writes deriv and the rows, whose number is returned.  absidx null:
+// the requested atoms are distinct atoms.
+inline int launch_pairs64(hipStream_t s, int nA, int nB, int use_pbc, const PbcArg& P, const p2a_switch& sw,
+                          const double* pos, const long long* absidx, double* deriv, double* partial,
+                          const int* nbr_start = nullptr, const int* nbr = nullptr, int64_t nbr_total = 0) {
+  const int pbc = !use_pbc || P.type == 0 ? 0 : P.type;
+  const int kind = switch64_kind(sw);
+  const bool two = nB > 0;
+  Side64 S0, S1;
+  ListSide64 L0, L1;
+  int grid;
+  if (nbr_start) {
+    // a symmetric list: with two groups each side holds half of the partners
+    L0 = list_side64(0, nA, two ? nbr_total / 2 : nbr_total);
+    L1 = list_side64(nA, nB, nbr_total / 2);
+    grid = L0.blocks + L1.blocks;
+  } else {
+    S0 = side64(0, nA, two ? nA : 0, two ? nB : nA, two ? kMaxBlocks64 / 2 : kMaxBlocks64);
+    S1 = side64(nA, nB, 0, nA, kMaxBlocks64 - S0.blocks);
+    grid = S0.blocks + S1.blocks;
+  }
+#define P2A_A(PBC, K)                                                                                            \
+  do {                                                                                                           \
+    if (nbr_start)                                                                                               \
+      hipLaunchKernelGGL((k_listpairs<PBC, K>), dim3(grid), dim3(256), 0, s, L0, L1, P, sw, pos, absidx, deriv,  \
+                         partial, nbr_start, nbr);                                                               \
+    else                                                                                                         \
+      hipLaunchKernelGGL((k_allpairs<PBC, K>), dim3(grid), dim3(256), 0, s, S0, S1, P, sw, pos, absidx, deriv,   \
+                         partial);                                                                               \
+  } while (0)
+#define P2A_AK(PBC)                    \
+  do {                                 \
+    if (kind == 3) P2A_A(PBC, 3);      \
+    else if (kind == 4) P2A_A(PBC, 4); \
+    else P2A_A(PBC, 0);                \
+  } while (0)
+  if (pbc == 0) P2A_AK(0);
+  else if (pbc == 1) P2A_AK(1);
+  else P2A_AK(2);
+#undef P2A_AK
+#undef P2A_A
+  return grid;
 }
 
 // the chunk size (entries per work item) and the grid of the pair kernel
