@@ -2,13 +2,13 @@
 // bias/force, the fused per-step METAD kernel and the force chain rule.
 //
 // What each piece replaces in the reference:
-//   k_deposit_seq   MetaD::update -> getHeight -> addGaussian -> evaluate-
-//                   GaussianAndDerivatives -> Grid::addValueAndDerivatives
-//                   (src/bias/MetaD.cpp:2377-2470, 2280-2305, 1886-1937,
-//                   2186-2278; src/tools/Grid.cpp:55-106, 904-910), looping
-//                   over many hills inside one persistent workgroup because
-//                   each well-tempered height depends on the grid left by the
-//                   previous hill
+//   k_hill_chain,   MetaD::update -> getHeight -> addGaussian -> evaluate-
+//   k_hill_nodes,   GaussianAndDerivatives -> Grid::addValueAndDerivatives
+//   k_deposit_seq   (src/bias/MetaD.cpp:2377-2470, 2280-2305, 1886-1937,
+//                   2186-2278; src/tools/Grid.cpp:55-106, 904-910) for many
+//                   hills in order (each well-tempered height depends on the
+//                   grid left by the previous hill): heights and grid in turn
+//                   for many hills, one workgroup for a few
 //   k_add_hills     addGaussian for hills of known heights (HILLS restart,
 //                   MetaD::readGaussians :1807-1829), all hills in parallel
 //   spline()        GridBase::getValueAndDerivatives spline branch
@@ -61,6 +61,7 @@ struct GridArg {
   double invsigma[kMaxCv];
   double height0, biasf, kbt, stretchA, stretchB;
   double inv_wt;          // 1 / (kbt (biasf - 1)) for biasf > 1, else 1 / kbt
+  double kd[kMaxCv];      // -invsigma * stretchA: scaled distance -> gradient factor
   int welltemp;
   int support;            // prod(2*nneigh+1)
   int may_alias;          // a periodic support wider than the grid visits a node twice
@@ -213,8 +214,76 @@ __device__ __forceinline__ bool support_node(const GridArg& G, const unsigned* i
   return true;
 }
 
+// exp(x), |x| < 2^20, for the heights and the shapes: ln2 reduction and the
+// Taylor polynomial of degree 13 on |r| <= ln2/2 (truncation 4e-18) in pairs,
+// so that its depth is 5 multiply-adds instead of a dozen in a row; within
+// 1.5 ulp.  The chain of heights keeps the constants in registers (a 64-bit
+// literal costs two moves): ExpK, made opaque there.
+struct ExpK {
+  double log2e = 1.4426950408889634;
+  // ln2 in two parts, the first of 32 bits (its product with n is exact)
+  double hi = -0x1.62e42fee00000p-1, lo = -0x1.a39ef35793c76p-33;
+  double m[6] = {1.0 / 6, 1.0 / 120, 1.0 / 5040, 1.0 / 362880, 1.0 / 39916800, 1.0 / 6227020800.0};
+  double a[5] = {1.0 / 24, 1.0 / 720, 1.0 / 40320, 1.0 / 3628800, 1.0 / 479001600};
+};
+// exp(x) = 2^n p: p from x and n = rint(x log2e)
+__device__ __forceinline__ double exp_part(double x, double n, const ExpK& C) {
+  double r = fma(n, C.hi, x);
+  r = fma(n, C.lo, r);
+  const double r2 = r * r, r4 = r2 * r2, r8 = r4 * r4;
+  const double p01 = 1.0 + r, p23 = fma(r, C.m[0], 0.5);
+  const double p45 = fma(r, C.m[1], C.a[0]), p67 = fma(r, C.m[2], C.a[1]);
+  const double p89 = fma(r, C.m[3], C.a[2]), pab = fma(r, C.m[4], C.a[3]), pcd = fma(r, C.m[5], C.a[4]);
+  const double q0 = fma(r2, p23, p01), q1 = fma(r2, p67, p45), q2 = fma(r2, pab, p89);
+  const double lo = fma(r4, q1, q0), hi = fma(r4, pcd, q2);
+  return fma(r8, hi, lo);
+}
+__device__ __forceinline__ double exp_core(double x) {
+  const ExpK C;
+  const double n = rint(x * C.log2e);
+  return ldexp(exp_part(x, n, C), (int)n);
+}
+
+// One hill at a node, as every deposition in hill order forms it.  Per CV:
+// s = dp^2/2 of the scaled distance dp, the factor f = exp(-s), and w, dp
+// times the gradient's constant; the shape is the product of the factors
+// (exp(-dp^2/2) up to rounding, so that the factors of a grid line serve all
+// its nodes), and the value and gradient receive fma(height, term, .).  The
+// heights' corners and the grid nodes go through the same operations in the
+// same order, so a node holds the same bits however the hills were grouped.
+struct HillDim {
+  double s, f, w;
+};
+// scaled distance along CV i; PER: some CV is periodic
+template <bool PER>
+__device__ __forceinline__ double hill_scaled(const GridArg& G, int i, double c, double x) {
+  if constexpr (PER) return vdiff(G, i, c, x) * G.invsigma[i];
+  return (x - c) * G.invsigma[i];
+}
+template <bool PER>
+__device__ __forceinline__ HillDim hill_dim(const GridArg& G, int i, double c, double x) {
+  HillDim H;
+  const double dp = hill_scaled<PER>(G, i, c, x);
+  H.s = 0.5 * (dp * dp);
+  H.f = exp_core(-H.s);
+  H.w = dp * G.kd[i];
+  return H;
+}
+// the shape (negative beyond the cutoff: no term)
+template <int NCV>
+__device__ __forceinline__ double hill_shape(const HillDim* H) {
+  double s = H[0].s, e = H[0].f;
+#pragma unroll
+  for (int i = 1; i < NCV; i++) {
+    s += H[i].s;
+    e *= H[i].f;
+  }
+  return s < 6.25 ? e : -1.0;
+}
+
 // add one hill of height h centred at c to the grid, all threads of the block
 // (distinct nodes per thread unless may_alias, then thread 0 alone)
+template <int NCV>
 __device__ void add_hill_block(const GridArg& G, double* __restrict__ val, double* __restrict__ der,
                                const unsigned* ind, const double* c, double h) {
   const int t0 = G.may_alias ? 0 : (int)threadIdx.x;
@@ -224,52 +293,38 @@ __device__ void add_hill_block(const GridArg& G, double* __restrict__ val, doubl
     unsigned ni[kMaxCv];
     if (!support_node(G, ind, s, ni)) continue;
     const long long node = flat(G, ni);
-    double xx[kMaxCv], d[kMaxCv];
-    for (int i = 0; i < G.ncv; i++) xx[i] = G.min[i] + (double)ni[i] * G.dx[i];
-    const double b = gaussian(G, xx, c, h, d);
-    val[node] += b;
-    for (int i = 0; i < G.ncv; i++) der[node * G.ncv + i] += d[i];
+    double d[NCV];
+    // the node's values are on their way while the factors are formed
+    const double v = val[node];
+#pragma unroll
+    for (int i = 0; i < NCV; i++) d[i] = der[node * NCV + i];
+    HillDim H[NCV];
+#pragma unroll
+    for (int i = 0; i < NCV; i++) H[i] = hill_dim<true>(G, i, c[i], G.min[i] + (double)ni[i] * G.dx[i]);
+    const double e = hill_shape<NCV>(H);
+    if (e < 0.0) continue;
+    val[node] = fma(h, fma(G.stretchA, e, G.stretchB), v);
+#pragma unroll
+    for (int i = 0; i < NCV; i++) der[node * NCV + i] = fma(h, e * H[i].w, d[i]);
   }
 }
 
 // MetaD::getHeight (MetaD.cpp:2280-2305): height0 exp(-V / (kbt (biasf - 1)));
 // the division is a product with its reciprocal, formed once on the host, so
 // that the sequential chain of heights carries no division (the heights move
-// by about one rounding of the exponent's argument)
+// by about one rounding of the exponent's argument).  2^n height0 is formed
+// beside the polynomial.
+__device__ __forceinline__ double wt_fast(double height0, double inv_wt, double inv_wt2, double vbias,
+                                          const ExpK& C) {
+  const double n = rint(vbias * -inv_wt2);
+  return exp_part(-vbias * inv_wt, n, C) * ldexp(height0, (int)n);
+}
+// where wt_fast holds: finite heights of any run
+__device__ __forceinline__ bool wt_in_range(double inv_wt, double vbias) { return fabs(vbias * inv_wt) < 700.0; }
 __device__ __forceinline__ double wt_height(const GridArg& G, double vbias) {
   if (!G.welltemp) return G.height0;
+  if (wt_in_range(G.inv_wt, vbias)) return wt_fast(G.height0, G.inv_wt, G.inv_wt * ExpK().log2e, vbias, ExpK());
   return G.height0 * exp(-vbias * G.inv_wt);
-}
-
-// spline value (no gradient) at x from the corner ip of its cell: the term
-// `value += grid * ff` of GridBase::getValueAndDerivatives for one ip
-__device__ double spline_corner(const GridArg& G, const double* __restrict__ val, const double* __restrict__ der,
-                                const double* x, const unsigned* ind, unsigned ip) {
-  unsigned ni[kMaxCv];
-  unsigned t = ip;
-  int cnt = 0;
-  for (int j = 0; j < G.ncv; j++) {
-    unsigned i0 = t % 2 + ind[j];
-    t /= 2;
-    if (!G.pbc[j] && i0 == G.nbin[j]) continue;
-    if (G.pbc[j] && i0 == G.nbin[j]) i0 = 0;
-    ni[cnt++] = i0;
-  }
-  if (cnt != G.ncv) return 0.0;
-  const long long node = flat(G, ni);
-  const double grid = val[node];
-  double ff = 1.0;
-  for (int j = 0; j < G.ncv; j++) {
-    const int x0 = (ni[j] == ind[j]) ? 0 : 1;
-    const double dx = G.dx[j];
-    const double xfloor = G.min[j] + (double)ind[j] * dx;
-    const double X = fabs((x[j] - xfloor) / dx - (double)x0);
-    const double X2 = X * X, X3 = X2 * X;
-    const double yy = fabs(grid) < 0.0000001 ? 0.0 : -der[node * G.ncv + j] / grid;
-    const double sg = x0 ? -1.0 : 1.0;
-    ff *= (1.0 - 3.0 * X2 + 2.0 * X3) - sg * yy * (X - 2.0 * X2 + X3) * dx;
-  }
-  return grid * ff;
 }
 
 // value and gradient terms of the corner ip of the cell of x: the terms
@@ -324,115 +379,34 @@ __device__ void spline_corner_grad(const GridArg& G, const double* __restrict__ 
   value = grid * ff;
 }
 
-// Sequential well-tempered deposition of many hills in one workgroup: each
-// hill's height needs the bias of the grid left by the previous hill
-// (MetaD::update -> getHeight).  Per hill, the first wave evaluates the
-// 2^ncv spline corners in parallel and sums them in corner order; then the
-// whole workgroup adds the hill, one support node per thread.
-constexpr int kSeqThreads = 1024;
-__global__ __launch_bounds__(kSeqThreads) void k_deposit_seq(GridArg G, double* __restrict__ val,
-                                                             double* __restrict__ der, long long nhills,
-                                                             const double* __restrict__ centers,
-                                                             double* __restrict__ heights, int* __restrict__ err) {
-  __shared__ double sh_h;
-  __shared__ int sh_ok;
-  __shared__ unsigned sh_ind[kMaxCv];
-  __shared__ double sh_c[kMaxCv];
-  const int t = threadIdx.x;
-  const unsigned nn = 1u << G.ncv;
-  for (long long k = 0; k < nhills; k++) {
-    if (t < WAVE_M) {
-      double c[kMaxCv];
-      for (int i = 0; i < G.ncv; i++) c[i] = centers[k * G.ncv + i];
-      unsigned ind[kMaxCv];
-      const int ok = grid_index_of(G, c, ind) >= 0;
-      double v = 0.0;
-      if (ok && G.welltemp && (unsigned)t < nn) v = spline_corner(G, val, der, c, ind, (unsigned)t);
-      // corner order 0, 1, 2, ... as the sequential loop adds them
-      double tot = 0.0;
-      for (unsigned q = 0; q < nn; q++) tot += __shfl(v, (int)q, WAVE_M);
-      if (t == 0) {
-        const double h = (ok && G.welltemp) ? wt_height(G, tot) : G.height0;
-        if (!ok) atomicCAS(err, 0, (int)(1 + (k < 0x3fffffff ? k : 0x3fffffff)));
-        for (int i = 0; i < G.ncv; i++) {
-          sh_ind[i] = ind[i];
-          sh_c[i] = c[i];
-        }
-        sh_h = h;
-        sh_ok = ok;
-        if (heights) heights[k] = ok ? h : 0.0;
-      }
-    }
-    __syncthreads();
-    if (!sh_ok) return;  // uniform: every thread reads the same flag
-    unsigned ind[kMaxCv];
-    double c[kMaxCv];
-    for (int i = 0; i < G.ncv; i++) {
-      ind[i] = sh_ind[i];
-      c[i] = sh_c[i];
-    }
-    add_hill_block(G, val, der, ind, c, sh_h);
-    __syncthreads();
-  }
+// ------------------------------------------------------------------------
+// deposition of hills in order
+// ------------------------------------------------------------------------
+
+// 1/x without the scaling steps of a division (|x| is at least 1e-7 where it
+// counts): v_rcp_f64, good to 2^-23, and one step of third order
+__device__ __forceinline__ double rcp64(double x) {
+  const double r = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, r, 1.0);
+  return fma(r, fma(e, e, e), r);
 }
 
-// Two non-periodic CVs: the same sequential deposition with the grid around
-// the walk held in LDS (a tile of tw x th <= kTileNodes nodes, shaped like
-// the hill support: value and the two gradient components), in runs of up
-// to kRun consecutive hills that the tile holds (support and upper spline
-// corner).  A run's heights are found by wave 0 alone (lane 4r+q holds
-// corner q of hill r: hill k's height comes from its four corners, then
-// every later corner in hill k's support adds hill k's Gaussian), from the
-// shapes of each hill at the corners of the later hills of the run, which
-// the whole workgroup evaluates beforehand.  Runs are pipelined: while waves
-// 1-15 add the current run to the tile (one node per thread, the run's hills
-// in order), wave 0 finds the heights of the next run, whose corners start
-// from the tile as it was before the current run plus the current run's
-// hills added in order; only a run that needs another tile (the old one is
-// written back first) waits for the current run.  Every node, and every
-// corner read for a height, receives the same FP64 additions in the same
-// order as hill-by-hill deposition, so grids and heights are identical to it.
-constexpr int kTileNodes = 5120;
-constexpr int kRun = 16;  // hills per run: 4 corners each on one wave
-constexpr int kFacLen = 160;  // tile width + height at most: factor tables
-
-// The 2-CV kernel takes the Gaussian as a product of one factor per CV,
-// exp(-dp0^2/2) exp(-dp1^2/2) (the same value as exp(-dp2) up to rounding),
-// so that a run's deposition evaluates one exponential per hill and grid
-// column or row; the support and the cutoff test are those of gauss_shape.
-__device__ __forceinline__ double gfac(double x) { return exp(-0.5 * (x * x)); }
-__device__ __forceinline__ double gscaled(const GridArg& G, int i, double c, double x) {
-  return vdiff(G, i, c, x) * G.invsigma[i];
+template <int CTRL>
+__device__ __forceinline__ double dpp_m(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)(b & 0xffffffffll), CTRL, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xF, 0xF, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
-__device__ __forceinline__ bool gauss_shape_f2(const GridArg& G, const double* xx, const double* c, double* dp,
-                                               double& e) {
-  dp[0] = gscaled(G, 0, c[0], xx[0]);
-  dp[1] = gscaled(G, 1, c[1], xx[1]);
-  double dp2 = dp[0] * dp[0];
-  dp2 += dp[1] * dp[1];
-  dp2 *= 0.5;
-  e = 0.0;
-  if (!(dp2 < 6.25)) return false;
-  e = gfac(dp[0]) * gfac(dp[1]);
-  return true;
+// sum over the aligned group of 2^NCV lanes, in every lane of it
+template <int NCV>
+__device__ __forceinline__ double corner_sum(double v) {
+  v += dpp_m<0xB1>(v);                             // quad_perm 1,0,3,2
+  if constexpr (NCV >= 2) v += dpp_m<0x4E>(v);     // quad_perm 2,3,0,1
+  if constexpr (NCV >= 3) v += dpp_m<0x141>(v);    // row_half_mirror
+  if constexpr (NCV >= 4) v += dpp_m<0x140>(v);    // row_mirror
+  return v;
 }
-
-__device__ __forceinline__ double spline_corner_vals(const GridArg& G, const double* x, const unsigned* ind,
-                                                     const unsigned* ni, double grid, const double* der) {
-  double ff = 1.0;
-  for (int j = 0; j < 2; j++) {
-    const int x0 = (ni[j] == ind[j]) ? 0 : 1;
-    const double dx = G.dx[j];
-    const double xfloor = G.min[j] + (double)ind[j] * dx;
-    const double X = fabs((x[j] - xfloor) / dx - (double)x0);
-    const double X2 = X * X, X3 = X2 * X;
-    const double yy = fabs(grid) < 0.0000001 ? 0.0 : -der[j] / grid;
-    const double sg = x0 ? -1.0 : 1.0;
-    ff *= (1.0 - 3.0 * X2 + 2.0 * X3) - sg * yy * (X - 2.0 * X2 + X3) * dx;
-  }
-  return grid * ff;
-}
-
 // value of lane `l` (uniform) of a double, through the scalar unit
 __device__ __forceinline__ double readlane_d(double v, int l) {
   const long long b = __double_as_longlong(v);
@@ -441,385 +415,564 @@ __device__ __forceinline__ double readlane_d(double v, int l) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
-__global__ __launch_bounds__(kSeqThreads) void k_deposit_seq_tile2(GridArg G, double* __restrict__ val,
-                                                                   double* __restrict__ der, long long nhills,
-                                                                   const double* __restrict__ centers,
-                                                                   double* __restrict__ heights,
-                                                                   int* __restrict__ err, int tw, int th) {
-  __shared__ double tv[kTileNodes], tdx[kTileNodes], tdy[kTileNodes];
-  // two runs: the current one (heights known, not yet on the tile) and the next
-  __shared__ double sh_c[2][kRun][2], sh_h[2][kRun];
-  __shared__ int sh_ind[2][kRun][2];
-  // shape of hill j at corner lane l (e, negative: no contribution; scaled
-  // distances): of the next run's hills (j < r), or of the current run's
-  // hills at the next run's corners
-  __shared__ double sh_e[kRun][4 * kRun];
-  // the same for the current run's hills at the next run's corners
-  __shared__ double sh_ex[kRun][4 * kRun];
-  // per hill of the current run: its factor at each column of the run's
-  // box, then at each row (sh_box: the box)
-  __shared__ double sh_f[kRun][kFacLen];
-  __shared__ int sh_box[4];
-  // value and gradient at each corner of the next run before its own hills
-  __shared__ double sh_y[4 * kRun][3];
-  __shared__ int sh_nb, sh_fit, sh_nox, sh_noy;
-  const int t = threadIdx.x;
-  const int lane = t & (WAVE_M - 1);
-  const bool wave0 = t < WAVE_M;
-  const int nx = (int)G.nbin[0], ny = (int)G.nbin[1];
-  const int nn0 = G.nneigh[0], nn1 = G.nneigh[1];
-  int ox = -1, oy = -1;  // tile origin in nodes (-1: no tile loaded)
-  auto flush = [&]() {
-    if (ox < 0) return;
-    for (int j = t; j < tw * th; j += blockDim.x) {
-      const int lx = j % tw, ly = j / tw;
-      const long long node = (long long)(oy + ly) * nx + (ox + lx);
-      const int l = lx + tw * ly;
-      val[node] = tv[l];
-      der[2 * node] = tdx[l];
-      der[2 * node + 1] = tdy[l];
-    }
-  };
-  // wave 0: the run of hills from k0 into buffer b; sh_fit = it lies in the
-  // current tile, else the tile centred on its first hill is sh_nox/noy.
-  // Lane l's centre (hill k0 + l) comes in c0, c1 when `pre`.
-  auto decide = [&](long long k0, int b, bool pre, double c0, double c1) {
-    const long long k = k0 + lane;
-    const bool valid = k < nhills;
-    double c[2] = {0.0, 0.0};
-    unsigned ind[2] = {0u, 0u};
-    int ok = 0;
-    if (valid) {
-      if (pre) {
-        c[0] = c0;
-        c[1] = c1;
-      } else {
-        c[0] = centers[2 * k];
-        c[1] = centers[2 * k + 1];
-      }
-      ok = grid_index_of(G, c, ind) >= 0;
-    }
-    // nodes the hill touches: support, and the cell's upper spline corner
-    const int xl = max(0, (int)ind[0] - nn0), xh = min(nx - 1, (int)ind[0] + nn0 + 1);
-    const int yl = max(0, (int)ind[1] - nn1), yh = min(ny - 1, (int)ind[1] + nn1 + 1);
-    const int xl0 = __builtin_amdgcn_readfirstlane(xl), xh0 = __builtin_amdgcn_readfirstlane(xh);
-    const int yl0 = __builtin_amdgcn_readfirstlane(yl), yh0 = __builtin_amdgcn_readfirstlane(yh);
-    const int i00 = __builtin_amdgcn_readfirstlane((int)ind[0]);
-    const int i01 = __builtin_amdgcn_readfirstlane((int)ind[1]);
-    const bool fit0 = ox >= 0 && xl0 >= ox && xh0 < ox + tw && yl0 >= oy && yh0 < oy + th;
-    // a tile centred on the hill holds it whenever nneigh + 2 <= tile / 2,
-    // which the launch guarantees; checked anyway before any LDS index
-    const int nox = max(0, min(nx - tw, i00 - tw / 2));
-    const int noy = max(0, min(ny - th, i01 - th / 2));
-    const int bx = fit0 ? ox : nox, by = fit0 ? oy : noy;
-    const bool fits = lane < kRun && valid && ok && xl >= bx && xh < bx + tw && yl >= by && yh < by + th;
-    const unsigned long long bad = __ballot(!fits);
-    const int nb = min(kRun, __ffsll((long long)bad) - 1);
-    if (lane < nb) {
-      sh_c[b][lane][0] = c[0];
-      sh_c[b][lane][1] = c[1];
-      sh_ind[b][lane][0] = (int)ind[0];
-      sh_ind[b][lane][1] = (int)ind[1];
-    }
-    if (lane == 0) {
-      sh_nb = nb;
-      sh_fit = fit0;
-      sh_nox = nox;
-      sh_noy = noy;
-      // a first hill that no tile can hold lies outside the grid
-      if (nb == 0 && k0 < nhills) atomicCAS(err, 0, (int)(1 + (k0 < 0x3fffffff ? k0 : 0x3fffffff)));
-    }
-  };
-  // the shapes of the hills j < nsrc of run bs at the corners of the hills
-  // r < ndst of run bd (only j < r when both are the same run)
-  auto shapes = [&](int bs, int nsrc, int bd, int ndst, double (*out)[4 * kRun]) {
-    for (int p = t; p < kRun * 4 * kRun; p += blockDim.x) {
-      const int j = p / (4 * kRun), l = p % (4 * kRun);
-      const int r = l >> 2, q = l & 3;
-      double e = -1.0, dp[2] = {0.0, 0.0};
-      if (j < nsrc && r < ndst && (bs != bd || j < r)) {
-        const unsigned n0 = (unsigned)sh_ind[bd][r][0] + (q & 1), n1 = (unsigned)sh_ind[bd][r][1] + (q >> 1);
-        if (n0 < G.nbin[0] && n1 < G.nbin[1] && abs((int)n0 - sh_ind[bs][j][0]) <= nn0 &&
-            abs((int)n1 - sh_ind[bs][j][1]) <= nn1) {
-          const double xx[2] = {G.min[0] + (double)n0 * G.dx[0], G.min[1] + (double)n1 * G.dx[1]};
-          const double cj[2] = {sh_c[bs][j][0], sh_c[bs][j][1]};
-          double ej;
-          if (gauss_shape_f2(G, xx, cj, dp, ej)) e = ej;
-        }
-      }
-      out[j][l] = e;
-    }
-  };
-  // threads t < 4 kRun: value and gradient at corner t of run b, from the
-  // tile, or from the grid in memory for a node outside the tile
-  auto snapshot = [&](int b, int nb) {
-    if (t < 4 * kRun) {
-      const int r = t >> 2, q = t & 3;
-      double y0 = 0.0, y1 = 0.0, y2 = 0.0;
-      if (r < nb) {
-        const unsigned n0 = (unsigned)sh_ind[b][r][0] + (q & 1), n1 = (unsigned)sh_ind[b][r][1] + (q >> 1);
-        if (n0 < G.nbin[0] && n1 < G.nbin[1]) {
-          if ((int)n0 >= ox && (int)n0 < ox + tw && (int)n1 >= oy && (int)n1 < oy + th) {
-            const int l = (int)(n0 - ox) + tw * (int)(n1 - oy);
-            y0 = tv[l];
-            y1 = tdx[l];
-            y2 = tdy[l];
-          } else {
-            const long long node = (long long)n1 * nx + n0;
-            y0 = val[node];
-            y1 = der[2 * node];
-            y2 = der[2 * node + 1];
-          }
-        }
-      }
-      sh_y[t][0] = y0;
-      sh_y[t][1] = y1;
-      sh_y[t][2] = y2;
-    }
-  };
-  // wave 0: the heights of run b (nb hills from hill kfirst), from sh_y plus
-  // the terms of the nprev hills of run 1 - b (sh_ex, added in order), and
-  // the run's own shapes
-  auto chain = [&](int b, int nb, long long kfirst, int nprev) {
-    const int r = lane >> 2, q = lane & 3;
-    const bool mine = r < nb;
-    double c[2] = {0.0, 0.0};
-    unsigned ind[2] = {0u, 0u}, ni[2] = {0u, 0u};
-    bool has = false;
-    double acc0 = 0.0, acc1 = 0.0, acc2 = 0.0;
-    if (mine) {
-      c[0] = sh_c[b][r][0];
-      c[1] = sh_c[b][r][1];
-      ind[0] = (unsigned)sh_ind[b][r][0];
-      ind[1] = (unsigned)sh_ind[b][r][1];
-      // corner q of the cell (Grid.cpp:442-505): absent past the last node
-      ni[0] = ind[0] + (q & 1);
-      ni[1] = ind[1] + (q >> 1);
-      has = ni[0] < G.nbin[0] && ni[1] < G.nbin[1];
-      if (has) {
-        acc0 = sh_y[lane][0];
-        acc1 = sh_y[lane][1];
-        acc2 = sh_y[lane][2];
-        const int pb = 1 - b;
-        for (int j0 = 0; j0 < nprev; j0 += 4) {
-          double tb[4], td0[4], td1[4];
-          bool add[4];
+// One corner of the spline cell of a hill centre: the node, its coordinates,
+// and the parts of the spline term (Grid.cpp:442-505) that depend on the
+// position only: the term `grid * prod_j C_j` with C_j = A_j + S_j der_j/grid.
+template <int NCV>
+struct Corner {
+  bool has;           // false past the last node of a non-periodic CV
+  int n[NCV];
+  double x[NCV], A[NCV], S[NCV];
+};
+template <int NCV>
+__device__ __forceinline__ Corner<NCV> corner_of(const GridArg& G, const double* c, const int* ind, int q) {
+  Corner<NCV> K;
+  K.has = true;
 #pragma unroll
-          for (int u = 0; u < 4; u++) {
-            const int j = min(j0 + u, nprev - 1);
-            const double e = sh_ex[j][lane];
-            add[u] = j0 + u < nprev && e >= 0.0;
-            const double dp[2] = {gscaled(G, 0, sh_c[pb][j][0], G.min[0] + (double)ni[0] * G.dx[0]),
-                                  gscaled(G, 1, sh_c[pb][j][1], G.min[1] + (double)ni[1] * G.dx[1])};
-            double d[2];
-            tb[u] = gauss_apply<2>(G, dp, e, sh_h[pb][j], d);
-            td0[u] = d[0];
-            td1[u] = d[1];
-          }
-#pragma unroll
-          for (int u = 0; u < 4; u++) {
-            if (add[u]) {
-              acc0 += tb[u];
-              acc1 += td0[u];
-              acc2 += td1[u];
-            }
-          }
-        }
-      }
+  for (int i = 0; i < NCV; i++) {
+    int n = ind[i] + ((q >> i) & 1);
+    if (n >= (int)G.nbin[i]) {
+      if (G.pbc[i]) n = 0;
+      else K.has = false;
     }
-    // the terms of spline_corner_vals that depend on the position only
-    double X[2] = {0.0, 0.0}, X2[2] = {0.0, 0.0}, X3[2] = {0.0, 0.0}, sg[2] = {1.0, 1.0};
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-      const int x0 = (ni[j] == ind[j]) ? 0 : 1;
-      const double dx = G.dx[j];
-      const double xfloor = G.min[j] + (double)ind[j] * dx;
-      X[j] = fabs((c[j] - xfloor) / dx - (double)x0);
-      X2[j] = X[j] * X[j];
-      X3[j] = X2[j] * X[j];
-      sg[j] = x0 ? -1.0 : 1.0;
-    }
-    // this lane's corner coordinates (the grid node of corner q of hill r)
-    const double xn0 = G.min[0] + (double)ni[0] * G.dx[0], xn1 = G.min[1] + (double)ni[1] * G.dx[1];
-    for (int k = 0; k < nb; k++) {
-      // hill k's shape at this lane's corner does not depend on hill k's
-      // height: read and scaled before the height is found
-      const double ek = sh_e[k][lane];
-      const double dpk[2] = {gscaled(G, 0, sh_c[b][k][0], xn0), gscaled(G, 1, sh_c[b][k][1], xn1)};
-      // corner term of this lane (used by the lanes of hill k only): the
-      // arithmetic of spline_corner_vals
-      double v = 0.0;
-      if (G.welltemp && has && r == k) {
-        const double grid = acc0;
-        const double dg[2] = {acc1, acc2};
-        double ff = 1.0;
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-          const double yy = fabs(grid) < 0.0000001 ? 0.0 : -dg[j] / grid;
-          ff *= (1.0 - 3.0 * X2[j] + 2.0 * X3[j]) - sg[j] * yy * (X[j] - 2.0 * X2[j] + X3[j]) * G.dx[j];
-        }
-        v = grid * ff;
-      }
-      // the four corners of hill k in corner order, on every lane
-      double tot = 0.0;
-#pragma unroll
-      for (int qq = 0; qq < 4; qq++) tot += readlane_d(v, 4 * k + qq);
-      const double h = G.welltemp ? wt_height(G, tot) : G.height0;
-      if (lane == 4 * k) {
-        sh_h[b][k] = h;
-        if (heights) heights[kfirst + k] = h;
-      }
-      if (r > k && mine) {
-        if (ek >= 0.0) {
-          double d[2];
-          const double bb = gauss_apply<2>(G, dpk, ek, h, d);
-          acc0 += bb;
-          acc1 += d[0];
-          acc2 += d[1];
-        }
-      }
-    }
-  };
-  // run b (nb hills) onto the tile: nodes t0, t0 + step, ..., hills in order
-  // the box and the factor tables of run b (all threads; a barrier follows)
-  auto factors = [&](int b, int nb) {
-    // nodes the run deposits on: ind -/+ nneigh, inside the grid
-    int bx0 = INT_MAX, bx1 = -1, by0 = INT_MAX, by1 = -1;
-    for (int k = 0; k < nb; k++) {
-      bx0 = min(bx0, max(0, sh_ind[b][k][0] - nn0));
-      bx1 = max(bx1, min(nx - 1, sh_ind[b][k][0] + nn0));
-      by0 = min(by0, max(0, sh_ind[b][k][1] - nn1));
-      by1 = max(by1, min(ny - 1, sh_ind[b][k][1] + nn1));
-    }
-    const int bw = bx1 - bx0 + 1, bh = by1 - by0 + 1;  // bw + bh <= tw + th <= kFacLen
-    if (t == 0) {
-      sh_box[0] = bx0;
-      sh_box[1] = by0;
-      sh_box[2] = bw;
-      sh_box[3] = bh;
-    }
-    for (int p = t; p < nb * (bw + bh); p += blockDim.x) {
-      const int k = p / (bw + bh), m = p % (bw + bh);
-      const int i = m < bw ? 0 : 1;
-      const int n = i == 0 ? bx0 + m : by0 + (m - bw);
-      sh_f[k][m] = gfac(gscaled(G, i, sh_c[b][k][i], G.min[i] + (double)n * G.dx[i]));
-    }
-  };
-  // run b (nb hills) onto the tile: nodes t0, t0 + step, ..., hills in order
-  // (factors() of the run first)
-  auto deposit = [&](int b, int nb, int t0, int step) {
-    const int bx0 = sh_box[0], by0 = sh_box[1], bw = sh_box[2], bh = sh_box[3];
-    for (int j = t0; j < bw * bh; j += step) {
-      const int cx = j % bw, cy = j / bw;
-      const int n0 = bx0 + cx, n1 = by0 + cy;
-      const int l = (n0 - ox) + tw * (n1 - oy);
-      const double xx[2] = {G.min[0] + (double)n0 * G.dx[0], G.min[1] + (double)n1 * G.dx[1]};
-      double v = tv[l], gx = tdx[l], gy = tdy[l];
-      for (int k = 0; k < nb; k++) {
-        if (abs(n0 - sh_ind[b][k][0]) <= nn0 && abs(n1 - sh_ind[b][k][1]) <= nn1) {
-          // gauss_shape_f2 with the factors from the tables, then gauss_apply
-          double dp[2];
-          dp[0] = gscaled(G, 0, sh_c[b][k][0], xx[0]);
-          dp[1] = gscaled(G, 1, sh_c[b][k][1], xx[1]);
-          double dp2 = dp[0] * dp[0];
-          dp2 += dp[1] * dp[1];
-          dp2 *= 0.5;
-          double bb = 0.0, d[2] = {0.0, 0.0};
-          if (dp2 < 6.25) bb = gauss_apply<2>(G, dp, sh_f[k][cx] * sh_f[k][bw + cy], sh_h[b][k], d);
-          v += bb;
-          gx += d[0];
-          gy += d[1];
-        }
-      }
-      tv[l] = v;
-      tdx[l] = gx;
-      tdy[l] = gy;
-    }
-  };
-
-  // the old tile written back, the tile at sh_nox/noy read
-  auto reload = [&]() {
-    flush();
-    // the tile written above may overlap the one read below
-    __threadfence();
-    __syncthreads();
-    ox = sh_nox;
-    oy = sh_noy;
-    for (int j = t; j < tw * th; j += blockDim.x) {
-      const int lx = j % tw, ly = j / tw;
-      const long long node = (long long)(oy + ly) * nx + (ox + lx);
-      const int l = lx + tw * ly;
-      tv[l] = val[node];
-      tdx[l] = der[2 * node];
-      tdy[l] = der[2 * node + 1];
-    }
-    __syncthreads();
-  };
-
-  long long k0 = 0;  // first hill not yet in a run
-  int cb = 0;        // buffer of the current run
-  int nbc = 0;       // hills of the current run (heights known, not on the tile)
-  // wave 0: the centres of the hills the next run decision starts with,
-  // loaded while the heights of the next run are found
-  bool pre = false;
-  double pc0 = 0.0, pc1 = 0.0;
-  auto prefetch = [&](long long kn) {
-    pre = true;
-    const long long k = kn + lane;
-    if (lane < kRun && k < nhills) {
-      pc0 = centers[2 * k];
-      pc1 = centers[2 * k + 1];
-    }
-  };
-  while (true) {
-    if (wave0) decide(k0, 1 - cb, pre, pc0, pc1);
-    __syncthreads();
-    const int nbn = sh_nb;  // uniform; 0: no hill left, or the next is outside the grid
-    const bool fit = sh_fit;
-    if (nbc > 0 && nbn > 0) {
-      // the next run's corners: the grid before the current run (tile, or
-      // memory outside it, which the current run does not touch), then the
-      // current run's hills in order (at the start of the chain); the next
-      // run's own shapes; the current run's factors
-      shapes(cb, nbc, 1 - cb, nbn, sh_ex);
-      shapes(1 - cb, nbn, 1 - cb, nbn, sh_e);
-      snapshot(1 - cb, nbn);
-      factors(cb, nbc);
-      __syncthreads();
-      // wave 0: the next run's heights; the other waves: the current run
-      if (wave0) {
-        prefetch(k0 + nbn);
-        chain(1 - cb, nbn, k0, nbc);
-      } else {
-        deposit(cb, nbc, t - WAVE_M, (int)blockDim.x - WAVE_M);
-      }
-      __syncthreads();
-      // the next run lies in another tile
-      if (!fit) reload();
-    } else {
-      // the first run, the end, or a hill outside the grid: in sequence
-      if (nbc > 0) {
-        factors(cb, nbc);
-        __syncthreads();
-        deposit(cb, nbc, t, blockDim.x);
-        __syncthreads();
-      }
-      if (nbn == 0) break;
-      if (!fit) reload();
-      shapes(1 - cb, nbn, 1 - cb, nbn, sh_e);
-      snapshot(1 - cb, nbn);
-      __syncthreads();
-      if (wave0) {
-        prefetch(k0 + nbn);
-        chain(1 - cb, nbn, k0, 0);
-      }
-      __syncthreads();
-    }
-    cb = 1 - cb;
-    nbc = nbn;
-    k0 += nbn;
+    K.n[i] = n;
+    const int x0 = n == ind[i] ? 0 : 1;
+    const double dx = G.dx[i];
+    K.x[i] = G.min[i] + (double)n * dx;
+    const double X = fabs((c[i] - (G.min[i] + (double)ind[i] * dx)) / dx - (double)x0);
+    const double X2 = X * X, X3 = X2 * X;
+    K.A[i] = 1.0 - 3.0 * X2 + 2.0 * X3;
+    K.S[i] = (x0 ? -1.0 : 1.0) * (X - 2.0 * X2 + X3) * dx;
   }
-  flush();
+  return K;
+}
+template <int NCV>
+__device__ __forceinline__ long long corner_node(const GridArg& G, const Corner<NCV>& K) {
+  long long node = K.n[NCV - 1];
+#pragma unroll
+  for (int i = NCV - 1; i > 0; --i) node = node * G.nbin[i - 1] + K.n[i - 1];
+  return node;
+}
+// the spline term from the node's value g and gradient d: the product of
+// A_j g + S_j d_j over a power of g, so that one reciprocal is all the division
+// on the way from one height to the next; below 1e-7 the gradient does not
+// count (an absent corner has g = 0 and gives 0)
+template <int NCV>
+__device__ __forceinline__ double corner_term(const Corner<NCV>& K, double g, const double* d) {
+  double flat = g, v = fma(K.S[0], d[0], K.A[0] * g);
+  double r = 1.0;
+  if constexpr (NCV > 1) {
+    const double r1 = rcp64(g);
+    r = r1;
+#pragma unroll
+    for (int i = 2; i < NCV; i++) r *= r1;
+  }
+#pragma unroll
+  for (int i = 0; i < NCV; i++) flat *= K.A[i];
+#pragma unroll
+  for (int i = 1; i < NCV; i++) v *= fma(K.S[i], d[i], K.A[i] * g);
+  v *= r;
+  return fabs(g) < 0.0000001 ? flat : v;
+}
+
+// Hills one after the other in one workgroup: per hill, one wave evaluates
+// the 2^NCV spline corners and the height, then the workgroup adds the hill,
+// one support node per thread (two L2 round trips a hill).  For the few
+// hills of a run in progress, and for periodic supports wider than the
+// grid.  Bit for bit the heights and the grid of the kernels below.
+constexpr int kSeqThreads = 1024;
+template <int NCV>
+__global__ __launch_bounds__(kSeqThreads) void k_deposit_seq(GridArg G, double* __restrict__ val,
+                                                             double* __restrict__ der, long long nhills,
+                                                             const double* __restrict__ centers,
+                                                             double* __restrict__ heights, int* __restrict__ err) {
+  __shared__ double sh_h;
+  const int t = threadIdx.x;
+  for (long long k = 0; k < nhills; k++) {
+    double c[kMaxCv];
+    unsigned ind[kMaxCv];
+    for (int i = 0; i < NCV; i++) c[i] = centers[k * NCV + i];
+    const bool ok = grid_index_of(G, c, ind) >= 0;  // uniform
+    if (t < WAVE_M) {
+      double v = 0.0;
+      if (ok && G.welltemp && t < (1 << NCV)) {
+        int in[NCV];
+        for (int i = 0; i < NCV; i++) in[i] = (int)ind[i];
+        const Corner<NCV> K = corner_of<NCV>(G, c, in, t);
+        if (K.has) {
+          const long long node = corner_node<NCV>(G, K);
+          double d[NCV];
+          for (int i = 0; i < NCV; i++) d[i] = der[node * NCV + i];
+          v = corner_term<NCV>(K, val[node], d);
+        }
+      }
+      v = corner_sum<NCV>(v);
+      if (t == 0) {
+        const double h = (ok && G.welltemp) ? wt_height(G, v) : G.height0;
+        if (!ok) atomicCAS(err, 0, (int)(1 + (k < 0x3fffffff ? k : 0x3fffffff)));
+        sh_h = h;
+        if (heights) heights[k] = ok ? h : 0.0;
+      }
+    }
+    __syncthreads();
+    if (!ok) return;
+    add_hill_block<NCV>(G, val, der, ind, c, sh_h);
+    __syncthreads();
+  }
+}
+
+// Many hills: epochs of kChainThreads / 2^NCV hills (256 with two CVs), two
+// launches each.
+//  - k_hill_chain finds the epoch's heights in one workgroup.  Thread t holds
+//    corner t mod 2^NCV of hill t / 2^NCV in registers: its value and gradient
+//    on the grid before the epoch, to which every earlier hill of the epoch is
+//    added as soon as its height is known.  Wave w owns a run of
+//    64 / 2^NCV hills: it finds their heights alone, one after the other (the
+//    corners of hill k give its height, then all later corners of the wave
+//    take hill k), and the later waves follow hill by hill through LDS, so
+//    that the next wave is one hill behind when its turn comes.
+//    The other workgroups of the launch evaluate the next epoch's shapes,
+//    which depend on the centres only: those exponentials are off the chain.
+//  - k_hill_nodes adds the epoch to the grid, a thread per node with the
+//    hills in order.
+// Bound by the latency of the chain height -> corners -> reciprocal ->
+// exponential -> height on one wave (0.23 us a hill: some 22 dependent FP64
+// operations).  Measured, one workgroup doing everything before -> this: 4,000
+// hills on two open CVs (513 x 513 nodes) 4.93 ms -> 0.93 ms (heights) + 0.30 ms
+// (grid); 500 hills on two torsions (100 x 100) 3.60 -> 0.21 ms.
+constexpr int kChainThreads = 1024;
+constexpr int kSeqHills = 4;  // at most this many hills go one after the other
+
+// cells of the hill centres (-1: outside the grid)
+template <int NCV>
+__global__ __launch_bounds__(256) void k_hill_cells(GridArg G, long long n, const double* __restrict__ centers,
+                                                    int* __restrict__ cells) {
+  const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  double c[kMaxCv];
+  unsigned ind[kMaxCv];
+  for (int i = 0; i < NCV; i++) c[i] = centers[k * NCV + i];
+  const bool ok = grid_index_of(G, c, ind) >= 0;
+  for (int i = 0; i < NCV; i++) cells[k * NCV + i] = ok ? (int)ind[i] : -1;
+}
+
+// node n within the support of a hill in bin `ind`
+__device__ __forceinline__ bool in_support(const GridArg& G, int i, int n, int ind) {
+  int d = abs(n - ind);
+  if (G.pbc[i]) d = min(d, (int)G.nbin[i] - d);
+  return d <= G.nneigh[i];
+}
+
+// hills of one epoch: their first index and count, centres and cells
+struct Epoch {
+  long long k0;
+  int n;
+  const double* centers;  // of the whole call
+  const int* cells;
+};
+
+template <int NCV, bool PER>
+__global__ __launch_bounds__(kChainThreads) void k_hill_chain(GridArg G, const double* __restrict__ val,
+                                                              const double* __restrict__ der, Epoch E,
+                                                              const double* __restrict__ shapes, Epoch N,
+                                                              double* __restrict__ shapes_next, int first,
+                                                              int* __restrict__ state, double* __restrict__ hbuf,
+                                                              double* __restrict__ heights, int* __restrict__ err) {
+  constexpr int NN = 1 << NCV;
+  constexpr int R = WAVE_M / NN;           // hills of one run
+  constexpr int RC = R < 16 ? R : 16;      // hills whose shapes are in registers at once
+  constexpr int EH = kChainThreads / NN;   // hills of one epoch
+  const int t = threadIdx.x;
+  const int r = t / NN, q = t % NN;
+  if (blockIdx.x > 0) {
+    // row j of the next epoch's shapes: hill j at the corners of the later hills
+    const int j = (int)blockIdx.x - 1;
+    if (j >= N.n || r / R < j / R) return;
+    double e = -1.0;
+    if (j < r && r < N.n) {
+      const long long kj = N.k0 + j, kr = N.k0 + r;
+      HillDim H[NCV];
+      bool in = true;
+#pragma unroll
+      for (int i = 0; i < NCV; i++) {
+        int n = N.cells[kr * NCV + i] + ((q >> i) & 1);
+        if (n >= (int)G.nbin[i]) {
+          if (G.pbc[i]) n = 0;
+          else in = false;
+        }
+        in = in && in_support(G, i, n, N.cells[kj * NCV + i]);
+        H[i] = hill_dim<PER>(G, i, N.centers[kj * NCV + i], G.min[i] + (double)n * G.dx[i]);
+      }
+      if (in) e = hill_shape<NCV>(H);
+    }
+    shapes_next[(size_t)j * kChainThreads + t] = e;
+    return;
+  }
+  if (E.n == 0) return;
+  __shared__ double sh_c[EH][NCV], sh_h[EH];
+  __shared__ int sh_bad;
+  const int lane = t & (WAVE_M - 1);
+  const int w = __builtin_amdgcn_readfirstlane(t / WAVE_M);
+  // state[0..1]: hills of the epoch before the first one outside the grid;
+  // state[2..3]: that one has been met (this epoch's parity and the last's)
+  const int par = (int)((E.k0 / EH) & 1);
+  const bool stopped = !first && state[2 + (1 - par)] != 0;
+  if (t == 0) sh_bad = stopped ? 0 : E.n;
+  // a height not found yet: a NaN with a payload that only an input could
+  // carry on, and the inputs' NaNs lose theirs below; so the word itself tells
+  // the followers
+  constexpr long long kPending = 0x7ff8c0ffee0dd001ll;
+  auto plain = [](double x) { return x == x ? x : __builtin_nan(""); };
+  if (t < EH) sh_h[t] = __longlong_as_double(kPending);
+  __syncthreads();
+  if (t < E.n) {
+    bool ok = true;
+    for (int i = 0; i < NCV; i++) {
+      ok = ok && E.cells[(E.k0 + t) * NCV + i] >= 0;
+      sh_c[t][i] = E.centers[(E.k0 + t) * NCV + i];
+    }
+    if (!ok) atomicMin(&sh_bad, t);
+  }
+  __syncthreads();
+  const int cnt = __builtin_amdgcn_readfirstlane(sh_bad);
+  if (t == 0) {
+    state[par] = cnt;
+    state[2 + par] = cnt < E.n;
+    if (!stopped && cnt < E.n) {
+      const long long k = E.k0 + cnt;
+      atomicCAS(err, 0, (int)(1 + (k < 0x3fffffff ? k : 0x3fffffff)));
+      if (heights) heights[k] = 0.0;
+    }
+  }
+  double* hb = hbuf + (size_t)par * EH;
+  if (!G.welltemp) {
+    if (t < cnt) {
+      hb[t] = G.height0;
+      if (heights) heights[E.k0 + t] = G.height0;
+    }
+    return;
+  }
+  if (w * R < cnt) {
+    // this thread's corner on the grid before the epoch
+    const bool mine = r < cnt;
+    Corner<NCV> K;
+    double g = 0.0, d[NCV];
+    {
+      double c[NCV];
+      int ind[NCV];
+#pragma unroll
+      for (int i = 0; i < NCV; i++) {
+        c[i] = mine ? sh_c[r][i] : G.min[i];
+        ind[i] = mine ? E.cells[(E.k0 + r) * NCV + i] : 0;
+        d[i] = 0.0;
+      }
+      K = corner_of<NCV>(G, c, ind, q);
+      if (mine && K.has) {
+        const long long node = corner_node<NCV>(G, K);
+        g = plain(val[node]);
+#pragma unroll
+        for (int i = 0; i < NCV; i++) d[i] = plain(der[node * NCV + i]);
+      }
+    }
+    // constants of the chain in registers
+    ExpK C;
+    double height0 = plain(G.height0), inv_wt = plain(G.inv_wt);
+    double inv_wt2 = inv_wt * C.log2e;
+    double sA = G.stretchA, sB = G.stretchB;
+    asm volatile("" : "+s"(C.hi), "+s"(C.lo), "+s"(sA), "+v"(sB), "+v"(height0), "+v"(inv_wt), "+v"(inv_wt2));
+#pragma unroll
+    for (int i = 0; i < 6; i++) asm volatile("" : "+s"(C.m[i]));
+#pragma unroll
+    for (int i = 0; i < 5; i++) asm volatile("" : "+v"(C.a[i]));
+    const double* sh = shapes + t;
+    auto load = [&](int b, double* e) {
+#pragma unroll
+      for (int k = 0; k < RC; k++) e[k] = b + k < cnt ? sh[(size_t)(b + k) * kChainThreads] : -1.0;
+    };
+    // the terms of hill k of shape e at this thread's corner, all but the
+    // height (0 outside the support), formed where this stands
+    auto terms = [&](int k, double e, double& tv, double* td) {
+      const bool in = e >= 0.0;
+      tv = in ? fma(sA, e, sB) : 0.0;
+      const double ez = in ? e : 0.0;
+      double c[NCV];
+#pragma unroll
+      for (int i = 0; i < NCV; i++) c[i] = sh_c[k][i];
+#pragma unroll
+      for (int i = 0; i < NCV; i++) td[i] = ez * (hill_scaled<PER>(G, i, c[i], K.x[i]) * G.kd[i]);
+      asm volatile("" : "+v"(tv));
+#pragma unroll
+      for (int i = 0; i < NCV; i++) asm volatile("" : "+v"(td[i]));
+    };
+    auto apply = [&](double h, double tv, const double* td) {
+      g = fma(h, tv, g);
+#pragma unroll
+      for (int i = 0; i < NCV; i++) d[i] = fma(h, td[i], d[i]);
+    };
+    // height k of an earlier wave, as soon as it is there (every wave of the
+    // workgroup is resident and only waits for earlier ones)
+    auto height = [&](int k) {
+      while (true) {
+        const double h = __hip_atomic_load(&sh_h[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (__double_as_longlong(h) != kPending) return h;
+        __builtin_amdgcn_s_sleep(1);
+      }
+    };
+    // the hills [b, b + RC) of an earlier wave, each as soon as it is there
+    auto follow = [&](int b, const double* e) {
+#pragma unroll
+      for (int k = 0; k < RC; k++) {
+        if (__ballot(e[k] >= 0.0) == 0ull) continue;
+        double tv, td[NCV];
+        terms(b + k, e[k], tv, td);
+        const double h = height(b + k);
+        if (e[k] >= 0.0) apply(h, tv, td);
+      }
+    };
+    double ex[RC], eo[RC];
+    const int b0 = w * R;
+    for (int b = 0; b + RC < b0; b += RC) {
+      load(b, ex);
+      follow(b, ex);
+    }
+    if (b0 > 0) load(b0 - RC, ex);
+    load(b0, eo);
+    if (b0 > 0) {
+      follow(b0 - RC, ex);
+      (void)height(b0 - 1);
+    }
+    __builtin_amdgcn_s_setprio(3);
+    for (int c = 0; c < R / RC; c++) {
+      const int b = b0 + c * RC;
+      if (c > 0) load(b, eo);
+      // (the hills of this wave's earlier chunks are in: every lane took them)
+      double tv, td[NCV];
+      terms(b, eo[0], tv, td);
+#pragma unroll
+      for (int k = 0; k < RC; k++) {
+        if (b + k < cnt) {
+          const double V = readlane_d(corner_sum<NCV>(corner_term<NCV>(K, g, d)), NN * (c * RC + k));
+          // the next hill's terms fill the waits of this hill's exponential
+          double tn = 0.0, dn[NCV];
+          if (k + 1 < RC) terms(b + k + 1, eo[k + 1], tn, dn);
+          double h = wt_fast(height0, inv_wt, inv_wt2, V, C);
+          if (__builtin_expect(!wt_in_range(inv_wt, V), 0)) {
+            h = height0 * exp(-V * inv_wt);
+            if (eo[k] >= 0.0) apply(h, tv, td);
+          } else {
+            apply(h, tv, td);
+          }
+          if (lane == 0) __hip_atomic_store(&sh_h[b + k], h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          tv = tn;
+#pragma unroll
+          for (int i = 0; i < NCV; i++) td[i] = k + 1 < RC ? dn[i] : 0.0;
+        }
+      }
+    }
+    __builtin_amdgcn_s_setprio(0);
+  }
+  __syncthreads();
+  if (t < cnt) {
+    hb[t] = sh_h[t];
+    if (heights) heights[E.k0 + t] = sh_h[t];
+  }
+}
+
+// tiles of 64 nodes (one wave): the smaller the tile, the fewer hills it meets
+template <int NCV>
+__host__ __device__ constexpr int tile_dim(int i) {
+  return NCV == 1 ? 64 : NCV == 2 ? 8 : NCV == 3 ? 4 : (i < 2 ? 4 : 2);
+}
+
+// The hills of one epoch onto the grid: a workgroup per tile, which lists the
+// hills that reach it (in order) and tabulates HillDim of each along the
+// tile's sides; wave 0 then takes its nodes' hills in order, four at a time up
+// to the addition, while the other waves tabulate the next hills.  Bound by
+// wave 0's walk through the hills of the busiest tiles.  Tiles that no hill
+// reaches leave after the list.
+template <int NCV, bool PER>
+__global__ __launch_bounds__(256) void k_hill_nodes(GridArg G, double* __restrict__ val, double* __restrict__ der,
+                                                    Epoch E, const int* __restrict__ state,
+                                                    const double* __restrict__ hbuf) {
+  constexpr int EH = kChainThreads >> NCV;
+  constexpr int ST = NCV == 1 ? 64 : NCV == 2 ? 16 : 12;  // sum of the tile's sides
+  constexpr int CH = NCV == 1 ? 8 : 32;                   // hills tabulated at once
+  constexpr int U = 4;
+  // the hills that reach the tile, in order: cell, centre, height
+  __shared__ int lcell[EH][NCV];
+  __shared__ double lx[EH][NCV], lh[EH];
+  __shared__ int wcnt[4];
+  __shared__ double2 tsf[2][CH][ST];
+  __shared__ double tw[2][CH][ST];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int par = (int)((E.k0 / EH) & 1);
+  const double* hb = hbuf + (size_t)par * EH;
+  int o[NCV];
+  {
+    long long b = blockIdx.x;
+#pragma unroll
+    for (int i = 0; i < NCV; i++) {
+      const int nt = ((int)G.nbin[i] + tile_dim<NCV>(i) - 1) / tile_dim<NCV>(i);
+      o[i] = (int)(b % nt) * tile_dim<NCV>(i);
+      b /= nt;
+    }
+  }
+  // everything the tile may need from memory goes out before the first wait:
+  // the epoch's hills (E.n of them, valid or not), their count, wave 0's node
+  constexpr int HP = (EH + 255) / 256;
+  int cell[HP][NCV];
+  double x[HP][NCV], hh[HP];
+#pragma unroll
+  for (int p = 0; p < HP; p++) {
+    const int h = min(p * 256 + t, E.n - 1);
+    hh[p] = hb[h];
+#pragma unroll
+    for (int i = 0; i < NCV; i++) {
+      cell[p][i] = E.cells[(E.k0 + h) * NCV + i];
+      x[p][i] = E.centers[(E.k0 + h) * NCV + i];
+    }
+  }
+  int l[NCV];
+  bool valid = w == 0;
+  long long node = 0;
+  {
+    int q = lane, base = 0, n[NCV];
+#pragma unroll
+    for (int i = 0; i < NCV; i++) {
+      const int a = q % tile_dim<NCV>(i);
+      q /= tile_dim<NCV>(i);
+      n[i] = o[i] + a;
+      l[i] = base + a;
+      base += tile_dim<NCV>(i);
+      valid = valid && n[i] < (int)G.nbin[i];
+    }
+    node = n[NCV - 1];
+#pragma unroll
+    for (int i = NCV - 1; i > 0; --i) node = node * G.nbin[i - 1] + n[i - 1];
+  }
+  double v = 0.0, d[NCV];
+#pragma unroll
+  for (int i = 0; i < NCV; i++) d[i] = 0.0;
+  if (valid) {
+    v = val[node];
+#pragma unroll
+    for (int i = 0; i < NCV; i++) d[i] = der[node * NCV + i];
+  }
+  const int cnt = state[par];
+  int nl = 0;
+#pragma unroll
+  for (int p = 0; p < HP; p++) {
+    bool hit = p * 256 + t < cnt;
+#pragma unroll
+    for (int i = 0; i < NCV; i++) {
+      const int T = min(tile_dim<NCV>(i), (int)G.nbin[i] - o[i]);
+      int s = o[i] - (cell[p][i] - G.nneigh[i]);  // the tile's first node from the support's first
+      if (PER && G.pbc[i]) {
+        const int N = (int)G.nbin[i];
+        if (s < 0) s += N;  // |o - cell| < N and the support is no wider than the grid
+        else if (s >= N) s -= N;
+        hit = hit && (s <= 2 * G.nneigh[i] || s + T - 1 >= N);
+      } else {
+        hit = hit && s <= 2 * G.nneigh[i] && s + T - 1 >= 0;
+      }
+    }
+    const unsigned long long m = __ballot(hit);
+    if (lane == 0) wcnt[w] = __popcll(m);
+    __syncthreads();
+    int at = nl;
+    for (int q = 0; q < 4; q++) {
+      if (q < w) at += wcnt[q];
+      nl += wcnt[q];
+    }
+    if (hit) {
+      at += __popcll(m & ((1ull << lane) - 1));
+      lh[at] = hh[p];
+#pragma unroll
+      for (int i = 0; i < NCV; i++) {
+        lcell[at][i] = cell[p][i];
+        lx[at][i] = x[p][i];
+      }
+    }
+    __syncthreads();
+  }
+  if (nl == 0) return;
+  // the tables of the hills [c0, c0 + CH) of the list, by threads q0, q0 + step, ...
+  auto tabulate = [&](int c0, int buf, int q0, int step) {
+    const int nc = min(CH, nl - c0);
+    for (int p = q0; p < nc * ST; p += step) {
+      const int c = p / ST;
+      int m = p % ST, i = 0;
+#pragma unroll
+      for (int u = 0; u < NCV - 1; u++)
+        if (i == u && m >= tile_dim<NCV>(u)) {
+          m -= tile_dim<NCV>(u);
+          i = u + 1;
+        }
+      // a distance beyond the cutoff marks the nodes outside the support
+      HillDim H = {1.0e3, 0.0, 0.0};
+#pragma unroll
+      for (int u = 0; u < NCV; u++) {
+        if (i != u) continue;
+        const int nd = o[u] + m;
+        if (nd < (int)G.nbin[u] && in_support(G, u, nd, lcell[c0 + c][u]))
+          H = hill_dim<PER>(G, u, lx[c0 + c][u], G.min[u] + (double)nd * G.dx[u]);
+      }
+      tsf[buf][c][p % ST] = make_double2(H.s, H.f);
+      tw[buf][c][p % ST] = H.w;
+    }
+  };
+  tabulate(0, 0, t, 256);
+  __syncthreads();
+  for (int c0 = 0, buf = 0; c0 < nl; c0 += CH, buf ^= 1) {
+    if (w > 0) {
+      tabulate(c0 + CH, buf ^ 1, t - WAVE_M, 256 - WAVE_M);
+    } else {
+      const int nc = min(CH, nl - c0);
+      // the next hills' entries are on their way while these are added
+      HillDim H[U][NCV];
+      double h[U];
+      auto fetch = [&](int cc) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const int c = min(cc + u, nc - 1);
+          h[u] = lh[c0 + c];
+#pragma unroll
+          for (int i = 0; i < NCV; i++) {
+            const double2 y = tsf[buf][c][l[i]];
+            H[u][i] = {y.x, y.y, tw[buf][c][l[i]]};
+          }
+        }
+      };
+      fetch(0);
+      for (int cc = 0; cc < nc; cc += U) {
+        double e[U], tv[U], td[U][NCV], hc[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          e[u] = hill_shape<NCV>(H[u]);
+          tv[u] = fma(G.stretchA, e[u], G.stretchB);
+#pragma unroll
+          for (int i = 0; i < NCV; i++) td[u][i] = e[u] * H[u][i].w;
+          if (cc + u >= nc) e[u] = -1.0;
+          hc[u] = h[u];
+        }
+        fetch(cc + U);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          if (e[u] >= 0.0) {
+            asm volatile("");  // masked lanes, not selects
+            v = fma(hc[u], tv[u], v);
+#pragma unroll
+            for (int i = 0; i < NCV; i++) d[i] = fma(hc[u], td[u][i], d[i]);
+          }
+        }
+      }
+    }
+    __syncthreads();
+  }
+  if (!valid) return;
+  val[node] = v;
+#pragma unroll
+  for (int i = 0; i < NCV; i++) der[node * NCV + i] = d[i];
 }
 
 // hills of given heights, in parallel (one block per hill)
@@ -926,7 +1079,12 @@ __global__ __launch_bounds__(kDepositThreads) void k_metad_step(GridArg G, doubl
     ind[i] = sh_ind[i];
     c[i] = sh_c[i];
   }
-  add_hill_block(G, val, der, ind, c, sh_h);
+  switch (G.ncv) {
+  case 1: add_hill_block<1>(G, val, der, ind, c, sh_h); break;
+  case 2: add_hill_block<2>(G, val, der, ind, c, sh_h); break;
+  case 3: add_hill_block<3>(G, val, der, ind, c, sh_h); break;
+  default: add_hill_block<4>(G, val, der, ind, c, sh_h); break;
+  }
 }
 
 __global__ void k_apply_force(long long natoms, const double* __restrict__ f, const double* __restrict__ deriv,
@@ -951,6 +1109,13 @@ struct p2a_metad {
   int* err = nullptr;
   double* scratch = nullptr;  // staging for host-array entry points
   size_t scratch_n = 0;
+  // workspace of the deposition in epochs: cells of the hills, shapes of two
+  // epochs, heights of two epochs, two epochs' counts
+  int* cells = nullptr;
+  size_t cells_n = 0;
+  double* shapes = nullptr;  // one block: shapes, then hbuf, then state
+  double* hbuf = nullptr;
+  int* state = nullptr;
   bool first_step = true;
 };
 
@@ -964,6 +1129,72 @@ static int metad_scratch(p2a_metad* m, size_t n) {
   if (hipMalloc(&m->scratch, n * sizeof(double)) != hipSuccess) return fail(P2A_ERR_NOMEM, "hipMalloc failed");
   m->scratch_n = n;
   return P2A_OK;
+}
+
+// The workspace of the deposition in epochs for nhills hills; false when it
+// cannot be had (memory, or a stream under capture, where nothing may be
+// allocated): the hills then go one after the other.
+static bool epoch_workspace(p2a_metad* m, size_t nhills) {
+  const size_t want = nhills * m->G.ncv;
+  const bool ready = m->shapes && m->cells_n >= want;
+  if (ready) return true;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(m->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return false;
+  }
+  const size_t eh = kChainThreads >> m->G.ncv;
+  auto get = [](void** p, size_t bytes) {
+    if (*p) return true;
+    if (hipMalloc(p, bytes) == hipSuccess) return true;
+    *p = nullptr;
+    (void)hipGetLastError();
+    return false;
+  };
+  if (m->cells_n < want) {
+    if (m->cells) (void)hipFree(m->cells);
+    m->cells = nullptr;
+    m->cells_n = 0;
+    if (!get((void**)&m->cells, want * sizeof(int))) return false;
+    m->cells_n = want;
+  }
+  const size_t nshape = 2 * eh * kChainThreads, nheight = 2 * eh;
+  if (!get((void**)&m->shapes, (nshape + nheight) * sizeof(double) + 4 * sizeof(int))) return false;
+  m->hbuf = m->shapes + nshape;
+  m->state = (int*)(m->hbuf + nheight);
+  return true;
+}
+
+template <int NCV>
+static void deposit_seq(p2a_metad* m, int64_t nhills, const double* centers, double* heights) {
+  hipLaunchKernelGGL(k_deposit_seq<NCV>, dim3(1), dim3(kSeqThreads), 0, m->stream, m->G, m->val, m->der,
+                     (long long)nhills, centers, heights, m->err);
+}
+
+template <int NCV, bool PER>
+static void deposit_epochs(p2a_metad* m, int64_t nhills, const double* centers, double* heights) {
+  constexpr int EH = kChainThreads >> NCV;
+  const GridArg& G = m->G;
+  hipStream_t s = m->stream;
+  long long tiles = 1;
+  for (int i = 0; i < NCV; i++) tiles *= (G.nbin[i] + tile_dim<NCV>(i) - 1) / tile_dim<NCV>(i);
+  hipLaunchKernelGGL(k_hill_cells<NCV>, dim3((unsigned)((nhills + 255) / 256)), dim3(256), 0, s, G,
+                     (long long)nhills, centers, m->cells);
+  const int64_t ne = (nhills + EH - 1) / EH;
+  // launch e finds the heights of epoch e and the shapes of epoch e + 1; e = -1: shapes only
+  for (int64_t e = -1; e < ne; e++) {
+    Epoch E = {e < 0 ? 0 : e * EH, e < 0 ? 0 : (int)std::min<int64_t>(EH, nhills - e * EH), centers, m->cells};
+    Epoch N = {(e + 1) * EH, e + 1 < ne ? (int)std::min<int64_t>(EH, nhills - (e + 1) * EH) : 0, centers, m->cells};
+    const int rows = G.welltemp ? N.n : 0;
+    if (E.n == 0 && rows == 0) continue;
+    const size_t half = (size_t)EH * kChainThreads;
+    hipLaunchKernelGGL((k_hill_chain<NCV, PER>), dim3(1 + rows), dim3(kChainThreads), 0, s, G, m->val, m->der, E,
+                       m->shapes + (e & 1) * half, N, m->shapes + ((e + 1) & 1) * half, e == 0 ? 1 : 0, m->state,
+                       m->hbuf, heights, m->err);
+    if (E.n > 0)
+      hipLaunchKernelGGL((k_hill_nodes<NCV, PER>), dim3((unsigned)tiles), dim3(256), 0, s, G, m->val, m->der, E, m->state,
+                         m->hbuf);
+  }
 }
 
 static int metad_read_err(p2a_metad* m, const char* what) {
@@ -1026,6 +1257,7 @@ int p2a_metad_create(p2a_metad** out, int device, const p2a_metad_spec* spec) {
   // dp2cutoff stretch (Tools.h:71-79, MetaD.cpp:762-765)
   G.stretchA = spec->nostretch ? 1.0 : 1.00193418799744762399;
   G.stretchB = spec->nostretch ? 0.0 : -.00193418799744762399;
+  for (int i = 0; i < ncv; i++) G.kd[i] = -(G.invsigma[i] * G.stretchA);
   int ndev = 0;
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) return fail(P2A_ERR_HIP, "no HIP device available");
   if (device < 0 || device >= ndev) return fail(P2A_ERR_ARG, "device index out of range");
@@ -1064,6 +1296,8 @@ int p2a_metad_destroy(p2a_metad* m) {
   if (m->der) (void)hipFree(m->der);
   if (m->err) (void)hipFree(m->err);
   if (m->scratch) (void)hipFree(m->scratch);
+  if (m->cells) (void)hipFree(m->cells);
+  if (m->shapes) (void)hipFree(m->shapes);
   if (m->own_stream) (void)hipStreamDestroy(m->own_stream);
   delete m;
   return P2A_OK;
@@ -1083,30 +1317,25 @@ int p2a_metad_deposit_device(p2a_metad* m, int64_t nhills, const double* centers
   if (nhills <= 0) return P2A_OK;
   P2A_HIPM(hipSetDevice(m->device));
   const GridArg& G = m->G;
-  // LDS tile of the 2-CV kernel: shaped like the hill support (a walk
-  // crosses it in a number of hills about equal along both CVs), at least
-  // two supports plus the spline corner wide, within the grid
-  int tw = 0, th = 0;
-  bool tile2 = G.ncv == 2 && !G.pbc[0] && !G.pbc[1] && !G.may_alias;
-  if (tile2) {
-    const int nx = (int)G.nbin[0], ny = (int)G.nbin[1];
-    const int need0 = 2 * G.nneigh[0] + 4, need1 = 2 * G.nneigh[1] + 4;
-    const double a0 = 2.0 * G.nneigh[0] + 1.0, a1 = 2.0 * G.nneigh[1] + 1.0;
-    tw = std::min(nx, std::max(need0, (int)std::floor(std::sqrt(kTileNodes * a0 / a1))));
-    th = std::min(ny, kTileNodes / std::max(tw, 1));
-    if (th < need1) {
-      th = std::min(ny, need1);
-      tw = std::min(nx, kTileNodes / th);
-    }
-    tile2 = tw >= std::min(nx, need0) && th >= std::min(ny, need1) && tw * th <= kTileNodes && tw + th <= kFacLen &&
-            need0 <= nx && need1 <= ny;
-  }
-  if (tile2)
-    hipLaunchKernelGGL(k_deposit_seq_tile2, dim3(1), dim3(kSeqThreads), 0, m->stream, m->G, m->val, m->der,
-                       (long long)nhills, centers_dev, heights_dev, m->err, tw, th);
-  else
-    hipLaunchKernelGGL(k_deposit_seq, dim3(1), dim3(kSeqThreads), 0, m->stream, m->G, m->val, m->der,
-                       (long long)nhills, centers_dev, heights_dev, m->err);
+  // A few hills: one workgroup, one launch (a host call with 1 / 2 hills takes
+  // 41 / 44 us, in epochs 51 us for 3 and 53 us for 8).  More: in epochs,
+  // unless a periodic support is wider than the grid (a node would count
+  // twice) or the grid's tiles exceed a launch.
+  const bool epochs = nhills > kSeqHills && !G.may_alias && m->size < ((size_t)1 << 36) &&
+                      epoch_workspace(m, (size_t)nhills);
+  bool per = false;
+  for (int i = 0; i < G.ncv; i++) per = per || G.pbc[i];
+#define P2A_DEP(N)                                                       \
+  do {                                                                   \
+    if (epochs && per) deposit_epochs<N, true>(m, nhills, centers_dev, heights_dev); \
+    else if (epochs) deposit_epochs<N, false>(m, nhills, centers_dev, heights_dev);  \
+    else deposit_seq<N>(m, nhills, centers_dev, heights_dev);            \
+  } while (0)
+  if (G.ncv == 1) P2A_DEP(1);
+  else if (G.ncv == 2) P2A_DEP(2);
+  else if (G.ncv == 3) P2A_DEP(3);
+  else P2A_DEP(4);
+#undef P2A_DEP
   P2A_HIPM(hipGetLastError());
   return P2A_OK;
 }
