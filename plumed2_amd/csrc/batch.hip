@@ -159,7 +159,7 @@ static int batch_step(p2a_batch* b, const double* pos, double* values, double* d
                        (const int*)A.nitems_dev, b->items_cap, (const int4*)b->items.p, nw, b->wave_start.p);
     A.wave_start = b->wave_start.p;
   }
-  launch_pairs(A, grid, s, false, chunk, b->items.p, b->ents.p, b->p.p, b->p.p, b->bb.p, b->bb.p, (const int*)nullptr,
+  launch_pairs<false>(A, grid, s, false, chunk, b->items.p, b->ents.p, b->p.p, b->p.p, b->bb.p, b->bb.p, (const int*)nullptr,
                (const int*)nullptr, b->fpart.p, b->partial.p);
   if ((rc = launch_check("batch: pair kernel"))) return rc;
   hipLaunchKernelGGL(k_gather_reduce, dim3(grid1(nslot * 3, 256)), dim3(256), 0, s, grid1(nslot * 3, 256), clc,

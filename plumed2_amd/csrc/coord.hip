@@ -517,7 +517,7 @@ static int run_pairs(p2a_coord* c, const double* box9, const double* pos_dev, do
       }
       A.wave_start = D.wave_start.p;
     }
-    launch_pairs(A, grids[d], s, value_only, c->tune.chunk, D.items.p, D.ents.p, GI.p.p, GJ.p.p, GI.bb.p, GJ.bb.p,
+    launch_pairs<true>(A, grids[d], s, value_only, c->tune.chunk, D.items.p, D.ents.p, GI.p.p, GJ.p.p, GI.bb.p, GJ.bb.p,
                  GI.abs_slot.p, GJ.abs_slot.p, D.fpart.p, c->partial.p + 8 * (size_t)off);
     off += grids[d];
   }

@@ -46,6 +46,7 @@
 #include <cstring>
 #include <string>
 
+#include "fp64_math.h"
 #include "p2a_internal.h"
 #include "switch_eval.h"
 
@@ -1344,12 +1345,73 @@ __device__ __forceinline__ int band_record(int staged, int ii, int kind) {
   return staged | (ii << 10) | (kind << 13);
 }
 
-// FP32 switch terms of one pair on its FP32 r^2
+// A switch other than fixedRational with its type known at compile time
+// (P2A_SW_*; kSwFastRational: RATIONAL of even exponents on r^2), FP64, for a
+// pair inside D_MAX.  Against switch_calc_sqr, whose type is a variable: one
+// reciprocal square root in place of a square root and a division, and no
+// code of the other types held in the kernel (together they took 560 spilled
+// registers in the pair kernel).
+constexpr int kSwFastRational = 100;
+template <int K>
+__device__ __forceinline__ double switch_known(const p2a_switch& sw, double d2, double& dfunc) {
+#pragma clang fp contract(off)
+  if constexpr (K == kSwFastRational) {
+    double f, df;
+    rational_core(sw, d2 * sw.invr0_2, sw.preSecDevF, sw.nnf, sw.mmf, sw.preDfuncF, sw.preRes, f, df);
+    df *= 2 * sw.invr0_2;
+    dfunc = df * sw.stretch;
+    return f * sw.stretch + sw.shift;
+  } else if constexpr (K == P2A_SW_FASTGAUSSIAN) {
+    // switch_calc_sqr at zero distance: 1, without stretch and shift
+    const double e = exp_core(-0.5 * d2);
+    dfunc = d2 > 0.0 ? -e * sw.stretch : 0.0;
+    return d2 > 0.0 ? e * sw.stretch + sw.shift : 1.0;
+  } else {
+    const double ir = rsqrt64(d2);
+    const double r = d2 > 0.0 ? d2 * ir : 0.0;
+    if constexpr (K == P2A_SW_Q) {
+      if (!(r > sw.d0)) {
+        dfunc = 0.0;
+        return sw.stretch + sw.shift;
+      }
+      const double e = exp(sw.beta * (r - sw.lambda * sw.ref));
+      const double s = 1.0 / (1.0 + e);
+      dfunc = -sw.beta / (e + 2.0 + 1.0 / e) * ir * sw.stretch;
+      return s * sw.stretch + sw.shift;
+    } else {
+      const double rdist = (r - sw.d0) * sw.invr0;
+      if (!(rdist > 0.0)) {
+        dfunc = 0.0;
+        return sw.stretch + sw.shift;
+      }
+      double f, df;
+      if constexpr (K == P2A_SW_EXP) {
+        f = exp_core(-rdist);
+        df = -f;
+      } else if constexpr (K == P2A_SW_GAUSSIAN) {
+        f = exp_core(-0.5 * rdist * rdist);
+        df = -rdist * f;
+      } else if constexpr (K == P2A_SW_RATIONAL) {
+        rational_core(sw, rdist, sw.preSecDev, sw.nn, sw.mm, sw.preDfunc, sw.preRes, f, df);
+      } else {
+        p2a_switch t = sw;
+        t.type = K;
+        base_function(t, rdist, f, df);
+      }
+      dfunc = df * sw.stretch * sw.invr0 * ir;
+      return f * sw.stretch + sw.shift;
+    }
+  }
+}
+
+// FP32 switch terms of one pair on its FP32 r^2.  GENERIC: P is the switch's
+// type for switch_known, 0 for any switch.
 template <int P, bool GENERIC>
 __device__ __forceinline__ void pair_switch(const PairArgs& A, float r2, float& sv, float& dfu) {
   if constexpr (GENERIC) {
     double dfd;
-    sv = (float)switch_calc_sqr(A.sw, (double)r2 * A.r2_real, dfd);
+    if constexpr (P == 0) sv = (float)switch_calc_sqr(A.sw, (double)r2 * A.r2_real, dfd);
+    else sv = (float)switch_known<P>(A.sw, (double)r2 * A.r2_real, dfd);
     dfu = (float)dfd;
   } else {
     sw_fixed<P>(A.invr0_2, r2, sv, dfu);
@@ -1395,9 +1457,8 @@ __device__ __forceinline__ void pair_term(const PairArgs& A, const P3& pj, const
   // a pair outside the cut gets sv = dfu = 0 from x = sw_far (fixed P) or by selection
   float sv, dfu;
   if constexpr (GENERIC) {
-    pair_switch<P, GENERIC>(A, r2, sv, dfu);
-    sv = cut ? sv : 0.f;
-    dfu = cut ? dfu : 0.f;
+    sv = dfu = 0.f;
+    if (cut) pair_switch<P, GENERIC>(A, r2, sv, dfu);
   } else {
     // positions are in units of R_0: x = r^2
     const float x = cut ? r2 : sw_far<P>();
@@ -2925,13 +2986,28 @@ inline void launch_rows(const PairArgs& A, bool weighted, int grid, hipStream_t 
     PairArgs G = A;
     pair_args_generic(G);
     const PairArgs& A = G;
-    P2A_RSW(1, true);
+    P2A_RSW(0, true);
   }
 #undef P2A_RSW
 #undef P2A_R
 }
 
-// launch of the pair kernel for a switch, group mode and tuning
+// the type a switch is compiled for in switch_known, 0 for none
+inline int switch_known_kind(const p2a_switch& sw) {
+  if (sw.type == P2A_SW_RATIONAL) return sw.fast ? kSwFastRational : P2A_SW_RATIONAL;
+  switch (sw.type) {
+    case P2A_SW_EXP: case P2A_SW_GAUSSIAN: case P2A_SW_FASTGAUSSIAN: case P2A_SW_SMAP: case P2A_SW_CUBIC:
+    case P2A_SW_TANH: case P2A_SW_COSINUS: case P2A_SW_Q: return sw.type;
+    default: return 0;
+  }
+}
+
+// launch of the pair kernel for a switch, group mode and tuning.  TWOG: the
+// caller has two groups (else only the kernels of one group are compiled).
+// The other switches have a kernel of their own for the default work items
+// with derivatives (20,000 atoms with EXP: pair pass 105 -> 62 us); value only and 32 entries
+// an item run the kernel that takes any switch.
+template <bool TWOG>
 inline void launch_pairs(const PairArgs& A, int grid, hipStream_t s, bool value_only, int chunk, const int4* items,
                          const Entry* ents, const float4* posI, const float4* posJ, const float4* bbI,
                          const float4* bbJ, const int* absI, const int* absJ, double* fpart, double* partial) {
@@ -2946,14 +3022,23 @@ inline void launch_pairs(const PairArgs& A, int grid, hipStream_t s, bool value_
   } while (0)
 #define P2A_KSW(P, GEN)                                     \
   do {                                                      \
-    if (A.twogroup) {                                       \
-      if (value_only) P2A_KCH(P, GEN, true, true);          \
-      else P2A_KCH(P, GEN, true, false);                    \
-    } else {                                                \
-      if (value_only) P2A_KCH(P, GEN, false, true);         \
-      else P2A_KCH(P, GEN, false, false);                   \
+    if constexpr (TWOG) {                                   \
+      if (A.twogroup) {                                     \
+        if (value_only) P2A_KCH(P, GEN, true, true);        \
+        else P2A_KCH(P, GEN, true, false);                  \
+        break;                                              \
+      }                                                     \
     }                                                       \
+    if (value_only) P2A_KCH(P, GEN, false, true);           \
+    else P2A_KCH(P, GEN, false, false);                     \
   } while (0)
+#define P2A_KKN(K)                                              \
+  case K:                                                       \
+    if constexpr (TWOG) {                                       \
+      if (A.twogroup) { P2A_K(K, true, true, false, 64); break; } \
+    }                                                           \
+    P2A_K(K, true, false, false, 64);                           \
+    break
   if (sw.type == P2A_SW_RATIONAL_FIXED) {
     switch (sw.nn / 2) {
       case 1: P2A_KSW(1, false); break;
@@ -2962,11 +3047,25 @@ inline void launch_pairs(const PairArgs& A, int grid, hipStream_t s, bool value_
       case 4: P2A_KSW(4, false); break;
       case 5: P2A_KSW(5, false); break;
       case 6: P2A_KSW(6, false); break;
-      default: P2A_KSW(1, true); break;
+      default: P2A_KSW(0, true); break;
     }
-  } else {
-    P2A_KSW(1, true);
+    return;
   }
+  const int kind = value_only || chunk != 64 ? 0 : switch_known_kind(sw);
+  switch (kind) {
+    P2A_KKN(kSwFastRational);
+    P2A_KKN(P2A_SW_RATIONAL);
+    P2A_KKN(P2A_SW_EXP);
+    P2A_KKN(P2A_SW_GAUSSIAN);
+    P2A_KKN(P2A_SW_FASTGAUSSIAN);
+    P2A_KKN(P2A_SW_SMAP);
+    P2A_KKN(P2A_SW_CUBIC);
+    P2A_KKN(P2A_SW_TANH);
+    P2A_KKN(P2A_SW_COSINUS);
+    P2A_KKN(P2A_SW_Q);
+    default: P2A_KSW(0, true); break;
+  }
+#undef P2A_KKN
 #undef P2A_KSW
 #undef P2A_KCH
 #undef P2A_K

@@ -30,6 +30,7 @@
 #include <string>
 #include <vector>
 
+#include "fp64_math.h"
 #include "p2a_internal.h"
 
 // The grid arithmetic follows the reference's FP64 operations one rounding at
@@ -212,36 +213,6 @@ __device__ __forceinline__ bool support_node(const GridArg& G, const unsigned* i
     node_ind[i] = (unsigned)i0;
   }
   return true;
-}
-
-// exp(x), |x| < 2^20, for the heights and the shapes: ln2 reduction and the
-// Taylor polynomial of degree 13 on |r| <= ln2/2 (truncation 4e-18) in pairs,
-// so that its depth is 5 multiply-adds instead of a dozen in a row; within
-// 1.5 ulp.  The chain of heights keeps the constants in registers (a 64-bit
-// literal costs two moves): ExpK, made opaque there.
-struct ExpK {
-  double log2e = 1.4426950408889634;
-  // ln2 in two parts, the first of 32 bits (its product with n is exact)
-  double hi = -0x1.62e42fee00000p-1, lo = -0x1.a39ef35793c76p-33;
-  double m[6] = {1.0 / 6, 1.0 / 120, 1.0 / 5040, 1.0 / 362880, 1.0 / 39916800, 1.0 / 6227020800.0};
-  double a[5] = {1.0 / 24, 1.0 / 720, 1.0 / 40320, 1.0 / 3628800, 1.0 / 479001600};
-};
-// exp(x) = 2^n p: p from x and n = rint(x log2e)
-__device__ __forceinline__ double exp_part(double x, double n, const ExpK& C) {
-  double r = fma(n, C.hi, x);
-  r = fma(n, C.lo, r);
-  const double r2 = r * r, r4 = r2 * r2, r8 = r4 * r4;
-  const double p01 = 1.0 + r, p23 = fma(r, C.m[0], 0.5);
-  const double p45 = fma(r, C.m[1], C.a[0]), p67 = fma(r, C.m[2], C.a[1]);
-  const double p89 = fma(r, C.m[3], C.a[2]), pab = fma(r, C.m[4], C.a[3]), pcd = fma(r, C.m[5], C.a[4]);
-  const double q0 = fma(r2, p23, p01), q1 = fma(r2, p67, p45), q2 = fma(r2, pab, p89);
-  const double lo = fma(r4, q1, q0), hi = fma(r4, pcd, q2);
-  return fma(r8, hi, lo);
-}
-__device__ __forceinline__ double exp_core(double x) {
-  const ExpK C;
-  const double n = rint(x * C.log2e);
-  return ldexp(exp_part(x, n, C), (int)n);
 }
 
 // One hill at a node, as every deposition in hill order forms it.  Per CV:
