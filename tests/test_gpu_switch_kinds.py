@@ -1,7 +1,7 @@
 """Every switch type through the cluster pair kernel compiled for it (one and
 two groups, derivatives), against the FP64 oracle, with D_0 > 0 (the flat part)
 among them, and two atoms at one place where the switch has a gradient there
-(TANH with D_0 = 0 has a kink at zero distance).  Tolerances of the cluster path: the pair
+(TANH and Q with D_0 = 0 have a kink at zero distance).  Tolerances of the cluster path: the pair
 terms are FP64 rounded to FP32 (2^-24 each, sums of at most ~500 a lane)."""
 import numpy as np
 import pytest
@@ -26,7 +26,7 @@ def test_switch_kind(sw, nb):
     n = 1500
     rng = np.random.default_rng(17)
     x = rng.uniform(0.0, 3.1, (n, 3))
-    if not sw.startswith("TANH"):
+    if not sw.startswith(("TANH", "Q ")):
         x[7] = x[1203]
     box = np.array([[3.1, 0.0, 0.0], [0.2, 3.0, 0.0], [-0.1, 0.25, 3.2]])
     groups = f"GROUPA=1-{n - nb}" + (f" GROUPB={n - nb + 1}-{n}" if nb else "")
