@@ -399,6 +399,17 @@ int p2a_cdist_calculate_device(p2a_cdist *ctx, void *stream, const double *box9,
  * force on this CV); forces_dev is the [natoms][3] array of all atoms. */
 int p2a_cdist_apply_force_device(p2a_cdist *ctx, void *stream, const double *f_dev, const double *deriv_dev,
                                  const double *virial_cv_dev, double *forces_dev, double *virial_dev);
+/* Forces of one METAD step on every atom and on the cell, written (not added)
+ * in one pass: forces[3N] = f[0] * deriv[3N] and virial[9] = f[0] *
+ * virial_cv[9] of the first CV, plus, with a cdist context (NULL: none), f[1]
+ * times the distance's derivatives and box derivative; the sums of
+ * p2a_apply_force_device and p2a_cdist_apply_force_device on cleared arrays.
+ * cv_force_dev: the METAD forces on the CVs.  Device arrays, asynchronous on
+ * `stream` (NULL: default stream). */
+int p2a_metad_forces_device(void *stream, int64_t natoms, const double *cv_force_dev, const double *deriv_dev,
+                            const double *virial_cv_dev, p2a_cdist *ctx, const double *dist_deriv_dev,
+                            const double *dist_virial_dev, double *forces_dev, double *virial_dev);
+
 
 /* COORDINATIONNUMBER on the cluster pair list of a COORDINATION context
  * (src/symfunc/CoordinationNumbers.cpp:326-372: CONTACT_MATRIX rows times

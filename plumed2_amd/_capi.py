@@ -92,6 +92,8 @@ _SIGS = {
     "p2a_cdist_destroy": ([C.c_void_p], C.c_int),
     "p2a_cdist_calculate_device": ([C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
                                     C.c_void_p], C.c_int),
+    "p2a_metad_forces_device": ([C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
+                                 C.c_void_p, C.c_void_p, C.c_void_p], C.c_int),
     "p2a_cdist_apply_force_device": ([C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
                                       C.c_void_p], C.c_int),
     "p2a_batch_create": ([C.POINTER(C.c_void_p), C.c_int, C.c_int, C.c_void_p, C.POINTER(p2a_switch), C.c_double],

@@ -141,15 +141,12 @@ class MetadStep:
         self.metad.step_device(step, cvp, self.bias.data_ptr(), self.cv_force.data_ptr(), self.height.data_ptr(),
                                stream=stream)
         # 2. forces on atoms and cell (this step's METAD forces only)
-        self.forces.zero_()
-        self.virial.zero_()
-        fp = self.cv_force.data_ptr()
-        A.check(A.lib().p2a_apply_force_device(C.c_void_p(stream), self.natoms, C.c_void_p(fp),
-                                               C.c_void_p(self.d_coord.data_ptr()),
-                                               C.c_void_p(self.w_coord.data_ptr()),
-                                               C.c_void_p(self.forces.data_ptr()), C.c_void_p(self.virial.data_ptr())))
-        if self.cdist is not None:
-            self.cdist.apply_force_device(stream, fp + 8, self.d_dist.data_ptr(), self.w_dist.data_ptr(),
-                                          self.forces.data_ptr(), self.virial.data_ptr())
+        cd = self.cdist
+        A.check(A.lib().p2a_metad_forces_device(
+            C.c_void_p(stream), self.natoms, C.c_void_p(self.cv_force.data_ptr()), C.c_void_p(self.d_coord.data_ptr()),
+            C.c_void_p(self.w_coord.data_ptr()), cd._ctx if cd is not None else None,
+            C.c_void_p(self.d_dist.data_ptr()) if cd is not None else None,
+            C.c_void_p(self.w_dist.data_ptr()) if cd is not None else None,
+            C.c_void_p(self.forces.data_ptr()), C.c_void_p(self.virial.data_ptr())))
         return {"cv": self.cv, "bias": self.bias, "cv_force": self.cv_force, "forces": self.forces,
                 "virial": self.virial, "height": self.height}
