@@ -54,7 +54,7 @@ struct p2a_batch {
   p2a::DBuf<double4> origin;
   p2a::DBuf<float4> bb0, bb, p;
   p2a::DBuf<float2> kr;
-  p2a::DBuf<int> ecount, estart, istart, totals, scan_bsum, bflag, wave_start;
+  p2a::DBuf<int> ecount, estart, istart, totals, scan_bsum, wave_start;
   p2a::DBuf<unsigned> ell;  // candidates the list count pass keeps for the fill pass
   p2a::DBuf<p2a::Entry> ents;
   p2a::DBuf<int4> items;
@@ -79,7 +79,6 @@ static int batch_reserve_lists(p2a_batch* b, int ent_cap, int items_cap) {
   if ((rc = b->ents.reserve(std::max(ent_cap, 1))) || (rc = b->items.reserve(std::max(items_cap, 1))) ||
       (rc = b->fpart.reserve((size_t)CL * 3 * std::max(items_cap, 1))) ||
       (rc = b->partial.reserve(8 * (size_t)std::max(items_cap, 1))) ||
-      (rc = b->bflag.reserve(std::max(items_cap, 1))) ||
       // the pair kernel's schedule: at most one wave per item (grid1(items_cap, 4) workgroups)
       (rc = b->wave_start.reserve((size_t)grid1(std::max(items_cap, 1), PAIR_BLOCK / WAVE) * (PAIR_BLOCK / WAVE) + 1)))
     return rc;
@@ -141,13 +140,11 @@ static int batch_step(p2a_batch* b, const double* pos, double* values, double* d
   A.nitems_dev = b->totals.p + 3;
   A.items_cap = b->items_cap;
   A.ent_cap = b->ent_cap;
-  A.twogroup = 0;
   A.pbc = b->pbc.p;
   A.cl_sys = b->cl_sys.p;
   A.pos64 = pos;
   A.item_partials = 1;  // per-system sums need the items' own partials
   A.ipart = b->partial.p;
-  A.bflag = b->bflag.p;
   int grid = grid1(std::max(b->items_cap, 1), PAIR_BLOCK / WAVE);
   A.wave_start = nullptr;
   if (b->tune.blocks_per_cu > 0) grid = std::min(grid, b->tune.blocks_per_cu * b->cu_count);
@@ -159,8 +156,8 @@ static int batch_step(p2a_batch* b, const double* pos, double* values, double* d
                        (const int*)A.nitems_dev, b->items_cap, (const int4*)b->items.p, nw, b->wave_start.p);
     A.wave_start = b->wave_start.p;
   }
-  launch_pairs<false>(A, grid, s, false, chunk, b->items.p, b->ents.p, b->p.p, b->p.p, b->bb.p, b->bb.p, (const int*)nullptr,
-               (const int*)nullptr, b->fpart.p, b->partial.p);
+  launch_pairs<false>(A, grid, s, false, chunk, b->items.p, b->ents.p, b->p.p, b->p.p, b->bb.p, b->bb.p,
+                      (const int*)nullptr, b->fpart.p, b->partial.p);
   if ((rc = launch_check("batch: pair kernel"))) return rc;
   hipLaunchKernelGGL(k_gather_reduce, dim3(grid1(nslot * 3, 256)), dim3(256), 0, s, grid1(nslot * 3, 256), clc,
                      ncl_dev, b->p.p, b->istart.p, b->items_cap, b->fpart.p, deriv, 0, RedArgs{});

@@ -25,7 +25,6 @@ struct Dir {  // one cluster-pair list: i clusters of group I against group J
   DBuf<int4> items;
   DBuf<double> fpart;  // per item: derivative partials of the 8 i atoms
   DBuf<double> rpart;  // per item: per-atom coordination-number rows of the 8 i atoms
-  DBuf<int> bflag;     // per item: band pairs found by the pair kernel
   DBuf<int> wave_start;  // the pair kernel's balanced schedule (k_wave_sched)
   int sched_waves = -1;  // the grid it was made for
   int64_t sched_gen = -1;  // and the list build
@@ -49,9 +48,10 @@ struct Group {
   DBuf<SysArg> sys;
   DBuf<int4> info;
   DBuf<double> key;
-  DBuf<int> col_count, col_start, col_cl, fill, tmp, slot_loc, cl_col, abs_slot;
+  DBuf<int> col_count, col_start, col_cl, fill, tmp, slot_loc, cl_col, twin_slot;
   DBuf<double4> origin;
   DBuf<float4> bb0, bb, p;
+  DBuf<float4> pw;  // p with the row weights (k_row_weights)
   DBuf<float2> kr;
 };
 
@@ -83,6 +83,7 @@ struct p2a_coord {
   p2a::DBuf<double> partial, red, stats, pos_buf, deriv_buf, out_buf;
   p2a::DBuf<int> scan_bsum;   // block sums of the list scans
   p2a::DBuf<long long> abs_dev;
+  p2a::DBuf<int> twin_dev;  // groups that share atoms: requested index of the atom in the other group, or -2
   int64_t rebuilds = 0;
   bool profiling = false;
   int prof_every = 1;       // events around every prof_every-th pair pass
@@ -117,9 +118,7 @@ struct p2a_coord {
   p2a::DBuf<long long> nl_total;
   bool nl_valid = false;
   int64_t nl_entries = 0;  // partners listed in nl_nbr
-  // per-atom coordination numbers: weights per requested atom; row and
-  // environment indices for the FP64 path
-  p2a::DBuf<float> wreq;
+  // per-atom coordination numbers: row and environment indices for the FP64 path
   p2a::DBuf<int> cn_rows, cn_env;
 };
 
@@ -161,6 +160,7 @@ static int rebuild(p2a_coord* c, const double* box9, const double* pos_dev) {
   // D_MAX + skin otherwise (skin 0: the list is rebuilt every step)
   c->rlist = (c->spec.nl_mode != P2A_NL_NONE ? std::max(c->spec.nl_cutoff, sw.dmax) : sw.dmax + c->skin_active) + 1e-4;
   const int ngroups = c->spec.nb > 0 ? 2 : 1;
+  const bool share = ngroups == 2 && !c->distinct;
   hipStream_t s = c->stream;
   int rc;
   for (int gi = 0; gi < ngroups; gi++) {
@@ -181,7 +181,7 @@ static int rebuild(p2a_coord* c, const double* box9, const double* pos_dev) {
         (rc = G.slot_loc.reserve((size_t)maxcl * CL)) || (rc = G.cl_col.reserve(maxcl)) ||
         (rc = G.origin.reserve(maxcl)) || (rc = G.bb0.reserve(2 * (size_t)maxcl)) ||
         (rc = G.bb.reserve(2 * (size_t)maxcl)) || (rc = G.p.reserve((size_t)maxcl * CL)) ||
-        (rc = G.kr.reserve(maxcl)) || (rc = G.abs_slot.reserve((size_t)maxcl * CL)))
+        (rc = G.kr.reserve(maxcl)) || (share && (rc = G.twin_slot.reserve((size_t)maxcl * CL))))
       return rc;
     // the descriptor goes to the device in stream order when it changed
     if (!G.S_valid || std::memcmp(&G.S, &G.S_dev, sizeof(SysArg)) != 0) {
@@ -284,8 +284,7 @@ static int rebuild(p2a_coord* c, const double* box9, const double* pos_dev) {
     c->nitems += D.nitems;
     tot_entries += D.nentries;
     if ((rc = D.ents.reserve(std::max<int64_t>(D.nentries, 1))) || (rc = D.items.reserve(std::max(D.nitems, 1))) ||
-        (rc = D.fpart.reserve((size_t)CL * 3 * std::max(D.nitems, 1))) ||
-        (rc = D.bflag.reserve(std::max(D.nitems, 1))))
+        (rc = D.fpart.reserve((size_t)CL * 3 * std::max(D.nitems, 1))))
       return rc;
     Ls[d].ent_cap = (int)D.ents.n;
     if (GI.ncl > 0) {
@@ -298,13 +297,12 @@ static int rebuild(p2a_coord* c, const double* box9, const double* pos_dev) {
     }
   }
   c->nentries = tot_entries;
-  // absolute index per slot (two groups: pairs of one atom with itself are skipped)
-  if (ngroups == 2) {
+  if (share) {
     for (int gi = 0; gi < 2; gi++) {
       Group& G = c->g[gi];
       if (G.ncl > 0)
-        hipLaunchKernelGGL(k_abs_slot, dim3(grid1((size_t)G.ncl * CL, 256)), dim3(256), 0, s, G.ncl * CL,
-                           (const int*)nullptr, G.slot_loc.p, G.off, (const long long*)c->abs_dev.p, G.abs_slot.p);
+        hipLaunchKernelGGL(k_twin_slot, dim3(grid1((size_t)G.ncl * CL, 256)), dim3(256), 0, s, G.ncl * CL,
+                           (const int*)G.slot_loc.p, G.off, (const int*)c->twin_dev.p, G.twin_slot.p);
     }
   }
   if ((rc = launch_check("rebuild: list fill"))) return rc;
@@ -457,7 +455,7 @@ static int run_pairs(p2a_coord* c, const double* box9, const double* pos_dev, do
   pack_positions(c, pos_dev);
   PairArgs A;
   std::memset(&A, 0, sizeof(A));
-  A.twogroup = ngroups == 2;
+  A.share = ngroups == 2 && !c->distinct;
   pair_args_switch(c->spec.sw, A);
   if ((rc = upload_pbc(c, box9))) return rc;
   A.pbc = c->pbc_dev.p;
@@ -503,7 +501,6 @@ static int run_pairs(p2a_coord* c, const double* box9, const double* pos_dev, do
     A.nitems = D.nitems;
     A.items_cap = (int)D.items.n;
     A.ent_cap = (int)D.ents.n;
-    A.bflag = D.bflag.p;
     A.wave_start = nullptr;
     if (c->tune.blocks_per_cu > 0) {
       // a persistent grid takes contiguous item ranges of balanced cost
@@ -518,7 +515,7 @@ static int run_pairs(p2a_coord* c, const double* box9, const double* pos_dev, do
       A.wave_start = D.wave_start.p;
     }
     launch_pairs<true>(A, grids[d], s, value_only, c->tune.chunk, D.items.p, D.ents.p, GI.p.p, GJ.p.p, GI.bb.p, GJ.bb.p,
-                 GI.abs_slot.p, GJ.abs_slot.p, D.fpart.p, c->partial.p + 8 * (size_t)off);
+                 GI.twin_slot.p, D.fpart.p, c->partial.p + 8 * (size_t)off);
     off += grids[d];
   }
   if (rec) {
@@ -692,16 +689,20 @@ static int run_rows(p2a_coord* c, const double* box9, const double* pos_dev, dou
   pack_positions(c, pos_dev);
   PairArgs A;
   std::memset(&A, 0, sizeof(A));
-  A.twogroup = ngroups == 2;
+  A.share = ngroups == 2 && !c->distinct;
   pair_args_switch(c->spec.sw, A);
   if ((rc = upload_pbc(c, box9))) return rc;
   A.pbc = c->pbc_dev.p;
   A.pos64 = pos_dev;
   const bool weighted = weights_dev != nullptr;
   if (weighted) {
-    if ((rc = c->wreq.reserve(std::max(c->natoms, 1)))) return rc;
-    hipLaunchKernelGGL(k_row_weights, dim3(grid1(c->natoms, 256)), dim3(256), 0, s, (int)c->spec.na, c->natoms,
-                       weights_dev, c->wreq.p);
+    for (int gi = 0; gi < ngroups; gi++) {
+      Group& G = c->g[gi];
+      if (G.ncl == 0) continue;
+      if ((rc = G.pw.reserve((size_t)G.maxcl * CL))) return rc;
+      hipLaunchKernelGGL(k_row_weights, dim3(grid1((size_t)G.ncl * CL, 256)), dim3(256), 0, s, G.ncl * CL,
+                         (int)c->spec.na, (const float4*)G.p.p, weights_dev, G.pw.p);
+    }
   }
   // the rows come from the first direction (i = GROUPA); the weighted
   // product needs every direction for the derivatives of all atoms
@@ -726,8 +727,8 @@ static int run_rows(p2a_coord* c, const double* box9, const double* pos_dev, dou
     A.nitems = D.nitems;
     A.items_cap = (int)D.items.n;
     A.ent_cap = (int)D.ents.n;
-    launch_rows(A, weighted, grids[d], s, c->wreq.p, D.items.p, D.ents.p, GI.p.p, GJ.p.p, GI.bb.p, GJ.bb.p,
-                GI.abs_slot.p, GJ.abs_slot.p, D.rpart.p, D.fpart.p, c->partial.p + 8 * (size_t)off);
+    launch_rows(A, weighted, grids[d], s, D.items.p, D.ents.p, GI.p.p, GJ.p.p, GI.pw.p, GJ.pw.p, GI.bb.p, GJ.bb.p,
+                GI.twin_slot.p, D.rpart.p, D.fpart.p, c->partial.p + 8 * (size_t)off);
     off += grids[d];
   }
   if ((rc = launch_check("row kernel"))) return rc;
@@ -1027,6 +1028,36 @@ int p2a_coord_create(p2a_coord** out, int device, const p2a_coord_spec* spec) {
   if ((rc = c->abs_dev.reserve(c->natoms))) {
     p2a_coord_destroy(c);
     return rc;
+  }
+  if (!c->distinct && !c->has_duplicates && c->spec.nb > 0) {
+    // (duplicates within a group take the FP64 path)
+    std::vector<std::pair<int64_t, int>> by[2];
+    std::vector<int> twin(c->natoms, -2);
+    for (int gi = 0; gi < 2; gi++) {
+      const int off = gi == 0 ? 0 : (int)spec->na, n = (int)(gi == 0 ? spec->na : spec->nb);
+      for (int k = 0; k < n; k++) by[gi].push_back({c->abs[off + k], off + k});
+      std::sort(by[gi].begin(), by[gi].end());
+    }
+    for (size_t a = 0, b = 0; a < by[0].size() && b < by[1].size();) {
+      if (by[0][a].first == by[1][b].first) {
+        twin[by[0][a].second] = by[1][b].second;
+        twin[by[1][b].second] = by[0][a].second;
+        a++;
+        b++;
+      } else if (by[0][a].first < by[1][b].first) {
+        a++;
+      } else {
+        b++;
+      }
+    }
+    if ((rc = c->twin_dev.reserve(c->natoms))) {
+      p2a_coord_destroy(c);
+      return rc;
+    }
+    if (hipMemcpy(c->twin_dev.p, twin.data(), twin.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess) {
+      p2a_coord_destroy(c);
+      return fail(P2A_ERR_HIP, "hipMemcpy of the shared atoms failed");
+    }
   }
   std::vector<long long> ab(c->abs.begin(), c->abs.end());
   if (hipMemcpy(c->abs_dev.p, ab.data(), ab.size() * sizeof(long long), hipMemcpyHostToDevice) != hipSuccess) {

@@ -679,15 +679,15 @@ __global__ __launch_bounds__(256) void k_rank(int ncol, const double* __restrict
   }
 }
 
-// absolute atom index of every slot of a group (two groups: an atom listed in
-// both is not paired with itself); padding slots get distinct negative tags
-__global__ void k_abs_slot(int nslot, const int* __restrict__ ncl_dev, const int* __restrict__ slot_loc, int off,
-                           const long long* __restrict__ absidx, int* __restrict__ abs_slot) {
+// Two groups that share atoms: for every slot, the requested index of the same
+// atom in the other group (twin, by requested index; negative: not in it), so
+// that the pair kernels leave out an atom's pair with itself
+__global__ void k_twin_slot(int nslot, const int* __restrict__ slot_loc, int off, const int* __restrict__ twin,
+                            int* __restrict__ twin_slot) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (ncl_dev) nslot = *ncl_dev * CL;
   if (s >= nslot) return;
   const int a = slot_loc[s];
-  abs_slot[s] = (a >= 0) ? (int)absidx[off + a] : -1 - s;
+  twin_slot[s] = (a >= 0) ? twin[off + a] : -2;
 }
 
 // candidates kept per i cluster between the count and fill passes of the
@@ -1279,7 +1279,7 @@ struct PairArgs {
   int nitems;
   const int* nitems_dev;  // device item count (null: nitems)
   int items_cap, ent_cap; // capacities of the item and entry arrays
-  int twogroup;
+  int share;              // the two groups have atoms in common (twinI tells them)
   float dmax2, prune2, band;
   float cut_lo, cut_hi;   // FP32 r^2 at or below cut_lo: inside; in (cut_lo, cut_hi): the band
   float contact2;         // FP32 r^2 of DBL_EPSILON (the contact-matrix rule)
@@ -1295,7 +1295,6 @@ struct PairArgs {
   // `partial` over all of its items.
   int item_partials;
   double* ipart;
-  int* bflag;             // band pairs of each item from a wave's 65th item on
   // Items of each wave of the grid: [wave_start[g], wave_start[g + 1]) for
   // wave g = xcd_block() * 4 + wave (k_wave_sched); null: items g, g + waves, ...
   const int* wave_start;
@@ -1319,25 +1318,28 @@ __device__ double exact_r2(const PbcArg* __restrict__ P, const double* __restric
   return d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
 }
 
-// a staged j atom in LDS: position in the i cluster's frame (12 B); its
-// origin (entry << 3 | slot, -1 for padding) is kept in a separate short
-struct P3 {
-  float x, y, z;
-};
-
 // per-lane FP32 sums of one work item: sv (counted pairs), dfu * d (i
 // derivative), dfu * d (x) d (virial, counted pairs)
 struct PairAcc {
   float sv, fx, fy, fz, vxx, vxy, vxz, vyy, vyz, vzz;
 };
 
-// the wave's LDS areas for one work item
+// entries a wave holds in LDS: those of an item, each kind from a multiple of
+// 8 and rounds by two, and two rounds of reading ahead
+template <int CH>
+constexpr int sent_cap() {
+  return (CH / CL + 2 + 2) * CL;
+}
+
+// The wave's LDS areas for one work item.  A staged j atom is 16 B: its
+// position in the i cluster's frame and, in w, its requested index (-1 for
+// padding), so that one read serves the pair, the test for an atom's pair with
+// itself (TWO) and the band decisions.
 struct WaveLds {
-  P3* sj;       // staged j atoms
-  short* sm;    // their origin: entry << 3 | slot, -1 for padding
-  int* sc;      // entry codes of the item
-  int* sa;      // absolute index of each staged atom (two groups)
-  int* sr;      // band records of the current round (kBandSlots)
+  float4* sj;
+  Entry* se;    // the item's entries within D_MAX, counting ones first
+  // band records of the current round (kBandSlots), once the item is staged
+  __device__ __forceinline__ int* sr() const { return (int*)se; }
 };
 
 // a band record: staged index (bits 0-9), i slot (10-12), kind (13-14)
@@ -1420,19 +1422,20 @@ __device__ __forceinline__ void pair_switch(const PairArgs& A, float r2, float& 
 
 // FP32 separation and r^2 of staged atom pj from i atom pi (the one sequence
 // of operations for a pair in the FP32 pass and in its band decisions)
-__device__ __forceinline__ float pair_d(const P3& pj, const float4& pi, float& dx, float& dy, float& dz) {
+__device__ __forceinline__ float pair_d(const float4& pj, const float4& pi, float& dx, float& dy, float& dz) {
   dx = pj.x - pi.x;
   dy = pj.y - pi.y;
   dz = pj.z - pi.z;
   return fmaf(dx, dx, fmaf(dy, dy, dz * dz));
 }
 
-// whether lane (ii, jj) evaluates its pair in a group of kind KIND
+// whether lane (ii, jj) evaluates its pair in a group of kind KIND; TWO: ai is
+// the requested index of atom i in the other group
 template <bool TWO, bool VO, int KIND>
-__device__ __forceinline__ bool pair_keep(const WaveLds& L, int g, int ii, int jj, int ai) {
+__device__ __forceinline__ bool pair_keep(const float4& pj, int ii, int jj, int ai) {
   bool keep = true;
   if constexpr (KIND == 0) keep = jj != ii;  // an atom is not paired with itself
-  if constexpr (TWO) keep = keep && (L.sa[g + jj] != ai);
+  if constexpr (TWO) keep = keep && (__float_as_int(pj.w) != ai);
   if constexpr (VO && KIND == 0) keep = keep && jj > ii;  // value only: each pair once
   return keep;
 }
@@ -1445,11 +1448,11 @@ __device__ __forceinline__ bool pair_keep(const WaveLds& L, int g, int ii, int j
 // cut_hi) is left out here and counted in nrec (uniform); band_terms
 // decides the item's band pairs on FP64 distances after the pass.
 template <int P, bool GENERIC, bool TWO, bool VO, int KIND>
-__device__ __forceinline__ void pair_term(const PairArgs& A, const P3& pj, const float4& pi, int ii, int jj, int g,
-                                          int ai, const WaveLds& L, int& nrec, int& npair, PairAcc& acc) {
+__device__ __forceinline__ void pair_term(const PairArgs& A, const float4& pj, const float4& pi, int ii, int jj,
+                                          int ai, int& nrec, int& npair, PairAcc& acc) {
   float dx, dy, dz;
   const float r2 = pair_d(pj, pi, dx, dy, dz);
-  const bool keep = pair_keep<TWO, VO, KIND>(L, g, ii, jj, ai);
+  const bool keep = pair_keep<TWO, VO, KIND>(pj, ii, jj, ai);
   // inside D_MAX and outside the band: r2 <= cut_lo; in the band: cut_lo < r2 < cut_hi
   const bool cut = keep && r2 <= A.cut_lo;
   const unsigned long long bcut = __ballot(cut);
@@ -1512,31 +1515,31 @@ template <int P, bool GENERIC, bool TWO, bool VO, int KIND>
 __device__ __forceinline__ void pair_groups(const PairArgs& A, int gb, int ge, const float4& pi, int ii, int jj,
                                             int ai, const WaveLds& L, int& nrec, int& npair, PairAcc& acc) {
   int g = gb;
-  P3 pa = L.sj[g + jj];
+  float4 pa = L.sj[g + jj];
   for (; g + CL < ge; g += 2 * CL) {
-    const P3 pb = L.sj[g + CL + jj];
-    pair_term<P, GENERIC, TWO, VO, KIND>(A, pa, pi, ii, jj, g, ai, L, nrec, npair, acc);
+    const float4 pb = L.sj[g + CL + jj];
+    pair_term<P, GENERIC, TWO, VO, KIND>(A, pa, pi, ii, jj, ai, nrec, npair, acc);
     pa = L.sj[g + 2 * CL + jj];
-    pair_term<P, GENERIC, TWO, VO, KIND>(A, pb, pi, ii, jj, g + CL, ai, L, nrec, npair, acc);
+    pair_term<P, GENERIC, TWO, VO, KIND>(A, pb, pi, ii, jj, ai, nrec, npair, acc);
   }
-  if (g < ge) pair_term<P, GENERIC, TWO, VO, KIND>(A, pa, pi, ii, jj, g, ai, L, nrec, npair, acc);
+  if (g < ge) pair_term<P, GENERIC, TWO, VO, KIND>(A, pa, pi, ii, jj, ai, nrec, npair, acc);
 }
 
 // The band test of pair_term again for one group, numbering the band pairs in
 // program order: those numbered [r0, r0 + kBandSlots) become the wave's band
 // records (one round of band_terms).
 template <bool TWO, bool VO, int KIND>
-__device__ __forceinline__ void band_collect(const PairArgs& A, const P3& pj, const float4& pi, int ii, int jj, int g,
+__device__ __forceinline__ void band_collect(const PairArgs& A, const float4& pj, const float4& pi, int ii, int jj, int g,
                                              int ai, const WaveLds& L, int r0, int& cnt) {
   float dx, dy, dz;
   const float r2 = pair_d(pj, pi, dx, dy, dz);
-  const bool keep = pair_keep<TWO, VO, KIND>(L, g, ii, jj, ai);
+  const bool keep = pair_keep<TWO, VO, KIND>(pj, ii, jj, ai);
   const bool cut = keep && r2 <= A.cut_lo;
   const unsigned long long bm = __ballot(keep && r2 < A.cut_hi) & ~__ballot(cut);
   if (bm != 0ull) {
     if ((bm >> (ii + CL * jj)) & 1ull) {
       const int k = cnt + bits_below(bm) - r0;
-      if (k >= 0 && k < kBandSlots) L.sr[k] = band_record(g + jj, ii, KIND);
+      if (k >= 0 && k < kBandSlots) L.sr()[k] = band_record(g + jj, ii, KIND);
     }
     cnt += __popcll(bm);
   }
@@ -1573,14 +1576,13 @@ __device__ __forceinline__ void band_terms(const PairArgs& A, const WaveLds& L, 
     int rii = 0, cnt = 0;
     float sv = 0.f, g[3] = {0.f, 0.f, 0.f}, d[3] = {0.f, 0.f, 0.f};
     if (lane < nr) {
-      const int rec = L.sr[lane];
+      const int rec = L.sr()[lane];
       const int st = rec & 1023, kind = (rec >> 13) & 3;
       rii = (rec >> 10) & 7;
       const float4 pi = posI[ci * CL + rii];
       const float r2 = pair_d(L.sj[st], pi, d[0], d[1], d[2]);
-      const int meta = L.sm[st];  // (entry << 3 | slot), -1 for padding
       const int reqi = __float_as_int(pi.w);
-      const int reqj = meta >= 0 ? __float_as_int(posJ[(L.sc[meta >> 3] & kCjMask) * CL + (meta & 7)].w) : -1;
+      const int reqj = __float_as_int(L.sj[st].w);
       if (reqi >= 0 && reqj >= 0 && switch_inside(A.sw, exact_r2(pbc, A.pos64, reqi, reqj))) {
         float dfu;
         pair_switch<P, GENERIC>(A, r2, sv, dfu);
@@ -1648,144 +1650,152 @@ __device__ __forceinline__ double item_row(const PairArgs& A, const PairAcc& acc
 
 // Staging of one work item by one wave (i cluster ci, entries [e0, e1)):
 //  1. lane-parallel pruning of the chunk's entries against the current
-//     bounding boxes (D_MAX);
-//  2. each passing lane loads the 8 atoms of its j cluster, adds the image
-//     offset and keeps the atoms within D_MAX of the i cluster's box; the
-//     kept atoms are staged in LDS, compacted and grouped by entry kind
-//     (self / counting / derivative-only), each kind padded to a multiple
-//     of 8 with far-away atoms, so that every group of 8 has one kind.
+//     bounding boxes (D_MAX); the entries left go to LDS, compacted, counting
+//     ones first, each kind from a multiple of 8;
+//  2. in rounds of 8 entries, lane (entry, atom) loads one atom of its entry's
+//     j cluster (128 B in a row per cluster), adds the image offset and keeps
+//     it if it lies within D_MAX of the i cluster's box; the kept atoms are
+//     staged in LDS, compacted in (entry, atom) order and grouped by kind
+//     (self / counting / derivative-only), each kind padded to a multiple of 8
+//     with far-away atoms, so that every group of 8 has one kind.
+// A list radius above D_MAX leaves about half of the entries: 5-6 rounds,
+// where one lane per listed entry took 8 loads and tests an item, each load 64
+// lines.  The slots of se without an entry hold one that lies far away (atoms of
+// cluster 0, no lane is switched off); rounds go by two, the next two's loads
+// in flight.
+// DENSE: an item of which kDenseEntries entries or more are left (a list without
+// a margin over D_MAX) takes one lane per entry, eight loads in flight at once:
+// the same order; 48 systems, list radius 1.2 = D_MAX: 759 us, in rounds 803.
+constexpr int kDenseEntries = 40;
 // Returns the group bounds (uniform): n0 (0 or 8), [b1, b1+n1), [b2, b2+n2).
-constexpr int kFewEntries = 16;
-template <bool TWO, bool VO, int CH>
-__device__ __forceinline__ void stage_item(const PairArgs& A, const Entry& my_e, int lane, int e0, int e1,
+template <bool VO, bool DENSE, int CH>
+__device__ __forceinline__ void stage_item(const PairArgs& A, const Entry& my, int lane, int e0, int e1, int ci,
                                            const float4& ic, const float4& ih, const float4* __restrict__ posJ,
-                                           const float4* __restrict__ bbJ, const int* __restrict__ absJ,
-                                           const WaveLds& L, int& n0, int& b1, int& n1, int& b2, int& n2) {
-  // Two groups: an item of at most kFewEntries entries (the dense group's
-  // side of a sparse group) stages each entry with four lanes of two atoms
-  // each instead of one lane of eight; lanes are ordered by (entry, atom)
-  // either way, so the staged order is the same.  Single groups keep the
-  // one-lane form (their items are mostly full, and the branch costs them).
-  const bool few = TWO && e1 - e0 <= kFewEntries;  // uniform over the wave
-  const int ent = few ? (lane >> 2) : lane;  // this lane's entry of the item
-  const int sub2 = few ? 2 * (lane & 3) : 0;  // its first atom (few)
-  Entry my = {0, 0.f, 0.f, 0.f};
+                                           const float4* __restrict__ bbJ, const WaveLds& L, int& n0, int& b1,
+                                           int& n1, int& b2, int& n2) {
   bool pass = false;
-  {
-    Entry src = my_e;
-    if (few) {
-      src.code = __shfl(my_e.code, ent);
-      src.dx = __shfl(my_e.dx, ent);
-      src.dy = __shfl(my_e.dy, ent);
-      src.dz = __shfl(my_e.dz, ent);
-    }
-    const int e = e0 + ent;
-    if (ent < CH && e < e1) {
-      my = src;
-      if (!VO || (my.code & kCountBit) || my.code < 0) {
-        const int cj = my.code & kCjMask;
-        const float4 jc = bbJ[2 * cj], jh = bbJ[2 * cj + 1];
-        const float gx = fmaxf(fabsf(jc.x + my.dx - ic.x) - ih.x - jh.x, 0.f);
-        const float gy = fmaxf(fabsf(jc.y + my.dy - ic.y) - ih.y - jh.y, 0.f);
-        const float gz = fmaxf(fabsf(jc.z + my.dz - ic.z) - ih.z - jh.z, 0.f);
-        pass = gx * gx + gy * gy + gz * gz <= A.prune2;
-      }
-    }
+  const Entry none = {0, 1.0e5f, 1.0e5f, 1.0e5f};
+  L.se[lane] = none;
+  if (lane < sent_cap<CH>() - WAVE) L.se[WAVE + lane] = none;
+  if (lane < CH && e0 + lane < e1 && (!VO || (my.code & kCountBit) || my.code < 0)) {
+    const int cj = my.code & kCjMask;
+    const float4 jc = bbJ[2 * cj], jh = bbJ[2 * cj + 1];
+    const float gx = fmaxf(fabsf(jc.x + my.dx - ic.x) - ih.x - jh.x, 0.f);
+    const float gy = fmaxf(fabsf(jc.y + my.dy - ic.y) - ih.y - jh.y, 0.f);
+    const float gz = fmaxf(fabsf(jc.z + my.dz - ic.z) - ih.z - jh.z, 0.f);
+    pass = fmaf(gz, gz, fmaf(gx, gx, gy * gy)) <= A.prune2;
   }
-  float4 q[CL];
-  int m8 = 0, kind = 3;
-  if (pass && few) {
-    const int cj = my.code & kCjMask;
+  const unsigned long long mp = __ballot(pass), md = __ballot(my.code < 0), mc = __ballot((my.code & kCountBit) != 0);
+  const unsigned long long m1 = mp & mc & ~md, m2 = VO ? 0ull : mp & ~mc & ~md;
+  const int p1 = __popcll(m1), p2 = __popcll(m2);
+  if (DENSE && p1 + p2 >= kDenseEntries) {  // uniform over the wave
+    float4 q[CL];
+    int m8 = 0;
+    if (pass) {
+      const float4* pj = posJ + (size_t)(my.code & kCjMask) * CL;
 #pragma unroll
-    for (int u = 0; u < 2; u++) {
-      const float4 v = posJ[cj * CL + sub2 + u];
-      q[u] = make_float4(v.x + my.dx, v.y + my.dy, v.z + my.dz, 0.f);
-    }
-    if (my.code < 0) {
-      kind = 0;
-      m8 = 3 << sub2;
-    } else {
-      kind = (my.code & kCountBit) ? 1 : 2;
-#pragma unroll
-      for (int u = 0; u < 2; u++) {
-        const float gx = fmaxf(fabsf(q[u].x - ic.x) - ih.x, 0.f);
-        const float gy = fmaxf(fabsf(q[u].y - ic.y) - ih.y, 0.f);
-        const float gz = fmaxf(fabsf(q[u].z - ic.z) - ih.z, 0.f);
-        if (gx * gx + gy * gy + gz * gz <= A.prune2) m8 |= 1 << (sub2 + u);
-      }
-    }
-  } else if (pass) {
-    const int cj = my.code & kCjMask;
-#pragma unroll
-    for (int t = 0; t < CL; t++) {
-      const float4 v = posJ[cj * CL + t];
-      q[t] = make_float4(v.x + my.dx, v.y + my.dy, v.z + my.dz, 0.f);
-    }
-    if (my.code < 0) {
-      kind = 0;
-      m8 = 0xFF;  // the i cluster with itself keeps slot order
-    } else {
-      kind = (my.code & kCountBit) ? 1 : 2;
+      for (int t = 0; t < CL; t++) q[t] = pj[t];
 #pragma unroll
       for (int t = 0; t < CL; t++) {
+        q[t].x += my.dx;
+        q[t].y += my.dy;
+        q[t].z += my.dz;
         const float gx = fmaxf(fabsf(q[t].x - ic.x) - ih.x, 0.f);
         const float gy = fmaxf(fabsf(q[t].y - ic.y) - ih.y, 0.f);
         const float gz = fmaxf(fabsf(q[t].z - ic.z) - ih.z, 0.f);
-        if (gx * gx + gy * gy + gz * gz <= A.prune2) m8 |= 1 << t;
+        if (fmaf(gz, gz, fmaf(gx, gx, gy * gy)) <= A.prune2) m8 |= 1 << t;
       }
     }
+    const bool self = pass && my.code < 0, count = (my.code & kCountBit) != 0;
+    if (self) m8 = 0xFF;  // keeps slot order
+    n0 = (mp & md) ? CL : 0;
+    const int cnt = __popc(m8);
+    int tot1, tot2 = 0;
+    const int o1 = wave_excl_scan_dpp(count && !self ? cnt : 0, tot1);
+    int o2 = 0;
+    if constexpr (!VO) o2 = wave_excl_scan_dpp(count || self ? 0 : cnt, tot2);
+    n1 = (tot1 + CL - 1) & ~(CL - 1);
+    n2 = (tot2 + CL - 1) & ~(CL - 1);
+    b1 = n0;
+    b2 = n0 + n1;
+    int p = self ? 0 : (count ? b1 + o1 : b2 + o2);
+#pragma unroll
+    for (int t = 0; t < CL; t++)
+      if ((m8 >> t) & 1) L.sj[p++] = q[t];
+    if (lane < CL) {
+      const float4 far = make_float4(1.0e5f, 1.0e5f, 1.0e5f, __int_as_float(-1));
+      if (tot1 + lane < n1) L.sj[b1 + tot1 + lane] = far;
+      if (tot2 + lane < n2) L.sj[b2 + tot2 + lane] = far;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    return;
   }
-  const int cnt = __popc(m8);
-  n0 = __ballot(kind == 0) ? CL : 0;  // at most one self entry per item
-  int tot1, tot2 = 0;
-  const int o1 = wave_excl_scan_dpp(kind == 1 ? cnt : 0, tot1);
-  int o2 = 0;
-  if constexpr (!VO) o2 = wave_excl_scan_dpp(kind == 2 ? cnt : 0, tot2);
-  n1 = (tot1 + CL - 1) & ~(CL - 1);
-  n2 = (tot2 + CL - 1) & ~(CL - 1);
+  const int r1 = (p1 + CL - 1) / CL, rounds = r1 + (p2 + CL - 1) / CL;
+  const int at1 = bits_below(m1), at2 = r1 * CL + bits_below(m2);
+  if (pass && my.code >= 0) L.se[(my.code & kCountBit) ? at1 : at2] = my;
+  // the i cluster with itself keeps slot order (at most one such entry)
+  n0 = (mp & md) ? CL : 0;
+  if (n0 && lane < CL) L.sj[lane] = posJ[ci * CL + lane];
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
   b1 = n0;
-  b2 = n0 + n1;
-  if (pass) {
-    if (sub2 == 0) L.sc[ent] = my.code;
-    const int cj = my.code & kCjMask;
-    int p = kind == 0 ? sub2 : (kind == 1 ? b1 + o1 : b2 + o2);
-    if (few) {
-#pragma unroll
-      for (int u = 0; u < 2; u++) {
-        const int t = sub2 + u;
-        if ((m8 >> t) & 1) {
-          L.sj[p] = P3{q[u].x, q[u].y, q[u].z};
-          L.sm[p] = (short)((ent << 3) | t);
-          if constexpr (TWO) L.sa[p] = absJ[cj * CL + t];
-          p++;
-        }
+  int at = n0;       // next staged slot (uniform)
+  n1 = 0;
+  const unsigned t16 = (unsigned)(lane & 7) * 16u;
+  const Entry* se = L.se + (lane >> 3);
+  auto pad = [&]() {
+    const int end = (at + CL - 1) & ~(CL - 1);
+    if (lane < end - at) L.sj[at + lane] = make_float4(1.0e5f, 1.0e5f, 1.0e5f, __int_as_float(-1));
+    at = end;
+  };
+  // atom lane & 7 of the entry: 128 B a cluster, fewer than 2^25 clusters, so
+  // the shift drops the code's other bits and the offset has 32
+  auto load = [&](const Entry& e) {
+    return *(const float4*)((const char*)posJ + (size_t)(((unsigned)e.code << 7) | t16));
+  };
+  auto keep_atom = [&](const Entry& e, float4 q) {
+    q.x += e.dx;
+    q.y += e.dy;
+    q.z += e.dz;
+    const float gx = fmaxf(fabsf(q.x - ic.x) - ih.x, 0.f);
+    const float gy = fmaxf(fabsf(q.y - ic.y) - ih.y, 0.f);
+    const float gz = fmaxf(fabsf(q.z - ic.z) - ih.z, 0.f);
+    const bool keep = fmaf(gz, gz, fmaf(gx, gx, gy * gy)) <= A.prune2;
+    const unsigned long long m = __ballot(keep);
+    if (keep) L.sj[at + bits_below(m)] = q;
+    at += __popcll(m);
+  };
+  if (rounds > 0) {
+    Entry ea = se[0], eb = se[CL];
+    float4 va = load(ea), vb = load(eb);
+    for (int r = 0; r < rounds; r += 2) {
+      const Entry qa = ea, qb = eb;
+      const float4 wa = va, wb = vb;
+      ea = se[(r + 2) * CL];
+      eb = se[(r + 3) * CL];
+      va = load(ea);
+      vb = load(eb);
+      if (r == r1) {
+        pad();
+        n1 = at - b1;
       }
-    } else {
-#pragma unroll
-      for (int t = 0; t < CL; t++) {
-        if ((m8 >> t) & 1) {
-          L.sj[p] = P3{q[t].x, q[t].y, q[t].z};
-          L.sm[p] = (short)((lane << 3) | t);
-          if constexpr (TWO) L.sa[p] = absJ[cj * CL + t];
-          p++;
-        }
+      keep_atom(qa, wa);
+      if (r + 1 == r1) {
+        pad();
+        n1 = at - b1;
       }
+      keep_atom(qb, wb);
     }
   }
-  // padding of each kind up to a multiple of 8: far away, never within D_MAX
-  if (lane < CL) {
-    const P3 far = {1.0e5f, 1.0e5f, 1.0e5f};
-    if (tot1 + lane < n1) {
-      L.sj[b1 + tot1 + lane] = far;
-      L.sm[b1 + tot1 + lane] = -1;
-      if constexpr (TWO) L.sa[b1 + tot1 + lane] = -1;
-    }
-    if (tot2 + lane < n2) {
-      L.sj[b2 + tot2 + lane] = far;
-      L.sm[b2 + tot2 + lane] = -1;
-      if constexpr (TWO) L.sa[b2 + tot2 + lane] = -1;
-    }
+  if (rounds == r1 && (rounds & 1) == 0) {
+    pad();
+    n1 = at - b1;
+  } else {
+    pad();
   }
+  b2 = b1 + n1;
+  n2 = at - b2;
   // the staging above is read by other lanes of this wave only
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -1804,8 +1814,9 @@ constexpr int stage_cap() {
 // staged atoms: lane l evaluates the pair (i = l&7 of cluster ci, j = staged
 // atom 8g + (l>>3)).  VO (value only): no derivatives and no virial;
 // derivative-only entries are skipped, so each unordered pair is visited
-// once.  The pairs in the band around D_MAX^2 are decided at the end of
-// their item on FP64 distances.
+// once.  TWO: the groups share atoms.  The pairs in the band around D_MAX^2
+// (rare) are decided at the end of their item on FP64 distances, from the
+// staged atoms.
 // Outputs: fpart[item][8][3], the derivative of each i atom over the item,
 // and the value / virial / pair count rows described at PairArgs, all over
 // the pairs outside the band plus the FP64 terms of the band pairs inside
@@ -1813,26 +1824,25 @@ constexpr int stage_cap() {
 // sums over all of the wave's items; their wave sums are taken once at the
 // end, converted to FP64 and added to the wave's band sums, and the waves'
 // rows are added in wave order.
+// Bound by VALU issue (16.1 M instructions a launch at 50,000 atoms, 18.1 M when
+// every listed entry was staged).  Known rational 6-12, 50,000 atoms: 38 us
+// (41 before); EXP, 20,000 atoms: 60 us.
 template <int P, bool GENERIC, bool TWO, bool VO, int CH>
 __global__ __launch_bounds__(PAIR_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void k_pairs(
     PairArgs A, const int4* __restrict__ items, const Entry* __restrict__ ents, const float4* __restrict__ posI,
     const float4* __restrict__ posJ, const float4* __restrict__ bbI, const float4* __restrict__ bbJ,
-    const int* __restrict__ absI, const int* __restrict__ absJ, double* __restrict__ fpart,
-    double* __restrict__ partial) {
+    const int* __restrict__ twinI, double* __restrict__ fpart, double* __restrict__ partial) {
   constexpr int NW = PAIR_BLOCK / WAVE;
   constexpr int CAP = stage_cap<CH>();
-  __shared__ P3 sj[NW][CAP];
-  __shared__ short sm[NW][CAP];
-  __shared__ int scode[NW][CH];
-  __shared__ int sabs[TWO ? NW : 1][TWO ? CAP : 1];
-  __shared__ int srec[NW][kBandSlots];
+  __shared__ float4 sj[NW][CAP];
+  __shared__ Entry sent[NW][sent_cap<CH>()];
   __shared__ double stot[NW][8];
   if (A.skip && *A.skip) return;
   const int lane = threadIdx.x & 63;
-  const int w = threadIdx.x >> 6;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int ii = lane & 7, jj = lane >> 3;
   const int nitems = A.nitems_dev ? min(*A.nitems_dev, A.items_cap) : A.nitems;
-  const WaveLds L = {sj[w], sm[w], scode[w], TWO ? sabs[w] : nullptr, srec[w]};
+  const WaveLds L = {sj[w], sent[w]};
   PairAcc acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   int ntot = 0;
   // lanes < 8: the wave's FP64 sums of the band pairs' row entries
@@ -1858,9 +1868,7 @@ __global__ __launch_bounds__(PAIR_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
     const int e = it_n.y + lane;
     if (lane < CH && e < min(it_n.z, A.ent_cap)) my_n = ents[e];
   }
-  // the wave's items with band pairs: bit j for its j-th item (j < 64)
-  unsigned long long bandbits = 0ull;
-  for (int j = 0; k < kend; k += kstride, j++) {
+  for (; k < kend; k += kstride) {
     const int item = k;
     const int4 it = it_n;
     const Entry my_e = my_n;
@@ -1869,10 +1877,10 @@ __global__ __launch_bounds__(PAIR_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
     const int ci = it.x;
     const int e1 = min(it.z, A.ent_cap);
     const float4 pi = posI[ci * CL + ii];
-    const int ai = TWO ? absI[ci * CL + ii] : 0;
+    const int ai = TWO ? twinI[ci * CL + ii] : 0;
     const float4 ic = bbI[2 * ci], ih = bbI[2 * ci + 1];
     int n0, b1, n1, b2, n2;
-    stage_item<TWO, VO, CH>(A, my_e, lane, it.y, e1, ic, ih, posJ, bbJ, absJ, L, n0, b1, n1, b2, n2);
+    stage_item<VO, true, CH>(A, my_e, lane, it.y, e1, ci, ic, ih, posJ, bbJ, L, n0, b1, n1, b2, n2);
     if (kn < kend) {
       const int e = it_n.y + lane;
       my_n = (lane < CH && e < min(it_n.z, A.ent_cap)) ? ents[e] : Entry{0, 0.f, 0.f, 0.f};
@@ -1886,85 +1894,34 @@ __global__ __launch_bounds__(PAIR_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
     // the pair loops issue ahead of the other waves' staging and item ends
     // (measured: the pass takes ~3% less time than with one priority)
     __builtin_amdgcn_s_setprio(1);
-    if (n0) pair_term<P, GENERIC, TWO, VO, 0>(A, L.sj[jj], pi, ii, jj, 0, ai, L, nrec, npair, acc);
+    if (n0) pair_term<P, GENERIC, TWO, VO, 0>(A, L.sj[jj], pi, ii, jj, ai, nrec, npair, acc);
     pair_groups<P, GENERIC, TWO, VO, 1>(A, b1, b1 + n1, pi, ii, jj, ai, L, nrec, npair, acc);
     if constexpr (!VO)
       pair_groups<P, GENERIC, TWO, VO, 2>(A, b2, b2 + n2, pi, ii, jj, ai, L, nrec, npair, acc);
     __builtin_amdgcn_s_setprio(0);
-    if (j < 64) {
-      if (nrec > 0) bandbits |= 1ull << j;
-    } else if (lane == 0) {
-      A.bflag[item] = nrec;
-    }
+    double fadd[3] = {0.0, 0.0, 0.0}, radd = 0.0;
+    if (nrec > 0)
+      band_terms<P, GENERIC, TWO, VO>(A, L, ci, posI, posJ, pi, ii, jj, lane, ai, n0, b1, n1, b2, n2, fadd, radd);
     if constexpr (!VO) {
       const float fx = sum_over_jj(acc.fx), fy = sum_over_jj(acc.fy), fz = sum_over_jj(acc.fz);
       if (jj == 0) {
         double* fp = fpart + (size_t)item * (CL * 3) + ii * 3;
-        fp[0] = -A.df_scale * (double)fx;
-        fp[1] = -A.df_scale * (double)fy;
-        fp[2] = -A.df_scale * (double)fz;
+        fp[0] = -A.df_scale * (double)fx + fadd[0];
+        fp[1] = -A.df_scale * (double)fy + fadd[1];
+        fp[2] = -A.df_scale * (double)fz + fadd[2];
       }
       acc.fx = acc.fy = acc.fz = 0.f;
     }
     if (A.item_partials) {
       const double o = item_row<VO>(A, acc, npair, lane);
-      if (lane < 8) A.ipart[(size_t)item * 8 + lane] = o;
+      if (lane < 8) A.ipart[(size_t)item * 8 + lane] = o + radd;
       acc = PairAcc{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     } else {
       // value and virial stay in the lanes' running sums over the wave's items
       ntot += npair;
+      if (nrec > 0 && lane < 8) stot[w][lane] += radd;
     }
     // the next item overwrites the staging read above
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-  }
-  // the band pairs of the wave's items (rare), item by item after the pass so
-  // that their FP64 registers are not held during it: the item is staged
-  // again and its band terms are added to its outputs in FP64 (each output
-  // by the lane that wrote it above)
-  for (int jb = 0, kb = kfirst; kb < kend; jb++, kb += kstride) {
-    if (jb < 64) {
-      // straight to the next item with band pairs
-      const unsigned long long rest = bandbits >> jb;
-      if (rest == 0ull) {
-        jb = 63;
-        kb = kfirst + 63 * kstride;
-        continue;
-      }
-      const int skip = __builtin_ctzll(rest);
-      jb += skip;
-      kb += skip * kstride;
-    } else if (__builtin_amdgcn_readfirstlane(A.bflag[kb]) == 0) {
-      continue;
-    }
-    const int4 it = items[kb];
-    const int ci = it.x;
-    const int e1 = min(it.z, A.ent_cap);
-    const float4 pi = posI[ci * CL + ii];
-    const int ai = TWO ? absI[ci * CL + ii] : 0;
-    const float4 ic = bbI[2 * ci], ih = bbI[2 * ci + 1];
-    const int e = it.y + lane;
-    const Entry my_e = (lane < CH && e < e1) ? ents[e] : Entry{0, 0.f, 0.f, 0.f};
-    int n0, b1, n1, b2, n2;
-    stage_item<TWO, VO, CH>(A, my_e, lane, it.y, e1, ic, ih, posJ, bbJ, absJ, L, n0, b1, n1, b2, n2);
-    n1 = __builtin_amdgcn_readfirstlane(n1);
-    n2 = __builtin_amdgcn_readfirstlane(n2);
-    b1 = __builtin_amdgcn_readfirstlane(b1);
-    b2 = __builtin_amdgcn_readfirstlane(b2);
-    double fadd[3] = {0.0, 0.0, 0.0}, radd = 0.0;
-    band_terms<P, GENERIC, TWO, VO>(A, L, ci, posI, posJ, pi, ii, jj, lane, ai, n0, b1, n1, b2, n2, fadd, radd);
-    if constexpr (!VO) {
-      if (jj == 0) {
-        double* fp = fpart + (size_t)kb * (CL * 3) + ii * 3;
-        fp[0] += fadd[0];
-        fp[1] += fadd[1];
-        fp[2] += fadd[2];
-      }
-    }
-    if (lane < 8) {
-      if (A.item_partials) A.ipart[(size_t)kb * 8 + lane] += radd;
-      else stot[w][lane] += radd;
-    }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
   }
@@ -2777,40 +2734,104 @@ struct PairTuning {
 // so atom i takes (w_i + w_j)(-dfunc d) from each partner and the box
 // derivative takes (w_i + w_j) dfunc d (x) d once per unordered pair.
 // Band pairs (r^2 within `band` of D_MAX^2) are decided on the spot on the
-// reference's FP64 Pbc::distance.
+// reference's FP64 Pbc::distance, so that they take their place in the lane's
+// sums.  With weights the staged atoms carry their weight where the others
+// carry their requested index (packed positions pwI / pwJ), which the rare band
+// pair then finds by going through the item's rounds again: a third array in
+// LDS would cost a quarter of the resident waves.
 // Outputs: rpart[item][8] (row sums of the i atoms), and with WT fpart
 // [item][8][3] and per-workgroup rows (0, six box-derivative products, 0).
+// 30,000 atoms, WT: 33 us (46 with the weights and indices in LDS arrays of their
+// own, three workgroups a CU).
 constexpr double kContactEps2 = 2.220446049250313e-16;  // DBL_EPSILON
 
-template <int P, bool GENERIC, bool TWO, bool WT, int KIND>
-__device__ __forceinline__ void row_term(const PairArgs& A, const P3& pj, const float4& pi, int ii, int jj, int g,
-                                         int ai, float wi, const float* __restrict__ swt, const WaveLds& L,
-                                         const float4* __restrict__ posJ, const PbcArg* __restrict__ pbc,
-                                         PairAcc& acc, float& cnt) {
-  const float dx = pj.x - pi.x;
-  const float dy = pj.y - pi.y;
-  const float dz = pj.z - pi.z;
-  const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-  const float t = r2 - A.dmax2;
+// requested index of staged atom p of the item in LDS (stage_item's rounds
+// again, on the positions that carry the indices); uniform over the wave
+template <int CH>
+__device__ int staged_index(const PairArgs& A, const WaveLds& L, int p, int n0, int ci, int lane, const float4& ic,
+                            const float4& ih, const float4* __restrict__ posJ) {
+  if (p < n0) return __float_as_int(posJ[ci * CL + p].w);
+  // (self entries come first, then counting and derivative-only ones, each
+  // kind padded to a multiple of 8)
+  int at = n0;
+  bool first = true;
+  for (int r = 0; r < sent_cap<CH>() / CL; r++) {
+    const Entry e = L.se[r * CL + (lane >> 3)];
+    // the first round of the derivative-only entries starts at a multiple of 8
+    const bool deriv = __ballot((lane & 7) == 0 && e.dx < 1.0e5f && !(e.code & kCountBit)) != 0ull;
+    if (deriv && first) {
+      at = (at + CL - 1) & ~(CL - 1);
+      first = false;
+    }
+    float4 q = posJ[(e.code & kCjMask) * CL + (lane & 7)];
+    const int req = __float_as_int(q.w);
+    q.x += e.dx;
+    q.y += e.dy;
+    q.z += e.dz;
+    const float gx = fmaxf(fabsf(q.x - ic.x) - ih.x, 0.f);
+    const float gy = fmaxf(fabsf(q.y - ic.y) - ih.y, 0.f);
+    const float gz = fmaxf(fabsf(q.z - ic.z) - ih.z, 0.f);
+    const bool keep = fmaf(gz, gz, fmaf(gx, gx, gy * gy)) <= A.prune2;
+    const unsigned long long m = __ballot(keep);
+    const int n = __popcll(m);
+    if (p < at + n) {
+      const unsigned long long mine = __ballot(keep && at + bits_below(m) == p);
+      return p >= at && mine ? __builtin_amdgcn_readlane(req, __builtin_ctzll(mine)) : -1;
+    }
+    at += n;
+  }
+  return -1;
+}
+
+// per-item constants of the row kernel
+struct RowItem {
+  int ci, n0, reqi;
+  float4 ic, ih;
+  const float4* idxJ;  // packed positions with requested indices
+  const PbcArg* pbc;
+};
+
+template <int P, bool GENERIC, bool TWO, bool WT, int KIND, int CH>
+__device__ __forceinline__ void row_term(const PairArgs& A, const RowItem& I, const float4& pj, const float4& pi,
+                                         int ii, int jj, int g, int lane, int ai, float wi, const WaveLds& L,
+                                         PairAcc& acc, int& cnt) {
+  float dx, dy, dz;
+  const float r2 = pair_d(pj, pi, dx, dy, dz);
   bool keep = r2 >= A.contact2;
   if constexpr (KIND == 0) keep = keep && jj != ii;
-  if constexpr (TWO) keep = keep && (L.sa[g + jj] != ai);
+  if constexpr (TWO && !WT) keep = keep && (__float_as_int(pj.w) != ai);
+  const float t = r2 - A.dmax2;
+  const unsigned long long bm = __ballot(keep && fabsf(t) < A.band);
   bool cut = keep && t <= 0.f;
-  if (keep && fabsf(t) < A.band) {
-    const int meta = L.sm[g + jj];
-    const int reqi = __float_as_int(pi.w);
-    if (reqi >= 0 && meta >= 0) {
-      const int cj = L.sc[meta >> 3] & kCjMask;
-      const int reqj = __float_as_int(posJ[cj * CL + (meta & 7)].w);
-      if (reqj >= 0) cut = switch_inside(A.sw, exact_r2(pbc, A.pos64, reqi, reqj));
+  if constexpr (TWO && WT) {
+    // (rare groups that share atoms: the index decides each pair inside)
+    for (unsigned long long m = __ballot(cut) | bm; m; m &= m - 1) {
+      const int l = __builtin_ctzll(m);
+      const int reqj = staged_index<CH>(A, L, g + (l >> 3), I.n0, I.ci, lane, I.ic, I.ih, I.idxJ);
+      if (lane == l && reqj == ai) cut = keep = false;
+    }
+  }
+  if (bm != 0ull) {  // uniform, rare
+    for (unsigned long long m = bm; m; m &= m - 1) {
+      const int l = __builtin_ctzll(m);
+      int reqj;
+      if constexpr (WT) reqj = staged_index<CH>(A, L, g + (l >> 3), I.n0, I.ci, lane, I.ic, I.ih, I.idxJ);
+      else reqj = __float_as_int(pj.w);
+      if (lane == l && keep && I.reqi >= 0 && reqj >= 0)
+        cut = switch_inside(A.sw, exact_r2(I.pbc, A.pos64, I.reqi, reqj));
     }
   }
   float sv, dfu;
-  pair_switch<P, GENERIC>(A, r2, sv, dfu);
-  acc.sv += cut ? sv : 0.f;
-  cnt += cut ? 1.f : 0.f;
+  if constexpr (GENERIC) {
+    sv = dfu = 0.f;
+    if (cut) pair_switch<P, GENERIC>(A, r2, sv, dfu);
+  } else {
+    sw_fixed_x<P>(cut ? r2 : sw_far<P>(), sv, dfu);
+  }
+  acc.sv += sv;
+  cnt += cut ? 1 : 0;
   if constexpr (WT) {
-    const float wg = cut ? (wi + swt[g + jj]) * dfu : 0.f;
+    const float wg = (cut ? wi + pj.w : 0.f) * dfu;
     const float gx = wg * dx, gy = wg * dy, gz = wg * dz;
     acc.fx += gx;
     acc.fy += gy;
@@ -2830,27 +2851,22 @@ __device__ __forceinline__ void row_term(const PairArgs& A, const P3& pj, const 
 }
 
 template <int P, bool GENERIC, bool TWO, bool WT>
-__global__ __launch_bounds__(PAIR_BLOCK) void k_rows(PairArgs A, const float* __restrict__ wreq,
-                                                     const int4* __restrict__ items, const Entry* __restrict__ ents,
-                                                     const float4* __restrict__ posI, const float4* __restrict__ posJ,
-                                                     const float4* __restrict__ bbI, const float4* __restrict__ bbJ,
-                                                     const int* __restrict__ absI, const int* __restrict__ absJ,
-                                                     double* __restrict__ rpart, double* __restrict__ fpart,
-                                                     double* __restrict__ partial) {
+__global__ __launch_bounds__(PAIR_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void k_rows(
+    PairArgs A, const int4* __restrict__ items, const Entry* __restrict__ ents, const float4* __restrict__ posI,
+    const float4* __restrict__ posJ, const float4* __restrict__ pwI, const float4* __restrict__ pwJ,
+    const float4* __restrict__ bbI, const float4* __restrict__ bbJ, const int* __restrict__ twinI,
+    double* __restrict__ rpart, double* __restrict__ fpart, double* __restrict__ partial) {
   constexpr int CH = 64;
   constexpr int NW = PAIR_BLOCK / WAVE;
   constexpr int CAP = stage_cap<CH>();
-  __shared__ P3 sj[NW][CAP];
-  __shared__ short sm[NW][CAP];
-  __shared__ int scode[NW][CH];
-  __shared__ int sabs[TWO ? NW : 1][TWO ? CAP : 1];
-  __shared__ float swt[WT ? NW : 1][WT ? CAP : 1];
+  __shared__ float4 sj[NW][CAP];
+  __shared__ Entry sent[NW][sent_cap<CH>()];
   __shared__ double stot[NW][8];
   const int lane = threadIdx.x & 63;
-  const int w = threadIdx.x >> 6;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int ii = lane & 7, jj = lane >> 3;
   const int nitems = A.nitems_dev ? min(*A.nitems_dev, A.items_cap) : A.nitems;
-  const WaveLds L = {sj[w], sm[w], scode[w], TWO ? sabs[w] : nullptr};
+  const WaveLds L = {sj[w], sent[w]};
   if (lane < 8) stot[w][lane] = 0.0;
   for (int k = blockIdx.x * NW + w; k < nitems; k += gridDim.x * NW) {
     const int item = k;
@@ -2858,46 +2874,33 @@ __global__ __launch_bounds__(PAIR_BLOCK) void k_rows(PairArgs A, const float* __
     const int ci = it.x;
     const int e1 = min(it.z, A.ent_cap);
     const float4 pi = posI[ci * CL + ii];
-    const int ai = TWO ? absI[ci * CL + ii] : 0;
-    const float4 ic = bbI[2 * ci], ih = bbI[2 * ci + 1];
-    const PbcArg* pbc = A.pbc + nsys_of(A.cl_sys, ci);
+    const int ai = TWO ? twinI[ci * CL + ii] : 0;
+    RowItem I;
+    I.ci = ci;
+    I.reqi = __float_as_int(pi.w);
+    I.ic = bbI[2 * ci];
+    I.ih = bbI[2 * ci + 1];
+    I.idxJ = posJ;
+    I.pbc = A.pbc + nsys_of(A.cl_sys, ci);
     Entry my_e = {0, 0.f, 0.f, 0.f};
     if (lane < CH && it.y + lane < e1) my_e = ents[it.y + lane];
     int n0, b1, n1, b2, n2;
-    stage_item<TWO, false, CH>(A, my_e, lane, it.y, e1, ic, ih, posJ, bbJ, absJ, L, n0, b1, n1, b2, n2);
+    stage_item<false, false, CH>(A, my_e, lane, it.y, e1, ci, I.ic, I.ih, WT ? pwJ : posJ, bbJ, L, n0, b1, n1, b2, n2);
     n1 = __builtin_amdgcn_readfirstlane(n1);
     n2 = __builtin_amdgcn_readfirstlane(n2);
     b1 = __builtin_amdgcn_readfirstlane(b1);
     b2 = __builtin_amdgcn_readfirstlane(b2);
-    float wi = 0.f;
-    if constexpr (WT) {
-      // weights of the staged atoms (0 for padding)
-      const int nst = b2 + n2;
-      for (int p = lane; p < nst; p += WAVE) {
-        const int meta = L.sm[p];
-        float wv = 0.f;
-        if (meta >= 0) {
-          const int cj = L.sc[meta >> 3] & kCjMask;
-          const int req = __float_as_int(posJ[cj * CL + (meta & 7)].w);
-          if (req >= 0) wv = wreq[req];
-        }
-        swt[w][p] = wv;
-      }
-      const int reqi = __float_as_int(pi.w);
-      wi = reqi >= 0 ? wreq[reqi] : 0.f;
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-    }
-    const float* sw = WT ? swt[w] : nullptr;
+    I.n0 = n0;
+    const float wi = WT ? pwI[ci * CL + ii].w : 0.f;
     PairAcc acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    float cnt = 0.f;
-    if (n0) row_term<P, GENERIC, TWO, WT, 0>(A, L.sj[jj], pi, ii, jj, 0, ai, wi, sw, L, posJ, pbc, acc, cnt);
+    int cnt = 0;
+    if (n0) row_term<P, GENERIC, TWO, WT, 0, CH>(A, I, L.sj[jj], pi, ii, jj, 0, lane, ai, wi, L, acc, cnt);
     for (int g = b1; g < b1 + n1; g += CL)
-      row_term<P, GENERIC, TWO, WT, 1>(A, L.sj[g + jj], pi, ii, jj, g, ai, wi, sw, L, posJ, pbc, acc, cnt);
+      row_term<P, GENERIC, TWO, WT, 1, CH>(A, I, L.sj[g + jj], pi, ii, jj, g, lane, ai, wi, L, acc, cnt);
     for (int g = b2; g < b2 + n2; g += CL)
-      row_term<P, GENERIC, TWO, WT, 2>(A, L.sj[g + jj], pi, ii, jj, g, ai, wi, sw, L, posJ, pbc, acc, cnt);
+      row_term<P, GENERIC, TWO, WT, 2, CH>(A, I, L.sj[g + jj], pi, ii, jj, g, lane, ai, wi, L, acc, cnt);
     // rows of the 8 i atoms: s = stretch * s~ + shift per contributing pair
-    const float cs = sum_over_jj(acc.sv), cc = sum_over_jj(cnt);
+    const float cs = sum_over_jj(acc.sv), cc = sum_over_jj((float)cnt);
     if (jj == 0) rpart[(size_t)item * CL + ii] = A.sv_scale * (double)cs + A.sv_shift * (double)cc;
     if constexpr (WT) {
       const float fx = sum_over_jj(acc.fx), fy = sum_over_jj(acc.fy), fz = sum_over_jj(acc.fz);
@@ -2953,25 +2956,31 @@ __global__ __launch_bounds__(256) void k_gather_rows(int nslot, const float4* __
   rows[req] = sum;
 }
 
-// FP32 weight of every requested atom: w[k] for the first nrows, 0 after
-__global__ void k_row_weights(int nrows, int natoms, const double* __restrict__ w, float* __restrict__ wreq) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < natoms) wreq[k] = k < nrows ? (float)w[k] : 0.f;
+// packed positions with the atom's FP32 weight in w: w[k] for the first nrows
+// requested atoms, 0 for the others and for padding
+__global__ void k_row_weights(int nslot, int nrows, const float4* __restrict__ p, const double* __restrict__ w,
+                              float4* __restrict__ pw) {
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= nslot) return;
+  float4 q = p[s];
+  const int req = __float_as_int(q.w);
+  q.w = req >= 0 && req < nrows ? (float)w[req] : 0.f;
+  pw[s] = q;
 }
 
 inline void pair_args_generic(PairArgs& A);
 
-inline void launch_rows(const PairArgs& A, bool weighted, int grid, hipStream_t s, const float* wreq,
-                        const int4* items, const Entry* ents, const float4* posI, const float4* posJ,
-                        const float4* bbI, const float4* bbJ, const int* absI, const int* absJ, double* rpart,
+inline void launch_rows(const PairArgs& A, bool weighted, int grid, hipStream_t s, const int4* items,
+                        const Entry* ents, const float4* posI, const float4* posJ, const float4* pwI,
+                        const float4* pwJ, const float4* bbI, const float4* bbJ, const int* twinI, double* rpart,
                         double* fpart, double* partial) {
   const p2a_switch& sw = A.sw;
 #define P2A_R(P, GEN, TWO, WT)                                                                                   \
-  hipLaunchKernelGGL((k_rows<P, GEN, TWO, WT>), dim3(grid), dim3(PAIR_BLOCK), 0, s, A, wreq, items, ents, posI,   \
-                     posJ, bbI, bbJ, absI, absJ, rpart, fpart, partial)
+  hipLaunchKernelGGL((k_rows<P, GEN, TWO, WT>), dim3(grid), dim3(PAIR_BLOCK), 0, s, A, items, ents, posI, posJ,   \
+                     pwI, pwJ, bbI, bbJ, twinI, rpart, fpart, partial)
 #define P2A_RSW(P, GEN)                                        \
   do {                                                         \
-    if (A.twogroup) {                                          \
+    if (A.share) {                                             \
       if (weighted) P2A_R(P, GEN, true, true);                 \
       else P2A_R(P, GEN, true, false);                         \
     } else {                                                   \
@@ -3003,18 +3012,19 @@ inline int switch_known_kind(const p2a_switch& sw) {
 }
 
 // launch of the pair kernel for a switch, group mode and tuning.  TWOG: the
-// caller has two groups (else only the kernels of one group are compiled).
+// caller may have two groups that share atoms (else the kernels that compare
+// atom indices are not compiled); distinct groups run the kernels of one group.
 // The other switches have a kernel of their own for the default work items
 // with derivatives (20,000 atoms with EXP: pair pass 105 -> 62 us); value only and 32 entries
 // an item run the kernel that takes any switch.
 template <bool TWOG>
 inline void launch_pairs(const PairArgs& A, int grid, hipStream_t s, bool value_only, int chunk, const int4* items,
                          const Entry* ents, const float4* posI, const float4* posJ, const float4* bbI,
-                         const float4* bbJ, const int* absI, const int* absJ, double* fpart, double* partial) {
+                         const float4* bbJ, const int* twinI, double* fpart, double* partial) {
   const p2a_switch& sw = A.sw;
 #define P2A_K(P, GEN, TWO, VO, CH)                                                                                \
   hipLaunchKernelGGL((k_pairs<P, GEN, TWO, VO, CH>), dim3(grid), dim3(PAIR_BLOCK), 0, s, A, items, ents, posI,      \
-                     posJ, bbI, bbJ, absI, absJ, fpart, partial)
+                     posJ, bbI, bbJ, twinI, fpart, partial)
 #define P2A_KCH(P, GEN, TWO, VO)          \
   do {                                    \
     if (chunk == 32) P2A_K(P, GEN, TWO, VO, 32); \
@@ -3023,7 +3033,7 @@ inline void launch_pairs(const PairArgs& A, int grid, hipStream_t s, bool value_
 #define P2A_KSW(P, GEN)                                     \
   do {                                                      \
     if constexpr (TWOG) {                                   \
-      if (A.twogroup) {                                     \
+      if (A.share) {                                        \
         if (value_only) P2A_KCH(P, GEN, true, true);        \
         else P2A_KCH(P, GEN, true, false);                  \
         break;                                              \
@@ -3035,7 +3045,7 @@ inline void launch_pairs(const PairArgs& A, int grid, hipStream_t s, bool value_
 #define P2A_KKN(K)                                              \
   case K:                                                       \
     if constexpr (TWOG) {                                       \
-      if (A.twogroup) { P2A_K(K, true, true, false, 64); break; } \
+      if (A.share) { P2A_K(K, true, true, false, 64); break; }  \
     }                                                           \
     P2A_K(K, true, false, false, 64);                           \
     break
