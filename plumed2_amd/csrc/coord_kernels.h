@@ -1420,13 +1420,6 @@ __device__ __forceinline__ void pair_switch(const PairArgs& A, float r2, float& 
   }
 }
 
-// FP32 r^2 at which the switch of a pair in the band is evaluated once its FP64
-// distance has put it inside: at most a rounding below D_MAX^2, as an FP32 r^2
-// beyond it would give zero
-__device__ __forceinline__ float inside_r2(const PairArgs& A, float r2) {
-  return fminf(r2, A.dmax2 * (1.f - 0x1p-22f));
-}
-
 // FP32 separation and r^2 of staged atom pj from i atom pi (the one sequence
 // of operations for a pair in the FP32 pass and in its band decisions)
 __device__ __forceinline__ float pair_d(const float4& pj, const float4& pi, float& dx, float& dy, float& dz) {
@@ -1592,7 +1585,7 @@ __device__ __forceinline__ void band_terms(const PairArgs& A, const WaveLds& L, 
       const int reqj = __float_as_int(L.sj[st].w);
       if (reqi >= 0 && reqj >= 0 && switch_inside(A.sw, exact_r2(pbc, A.pos64, reqi, reqj))) {
         float dfu;
-        pair_switch<P, GENERIC>(A, GENERIC ? inside_r2(A, r2) : r2, sv, dfu);
+        pair_switch<P, GENERIC>(A, r2, sv, dfu);
         if constexpr (!VO) {
           g[0] = dfu * d[0];
           g[1] = dfu * d[1];
@@ -2810,7 +2803,6 @@ __device__ __forceinline__ void row_term(const PairArgs& A, const RowItem& I, co
   const float t = r2 - A.dmax2;
   const unsigned long long bm = __ballot(keep && fabsf(t) < A.band);
   bool cut = keep && t <= 0.f;
-  float rs = r2;
   if constexpr (TWO && WT) {
     // (rare groups that share atoms: the index decides each pair inside)
     for (unsigned long long m = __ballot(cut) | bm; m; m &= m - 1) {
@@ -2825,16 +2817,14 @@ __device__ __forceinline__ void row_term(const PairArgs& A, const RowItem& I, co
       int reqj;
       if constexpr (WT) reqj = staged_index<CH>(A, L, g + (l >> 3), I.n0, I.ci, lane, I.ic, I.ih, I.idxJ);
       else reqj = __float_as_int(pj.w);
-      if (lane == l && keep && I.reqi >= 0 && reqj >= 0) {
+      if (lane == l && keep && I.reqi >= 0 && reqj >= 0)
         cut = switch_inside(A.sw, exact_r2(I.pbc, A.pos64, I.reqi, reqj));
-        if (GENERIC && cut) rs = inside_r2(A, r2);
-      }
     }
   }
   float sv, dfu;
   if constexpr (GENERIC) {
     sv = dfu = 0.f;
-    if (cut) pair_switch<P, GENERIC>(A, rs, sv, dfu);
+    if (cut) pair_switch<P, GENERIC>(A, r2, sv, dfu);
   } else {
     sw_fixed_x<P>(cut ? r2 : sw_far<P>(), sv, dfu);
   }
