@@ -1586,6 +1586,8 @@ __device__ __forceinline__ void band_terms(const PairArgs& A, const WaveLds& L, 
       if (reqi >= 0 && reqj >= 0 && switch_inside(A.sw, exact_r2(pbc, A.pos64, reqi, reqj))) {
         float dfu;
         pair_switch<P, GENERIC>(A, r2, sv, dfu);
+        // as the any-switch kernel (P == 0), whose switch ends at D_MAX
+        if (GENERIC && P != 0 && !switch_inside(A.sw, (double)r2 * A.r2_real)) sv = dfu = 0.f;
         if constexpr (!VO) {
           g[0] = dfu * d[0];
           g[1] = dfu * d[1];
