@@ -107,7 +107,10 @@ struct SysArg {
   float rb[3];    // list radius as a fraction of the cell along a, b, c (r * |reciprocal row|)
   int ncx, ncy;   // columns along a and b
   int colbase;    // first column of this system in the shared column arrays
-  int pad_;
+  float icx, icy;  // 1/ncx, 1/ncy
+  // a cell along the axes (column_window): its squared edges a and b, 1/|c|
+  int ortho;
+  float aa, bb, invc;
 };
 
 struct PbcArg {
@@ -138,16 +141,24 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
-// exclusive prefix sum over the 64 lanes; *total = sum of all lanes
-__device__ __forceinline__ int wave_excl_scan(int v, int lane, int& total) {
-  int x = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_up(x, o, 64);
-    if (lane >= o) x += y;
-  }
-  total = __shfl(x, 63, 64);
-  return x - v;
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_i(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
+}
+constexpr int kShr1 = 0x111, kShr2 = 0x112, kShr4 = 0x114, kShr8 = 0x118;
+constexpr int kBcast15 = 0x142, kBcast31 = 0x143;
+// exclusive prefix sum over the 64 lanes (all active); total = sum of all lanes
+// (uniform)
+__device__ __forceinline__ int wave_excl_scan(int x, int& total) {
+  int v = x;
+  v += dpp_i<kShr1, 0xF>(v);
+  v += dpp_i<kShr2, 0xF>(v);
+  v += dpp_i<kShr4, 0xF>(v);
+  v += dpp_i<kShr8, 0xF>(v);
+  v += dpp_i<kBcast15, 0xA>(v);
+  v += dpp_i<kBcast31, 0xC>(v);
+  total = __builtin_amdgcn_readlane(v, 63);
+  return v - x;
 }
 
 // exclusive prefix sums of a and c over the workgroup (at most 1024 threads):
@@ -156,8 +167,8 @@ __device__ __forceinline__ int wave_excl_scan(int v, int lane, int& total) {
 __device__ __forceinline__ void block_excl_scan2(int& a, int& c, int& ta, int& tc, int* sw) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
   int wa, wc;
-  const int ea = wave_excl_scan(a, lane, wa);
-  const int ec = wave_excl_scan(c, lane, wc);
+  const int ea = wave_excl_scan(a, wa);
+  const int ec = wave_excl_scan(c, wc);
   if (lane == 0) {
     sw[w] = wa;
     sw[16 + w] = wc;
@@ -179,8 +190,6 @@ __device__ __forceinline__ void block_excl_scan2(int& a, int& c, int& ta, int& t
   c = pc + ec;
   __syncthreads();
 }
-
-__device__ __forceinline__ int floordiv(int a, int n) { return (a >= 0) ? a / n : -((-a + n - 1) / n); }
 
 __device__ __forceinline__ int nsys_of(const int* idx, int i) { return idx ? idx[i] : 0; }
 
@@ -291,22 +300,6 @@ __global__ __launch_bounds__(256) void k_bin(int n, const double* __restrict__ p
 // receive the two totals.
 constexpr int kScanBlock = 1024;  // elements per workgroup (256 threads x 4)
 
-__device__ __forceinline__ int block_excl_scan256(int v, int* sh, int& total) {
-  const int t = threadIdx.x;
-  sh[t] = v;
-  __syncthreads();
-  for (int o = 1; o < 256; o <<= 1) {
-    const int u = (t >= o) ? sh[t - o] : 0;
-    __syncthreads();
-    sh[t] += u;
-    __syncthreads();
-  }
-  total = sh[255];
-  const int r = sh[t] - v;
-  __syncthreads();
-  return r;
-}
-
 // the same two scans in one workgroup of 1024 threads (a contiguous run of at
 // most 8 counts per thread), for counts that one workgroup scans faster than
 // three launches
@@ -349,7 +342,7 @@ __global__ __launch_bounds__(1024) void k_scan2_one(int n, const int* __restrict
 
 __global__ __launch_bounds__(256) void k_scan2_sums(int n, const int* __restrict__ n_dev, const int* __restrict__ in,
                                                     int chunk, int* __restrict__ bsum) {
-  __shared__ int sh[256];
+  __shared__ int sw[32];
   if (n_dev) n = *n_dev;
   const int base = blockIdx.x * kScanBlock + threadIdx.x * 4;
   int a = 0, c = 0;
@@ -361,8 +354,7 @@ __global__ __launch_bounds__(256) void k_scan2_sums(int n, const int* __restrict
     }
   }
   int ta, tc;
-  block_excl_scan256(a, sh, ta);
-  block_excl_scan256(c, sh, tc);
+  block_excl_scan2(a, c, ta, tc, sw);
   if (threadIdx.x == 0) {
     bsum[2 * blockIdx.x] = ta;
     bsum[2 * blockIdx.x + 1] = tc;
@@ -412,7 +404,7 @@ __global__ __launch_bounds__(1024) void k_scan2_blocks(int nb, int n, const int*
 __global__ __launch_bounds__(256) void k_scan2_apply(int n, const int* __restrict__ n_dev, const int* __restrict__ in,
                                                      int chunk, const int* __restrict__ bsum, int* __restrict__ out0,
                                                      int* __restrict__ out1) {
-  __shared__ int sh[256];
+  __shared__ int sw[32];
   if (n_dev) n = *n_dev;
   if (blockIdx.x * kScanBlock >= n) return;  // uniform per workgroup
   const int base = blockIdx.x * kScanBlock + threadIdx.x * 4;
@@ -425,8 +417,8 @@ __global__ __launch_bounds__(256) void k_scan2_apply(int n, const int* __restric
     c += vc[k];
   }
   int ta, tc;
-  int ra = block_excl_scan256(a, sh, ta) + bsum[2 * blockIdx.x];
-  int rc = block_excl_scan256(c, sh, tc) + bsum[2 * blockIdx.x + 1];
+  block_excl_scan2(a, c, ta, tc, sw);
+  int ra = a + bsum[2 * blockIdx.x], rc = c + bsum[2 * blockIdx.x + 1];
   for (int k = 0; k < 4; k++) {
     const int i = base + k;
     if (i < n) {
@@ -767,12 +759,48 @@ struct ListArgs {
 // Candidates are the clusters of the (column, image) window around the i
 // cluster whose range of fractional c overlaps the i cluster's range widened
 // by the list radius: a pair closer than r differs by at most r*|c*| in
-// fractional c, so the window is exact, and the clusters of a column are
-// sorted along c, so each window is one binary-searched run of clusters.
+// fractional c, so the window is exact; in a cell along the axes by what the
+// radius leaves after the gap between the two columns (column_window).  (In a
+// skewed cell the boxes of clusters reach out of their columns, and an entry
+// left out for the columns' sake would move the list's work items, and with
+// them the FP32 sums.)  The clusters of a column are sorted along c, so each
+// window is one binary-searched run of clusters (both ends searched together).
 // Each column lane writes its runs into the wave's candidate list in LDS
 // (j cluster | image code, in column order), kCandCap at a time, and the
 // lanes then test the listed candidates, two per lane and trip.
+// Bound by VALU issue (half of its time at 50,000 atoms) and the search's chain
+// of loads.  50,000 atoms, radius 1.3: 14 us; 31 us with whole windows (nine by
+// nine columns, 520 candidates for 190 entries) searched end after end.
 constexpr int kCandCap = 512;
+
+// t / n and t % n for 0 <= t < 2^31, r = 1/n to a few roundings: the quotient is
+// off by one at most
+__device__ __forceinline__ int div_by(int t, int n, float r, int& rem) {
+  int q = (int)((float)t * r);
+  rem = t - q * n;
+  if (rem < 0) {
+    q--;
+    rem += n;
+  } else if (rem >= n) {
+    q++;
+    rem -= n;
+  }
+  return q;
+}
+
+// Half width, in fractional c, of the range around the i cluster that can hold a
+// cluster within the list radius, for a column whose differences in fractional a
+// and b lie in [a0, a1] and [b0, b1] (a cell along the axes: the boxes of
+// clusters stay within their columns, so the gap between the columns bounds the
+// gap between the boxes); negative where there is none.  The radius is widened
+// by more than the rounding of the boxes' coordinates.
+__device__ __forceinline__ float column_window(const SysArg& S, float rlist2, float a0, float a1, float b0, float b1) {
+  const float fa = fminf(fmaxf(0.f, a0), a1), fb = fminf(fmaxf(0.f, b0), b1);
+  const float left = rlist2 * 1.0001f - S.aa * fa * fa - S.bb * fb * fb;
+  if (left < 0.f) return -1.f;
+  return fminf(__builtin_amdgcn_sqrtf(left) * S.invc + 2.0e-6f, S.rb[2]);
+}
+
 template <int FILL>
 __global__ __launch_bounds__(256) void k_list(ListArgs L, const int* __restrict__ cl_colI,
                                               const int* __restrict__ cl_sysI, const SysArg* __restrict__ sysI,
@@ -783,8 +811,9 @@ __global__ __launch_bounds__(256) void k_list(ListArgs L, const int* __restrict_
                                               int* __restrict__ count, const int* __restrict__ start,
                                               Entry* __restrict__ out, unsigned* __restrict__ ell) {
   __shared__ unsigned s_cand[4][kCandCap];
+  __shared__ float4 s_img[4][27];  // FP32 lattice translation of each image code
   const int lane = threadIdx.x & 63;
-  const int wv = threadIdx.x / WAVE;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / WAVE);
   const int nclI = L.nclI_dev ? *L.nclI_dev : L.nclI;
   // FILL=0/1: cluster ci = the wave.  FILL=2: the wave's 64 clusters, of which
   // it searches those whose candidates did not all fit in ell (the others are
@@ -808,20 +837,34 @@ __global__ __launch_bounds__(256) void k_list(ListArgs L, const int* __restrict_
   const SysArg& SI = sysI[s];
   const SysArg& SJ = sysJ[s];
   const int colI = cl_colI[ci] - SI.colbase;
-  const int cxi = colI % SI.ncx, cyi = colI / SI.ncx;
+  int cxi;
+  const int cyi = div_by(colI, SI.ncx, SI.icx, cxi);
   const float4 ic = bbI[2 * ci], ih = bbI[2 * ci + 1];
   const float2 ki = krI[ci];
-  const int x0 = (int)floorf(((float)cxi / SI.ncx - SJ.rb[0]) * SJ.ncx) - 1;
-  const int x1 = (int)floorf(((float)(cxi + 1) / SI.ncx + SJ.rb[0]) * SJ.ncx) + 1;
-  const int y0 = (int)floorf(((float)cyi / SI.ncy - SJ.rb[1]) * SJ.ncy) - 1;
-  const int y1 = (int)floorf(((float)(cyi + 1) / SI.ncy + SJ.rb[1]) * SJ.ncy) + 1;
+  // columns that a pair closer than the list radius can lie in; the margin is
+  // above the rounding of the fractions
+  constexpr float kMargin = 4.0e-6f;
+  const bool ortho = SJ.ortho != 0;  // uniform
+  const float xi0 = (float)cxi * SI.icx - kMargin, xi1 = (float)(cxi + 1) * SI.icx + kMargin;
+  const float yi0 = (float)cyi * SI.icy - kMargin, yi1 = (float)(cyi + 1) * SI.icy + kMargin;
+  int x0, x1, y0, y1;
+  if (ortho) {
+    x0 = (int)floorf((xi0 - SJ.rb[0] * 1.00001f) * SJ.ncx);
+    x1 = (int)floorf((xi1 + SJ.rb[0] * 1.00001f) * SJ.ncx);
+    y0 = (int)floorf((yi0 - SJ.rb[1] * 1.00001f) * SJ.ncy);
+    y1 = (int)floorf((yi1 + SJ.rb[1] * 1.00001f) * SJ.ncy);
+  } else {
+    x0 = (int)floorf(((float)cxi / SI.ncx - SJ.rb[0]) * SJ.ncx) - 1;
+    x1 = (int)floorf(((float)(cxi + 1) / SI.ncx + SJ.rb[0]) * SJ.ncx) + 1;
+    y0 = (int)floorf(((float)cyi / SI.ncy - SJ.rb[1]) * SJ.ncy) - 1;
+    y1 = (int)floorf(((float)(cyi + 1) / SI.ncy + SJ.rb[1]) * SJ.ncy) + 1;
+  }
   // images -1, 0, +1 along a and b cover every candidate when the cell is
   // wider than 2*rlist; each unwrapped column is a distinct (column, image)
   const int xa = max(x0, -SJ.ncx), xb = min(x1, 2 * SJ.ncx - 1);
   const int ya = max(y0, -SJ.ncy), yb = min(y1, 2 * SJ.ncy - 1);
   const int nx = xb - xa + 1, ny = yb - ya + 1;
   const int ncolw = nx * ny;
-  const float zlo = ki.x - SJ.rb[2] - 1.0e-6f, zhi = ki.y + SJ.rb[2] + 1.0e-6f;
   const double4 oi = orgI[ci];
   int n = 0;
   const int base = FILL ? start[ci] : 0;
@@ -837,41 +880,58 @@ __global__ __launch_bounds__(256) void k_list(ListArgs L, const int* __restrict_
       return;
     }
   }
+  if (lane < 27) {
+    const int mx = lane % 3 - 1, my = (lane / 3) % 3 - 1, mz = lane / 9 - 1;
+    s_img[wv][lane] = make_float4(mx * SJ.af[0] + my * SJ.af[3] + mz * SJ.af[6],
+                                  mx * SJ.af[1] + my * SJ.af[4] + mz * SJ.af[7],
+                                  mx * SJ.af[2] + my * SJ.af[5] + mz * SJ.af[8], 0.f);
+  }
+  const float sx = SJ.icx, sy = SJ.icy, inx = __builtin_amdgcn_rcpf((float)nx);
   // one lane per window column; it covers the images -1, 0, +1 along c, of
   // which only those whose shifted window meets [0, 1) are searched
   for (int t0 = 0; t0 < ncolw; t0 += WAVE) {
     const int t = t0 + lane;
     int f[3] = {0, 0, 0}, cnt[3] = {0, 0, 0}, img = 0;
     if (t < ncolw) {
-      const int cxu = xa + t % nx, cyu = ya + t / nx;
-      const int mx = floordiv(cxu, SJ.ncx), cxw = cxu - mx * SJ.ncx;
-      const int my = floordiv(cyu, SJ.ncy), cyw = cyu - my * SJ.ncy;
+      int tx;
+      const int ty = div_by(t, nx, inx, tx), cxu = xa + tx, cyu = ya + ty;
+      const int mx = cxu < 0 ? -1 : (cxu >= SJ.ncx ? 1 : 0), my = cyu < 0 ? -1 : (cyu >= SJ.ncy ? 1 : 0);
+      const int cxw = cxu - mx * SJ.ncx, cyw = cyu - my * SJ.ncy;
       const int col = SJ.colbase + cxw + SJ.ncx * cyw;
       const int c0 = col_clJ[col], c1 = col_clJ[col + 1];
       img = (mx + 1) | ((my + 1) << 2);
+      const float zw = ortho ? column_window(SJ, L.rlist2, cxu * sx - xi1, (cxu + 1) * sx - xi0, cyu * sy - yi1,
+                                             (cyu + 1) * sy - yi0)
+                             : SJ.rb[2];
+      const float zlo = ki.x - zw - 1.0e-6f, zhi = ki.y + zw + 1.0e-6f;
+      if (zw >= 0.f && c1 > c0) {
 #pragma unroll
-      for (int m = 0; m < 3; m++) {
-        const float lo = zlo - (float)(m - 1), hi = zhi - (float)(m - 1);
-        if (hi >= 0.f && lo < 1.f && c1 > c0) {
-          int a = c0, b = c1;
-          while (a < b) {  // first cluster whose upper key reaches lo
-            const int q = (a + b) >> 1;
-            if (krJ[q].y < lo) a = q + 1;
-            else b = q;
+        for (int m = 0; m < 3; m++) {
+          const float lo = zlo - (float)(m - 1), hi = zhi - (float)(m - 1);
+          if (hi >= 0.f && lo < 1.f) {
+            // [a, .): first cluster whose upper key reaches lo; [., u): first
+            // cluster whose lower key exceeds hi
+            int a = c0, b = c1, u = c0, v = c1;
+            while (a < b || u < v) {
+              const int q = min((a + b) >> 1, c1 - 1), r = min((u + v) >> 1, c1 - 1);
+              const float ky = krJ[q].y, kx = krJ[r].x;
+              if (a < b) {
+                if (ky < lo) a = q + 1;
+                else b = q;
+              }
+              if (u < v) {
+                if (kx <= hi) u = r + 1;
+                else v = r;
+              }
+            }
+            f[m] = a;
+            cnt[m] = max(u - a, 0);
           }
-          f[m] = a;
-          b = c1;
-          while (a < b) {  // first cluster whose lower key exceeds hi
-            const int q = (a + b) >> 1;
-            if (krJ[q].x <= hi) a = q + 1;
-            else b = q;
-          }
-          cnt[m] = a - f[m];
         }
       }
     }
     int total;
-    const int off = wave_excl_scan(cnt[0] + cnt[1] + cnt[2], lane, total);
+    const int off = wave_excl_scan(cnt[0] + cnt[1] + cnt[2], total);
     for (int c0 = 0; c0 < total; c0 += kCandCap) {
       const int nc = min(total - c0, kCandCap);
       // this lane's candidates with list index in [c0, c0 + nc)
@@ -887,45 +947,40 @@ __global__ __launch_bounds__(256) void k_list(ListArgs L, const int* __restrict_
       __builtin_amdgcn_wave_barrier();
       // two candidates per lane and trip: their box loads are in flight together
       for (int u0 = 0; u0 < nc; u0 += 2 * WAVE) {
-        int cj[2] = {0, 0}, mx[2] = {0, 0}, my[2] = {0, 0}, mz[2] = {0, 0};
+        unsigned pk[2] = {0u, 0u};
         float4 jc[2], jh[2];
-  #pragma unroll
+#pragma unroll
         for (int h = 0; h < 2; h++) {
           const int u = u0 + h * WAVE + lane;
           jc[h] = jh[h] = make_float4(0.f, 0.f, 0.f, 0.f);
           if (u < nc) {
-            const unsigned pk = s_cand[wv][u];
-            const int im = (int)(pk >> 26);
-            cj[h] = (int)(pk & kEllCj);
-            mx[h] = im % 3 - 1;
-            my[h] = (im / 3) % 3 - 1;
-            mz[h] = im / 9 - 1;
-            jc[h] = bbJ[2 * cj[h]];
-            jh[h] = bbJ[2 * cj[h] + 1];
+            pk[h] = s_cand[wv][u];
+            const int cj = (int)(pk[h] & kEllCj);
+            jc[h] = bbJ[2 * cj];
+            jh[h] = bbJ[2 * cj + 1];
           }
         }
-  #pragma unroll
+#pragma unroll
         for (int h = 0; h < 2; h++) {
           const int u = u0 + h * WAVE + lane;
           bool pass = false;
           if (u < nc) {
-            const float Tx = mx[h] * SJ.af[0] + my[h] * SJ.af[3] + mz[h] * SJ.af[6];
-            const float Ty = mx[h] * SJ.af[1] + my[h] * SJ.af[4] + mz[h] * SJ.af[7];
-            const float Tz = mx[h] * SJ.af[2] + my[h] * SJ.af[5] + mz[h] * SJ.af[8];
-            const float gx = fmaxf(fabsf(jc[h].x + Tx - ic.x) - ih.x - jh[h].x, 0.f);
-            const float gy = fmaxf(fabsf(jc[h].y + Ty - ic.y) - ih.y - jh[h].y, 0.f);
-            const float gz = fmaxf(fabsf(jc[h].z + Tz - ic.z) - ih.z - jh[h].z, 0.f);
-            pass = gx * gx + gy * gy + gz * gz < L.rlist2;
+            const float4 T = s_img[wv][pk[h] >> 26];
+            const float gx = fmaxf(fabsf(jc[h].x + T.x - ic.x) - ih.x - jh[h].x, 0.f);
+            const float gy = fmaxf(fabsf(jc[h].y + T.y - ic.y) - ih.y - jh[h].y, 0.f);
+            const float gz = fmaxf(fabsf(jc[h].z + T.z - ic.z) - ih.z - jh[h].z, 0.f);
+            pass = fmaf(gz, gz, fmaf(gx, gx, gy * gy)) < L.rlist2;
           }
           const unsigned long long bal = __ballot(pass);
           if (pass) {
             const int k = n + __popcll(bal & ((1ull << lane) - 1));
             if (FILL) {
+              const int cj = (int)(pk[h] & kEllCj), im = (int)(pk[h] >> 26);
               if (base + k < L.ent_cap)
-                out[base + k] = make_entry(L.mode, ci, cj[h], mx[h], my[h], mz[h], SJ, orgJ, oi, L.pscale);
+                out[base + k] =
+                    make_entry(L.mode, ci, cj, im % 3 - 1, (im / 3) % 3 - 1, im / 9 - 1, SJ, orgJ, oi, L.pscale);
             } else if (k < kEll) {
-              ell[(size_t)ci * kEll + k] =
-                  (unsigned)cj[h] | ((unsigned)((mx[h] + 1) + 3 * (my[h] + 1) + 9 * (mz[h] + 1)) << 26);
+              ell[(size_t)ci * kEll + k] = pk[h];
             }
           }
           n += __popcll(bal);
@@ -955,7 +1010,7 @@ __global__ __launch_bounds__(256) void k_list_stream(ListArgs L, const int* __re
                                                      const int* __restrict__ start, Entry* __restrict__ out,
                                                      const unsigned* __restrict__ ell) {
   const int lane = threadIdx.x & 63;
-  const int ci = blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
+  const int ci = blockIdx.x * (blockDim.x / WAVE) + __builtin_amdgcn_readfirstlane((int)threadIdx.x / WAVE);
   const int nclI = L.nclI_dev ? *L.nclI_dev : L.nclI;
   if (ci >= nclI) return;
   // everything that depends on ci only, and the first two kept candidates of
@@ -1130,13 +1185,7 @@ template <int CTRL>
 __device__ __forceinline__ float dpp_f(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
 }
-template <int CTRL, int ROWS>
-__device__ __forceinline__ int dpp_i(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
-}
 constexpr int kRor1 = 0x121, kRor2 = 0x122, kRor4 = 0x124, kRor8 = 0x128;
-constexpr int kShr1 = 0x111, kShr2 = 0x112, kShr4 = 0x114, kShr8 = 0x118;
-constexpr int kBcast15 = 0x142, kBcast31 = 0x143;
 
 // v[l] + v[l ^ 16]: odd 16-lane rows of one copy swap with even rows of the other
 __device__ __forceinline__ float xor16_sum(float v) {
@@ -1196,19 +1245,6 @@ __device__ __forceinline__ float wave_sum_f(float v) {
   v += dpp_f<kRor1>(v);
   return xor32_sum(xor16_sum(v));
 }
-// exclusive prefix sum over the 64 lanes; *total = sum of all lanes (uniform)
-__device__ __forceinline__ int wave_excl_scan_dpp(int x, int& total) {
-  int v = x;
-  v += dpp_i<kShr1, 0xF>(v);
-  v += dpp_i<kShr2, 0xF>(v);
-  v += dpp_i<kShr4, 0xF>(v);
-  v += dpp_i<kShr8, 0xF>(v);
-  v += dpp_i<kBcast15, 0xA>(v);
-  v += dpp_i<kBcast31, 0xC>(v);
-  total = __builtin_amdgcn_readlane(v, 63);
-  return v - x;
-}
-
 // number of set bits of m in the lanes below this one (v_mbcnt)
 __device__ __forceinline__ int bits_below(unsigned long long m) {
   return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
@@ -1713,9 +1749,9 @@ __device__ __forceinline__ void stage_item(const PairArgs& A, const Entry& my, i
     n0 = (mp & md) ? CL : 0;
     const int cnt = __popc(m8);
     int tot1, tot2 = 0;
-    const int o1 = wave_excl_scan_dpp(count && !self ? cnt : 0, tot1);
+    const int o1 = wave_excl_scan(count && !self ? cnt : 0, tot1);
     int o2 = 0;
-    if constexpr (!VO) o2 = wave_excl_scan_dpp(count || self ? 0 : cnt, tot2);
+    if constexpr (!VO) o2 = wave_excl_scan(count || self ? 0 : cnt, tot2);
     n1 = (tot1 + CL - 1) & ~(CL - 1);
     n2 = (tot2 + CL - 1) & ~(CL - 1);
     b1 = n0;
@@ -2620,6 +2656,12 @@ inline void sys_cell(const double* box9, double rlist, SysArg& S) {
   double w[3];
   pbc_widths(box9, w);
   for (int k = 0; k < 3; k++) S.rb[k] = (float)(rlist / w[k]);
+  S.ortho = 1;
+  for (int k = 0; k < 9; k++)
+    if (k % 4 && box9[k] != 0.0) S.ortho = 0;
+  S.aa = (float)(box9[0] * box9[0]);
+  S.bb = (float)(box9[4] * box9[4]);
+  S.invc = (float)(1.0 / std::fabs(box9[8]));
 }
 
 // columns of a group of n atoms in a cell: side ~ cbrt(8/rho), bounded count
@@ -2636,6 +2678,8 @@ inline void sys_columns(const double* box9, int n, SysArg& S) {
     S.ncx = std::max(1, S.ncx / 2);
     S.ncy = std::max(1, S.ncy / 2);
   }
+  S.icx = 1.f / S.ncx;
+  S.icy = 1.f / S.ncy;
 }
 
 // How one side of the all-pairs pass goes over the chip: many atoms with at
