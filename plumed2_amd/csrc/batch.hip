@@ -99,35 +99,55 @@ static int batch_step(p2a_batch* b, const double* pos, double* values, double* d
   const int* ncl_dev = b->totals.p + 1;
   hipLaunchKernelGGL(k_fill_int3, dim3(std::max(1, std::min(grid1(nslot, 256), 4096))), dim3(256), 0, s,
                      b->col_count.p, ncol + 1, 0, b->fill.p, ncol + 1, 0, b->slot_loc.p, (int)nslot, -1);
-  hipLaunchKernelGGL(k_bin, dim3(grid1(N, 256)), dim3(256), 0, s, N, pos, 0, (const SysArg*)b->sys.p,
-                     (const int*)b->atom_sys.p, b->info.p, b->key.p, b->col_count.p);
+  Two<BinSide> B;
+  std::memset(&B, 0, sizeof(B));
+  B.n0 = grid1(N, 256);
+  B.s[0] = BinSide{N, 0, 0, nullptr, b->sys.p, b->info.p, b->key.p, b->col_count.p, b->col_start.p, b->fill.p, b->tmp.p};
+  hipLaunchKernelGGL(k_bin, dim3(B.n0), dim3(256), 0, s, B, pos, (const int*)b->atom_sys.p, (int*)nullptr,
+                     (int*)nullptr);
   // atom and cluster starts of the columns; totals[0], [1]
-  launch_list_scans(s, ncol, nullptr, b->col_count.p, CL, b->scan_bsum.p, b->col_start.p, b->col_cl.p, b->totals.p, 0,
-                    1);
-  hipLaunchKernelGGL(k_scatter, dim3(grid1(N, 256)), dim3(256), 0, s, N, b->info.p, b->col_start.p, b->fill.p,
-                     b->tmp.p);
-  hipLaunchKernelGGL(k_rank, dim3(ncol), dim3(256), 0, s, ncol, b->key.p, b->col_start.p, b->col_cl.p, b->tmp.p,
-                     b->slot_loc.p, b->info.p, pos, 0, (const SysArg*)b->sys.p, (const int*)b->atom_sys.p,
-                     b->origin.p, b->bb0.p, b->kr.p, b->cl_sys.p, b->cl_col.p, b->p.p, b->bb.p, pack_scale(b->sw));
-  ListArgs L;
+  const ScanSide cols{ncol, nullptr, b->col_count.p, b->col_start.p, b->col_cl.p, 0, 1, b->scan_bsum.p};
+  launch_list_scans(s, &cols, 1, CL, b->totals.p);
+  hipLaunchKernelGGL(k_scatter, dim3(B.n0), dim3(256), 0, s, B);
+  Two<RankSide> R;
+  std::memset(&R, 0, sizeof(R));
+  R.n0 = ncol;
+  R.s[0] = RankSide{ncol,         0,           b->key.p, b->col_start.p, b->col_cl.p, b->tmp.p, b->slot_loc.p,
+                    b->info.p,    b->sys.p,    b->origin.p, b->bb0.p, b->kr.p, b->cl_sys.p, b->cl_col.p, b->p.p,
+                    b->bb.p,      nullptr,     nullptr};
+  hipLaunchKernelGGL(k_rank, dim3(ncol), dim3(256), 0, s, R, pos, (const int*)b->atom_sys.p, pack_scale(b->sw));
+  Two<ListSide> T;
+  std::memset(&T, 0, sizeof(T));
+  ListSide& S = T.s[0];
+  ListArgs& L = S.L;
   L.nclI = clc;
   L.nclI_dev = ncl_dev;
   L.mode = 0;
   L.ent_cap = b->ent_cap;
   L.rlist2 = (float)(b->rlist * b->rlist);
   L.pscale = pack_scale(b->sw);
+  S.cl_colI = b->cl_col.p;
+  S.cl_sysI = b->cl_sys.p;
+  S.sysI = S.sysJ = b->sys.p;
+  S.bbI = S.bbJ = b->bb0.p;
+  S.krI = S.krJ = b->kr.p;
+  S.col_clJ = b->col_cl.p;
+  S.orgI = S.orgJ = b->origin.p;
+  S.count = b->ecount.p;
+  S.start = b->estart.p;
+  S.out = b->ents.p;
+  S.ell = b->ell.p;
   const int wpb = 256 / WAVE;
-  hipLaunchKernelGGL(k_list<0>, dim3(grid1(clc, wpb)), dim3(256), 0, s, L, b->cl_col.p, (const int*)b->cl_sys.p,
-                     (const SysArg*)b->sys.p, (const SysArg*)b->sys.p, b->bb0.p, b->bb0.p, b->kr.p, b->kr.p,
-                     b->col_cl.p, b->origin.p, b->origin.p, b->ecount.p, (const int*)nullptr, (Entry*)nullptr, b->ell.p);
-  launch_list_scans(s, clc, ncl_dev, b->ecount.p, chunk, b->scan_bsum.p, b->estart.p, b->istart.p, b->totals.p, 2, 3);
+  T.n0 = grid1(clc, wpb);
+  hipLaunchKernelGGL(k_list<0>, dim3(T.n0), dim3(256), 0, s, T);
+  const ScanSide lists{clc, ncl_dev, b->ecount.p, b->estart.p, b->istart.p, 2, 3, b->scan_bsum.p};
+  launch_list_scans(s, &lists, 1, chunk, b->totals.p);
   hipLaunchKernelGGL(k_list_stream, dim3(grid1(clc, wpb)), dim3(256), 0, s, L, (const int*)b->cl_sys.p,
                      (const SysArg*)b->sys.p, b->origin.p, b->origin.p, b->ecount.p, (const int*)b->estart.p, b->ents.p,
                      b->ell.p);
   // k_list<2>: 64 clusters per wave
-  hipLaunchKernelGGL(k_list<2>, dim3(grid1(clc, wpb * WAVE)), dim3(256), 0, s, L, b->cl_col.p, (const int*)b->cl_sys.p,
-                     (const SysArg*)b->sys.p, (const SysArg*)b->sys.p, b->bb0.p, b->bb0.p, b->kr.p, b->kr.p,
-                     b->col_cl.p, b->origin.p, b->origin.p, b->ecount.p, (const int*)b->estart.p, b->ents.p, b->ell.p);
+  T.n0 = grid1(clc, wpb * WAVE);
+  hipLaunchKernelGGL(k_list<2>, dim3(T.n0), dim3(256), 0, s, T);
   hipLaunchKernelGGL(k_items, dim3(grid1(clc, 256)), dim3(256), 0, s, clc, ncl_dev, b->ecount.p, b->estart.p,
                      b->istart.p, b->items.p, chunk, b->items_cap);
   // k_rank has packed the positions of this step (the list is built at every step)
@@ -159,8 +179,11 @@ static int batch_step(p2a_batch* b, const double* pos, double* values, double* d
   launch_pairs<false>(A, grid, s, false, chunk, b->items.p, b->ents.p, b->p.p, b->p.p, b->bb.p, b->bb.p,
                       (const int*)nullptr, b->fpart.p, b->partial.p);
   if ((rc = launch_check("batch: pair kernel"))) return rc;
-  hipLaunchKernelGGL(k_gather_reduce, dim3(grid1(nslot * 3, 256)), dim3(256), 0, s, grid1(nslot * 3, 256), clc,
-                     ncl_dev, b->p.p, b->istart.p, b->items_cap, b->fpart.p, deriv, 0, RedArgs{});
+  Two<GatherSide> Gt;
+  std::memset(&Gt, 0, sizeof(Gt));
+  Gt.n0 = grid1(nslot * 3, 256);
+  Gt.s[0] = GatherSide{clc, ncl_dev, b->p.p, b->istart.p, b->items_cap, b->fpart.p};
+  hipLaunchKernelGGL(k_gather_reduce, dim3(Gt.n0), dim3(256), 0, s, Gt, deriv, 0, RedArgs{});
   hipLaunchKernelGGL(k_sys_reduce, dim3(b->nsys), dim3(256), 0, s, b->nsys, b->sys_colbase.p, b->col_cl.p,
                      b->istart.p, b->items_cap, b->partial.p, values, virials, b->npairs.p);
   return launch_check("batch: reductions");

@@ -45,6 +45,8 @@ struct Group {
   // atoms of the next one; 0 = no such order
   int order_nslot = 0;
   const int* order_ptr = nullptr;
+  // col_count and fill hold zeros (k_rank leaves them so), at these addresses
+  const int *zero_count = nullptr, *zero_fill = nullptr;
   DBuf<SysArg> sys;
   DBuf<int4> info;
   DBuf<double> key;
@@ -153,6 +155,12 @@ static int choose_path_uncached(p2a_coord* c, const double* box9) {
   return 0;
 }
 
+// workgroups of the pair kernel over nitems items
+static int pair_grid(const p2a_coord* c, int nitems) {
+  const int grid = grid1(nitems, PAIR_BLOCK / WAVE);
+  return c->tune.blocks_per_cu > 0 ? std::min(grid, c->tune.blocks_per_cu * c->cu_count) : grid;
+}
+
 static int rebuild(p2a_coord* c, const double* box9, const double* pos_dev) {
   const p2a_switch& sw = c->spec.sw;
   // list radius: NL_CUTOFF when a neighbour list is requested (its candidates
@@ -197,6 +205,18 @@ static int rebuild(p2a_coord* c, const double* box9, const double* pos_dev) {
   }
   // two alternating slots for the largest wrap of this rebuild
   const int wslot = 12 + (int)(c->rebuilds & 1);
+  Two<BinSide> B;
+  Two<RankSide> R;
+  ScanSide cols[2];
+  std::memset(&B, 0, sizeof(B));
+  std::memset(&R, 0, sizeof(R));
+  int nbin[2] = {0, 0}, nrank[2] = {0, 0};
+  size_t nbsum = 0;  // block sums of the scans: columns first, then the lists
+  for (int gi = 0; gi < ngroups; gi++)
+    nbsum += 2 * (size_t)grid1(std::max(c->g[gi].ncol, c->g[gi].maxcl), kScanBlock) + 2;
+  if ((rc = c->scan_bsum.reserve(nbsum))) return rc;
+  int* bsum[2] = {c->scan_bsum.p,
+                  c->scan_bsum.p + 2 * (size_t)grid1(std::max(c->g[0].ncol, c->g[0].maxcl), kScanBlock) + 2};
   for (int gi = 0; gi < ngroups; gi++) {
     Group& G = c->g[gi];
     // the atoms are binned in the slot order of the last build when it is
@@ -205,29 +225,39 @@ static int rebuild(p2a_coord* c, const double* box9, const double* pos_dev) {
     // clusters, padding included
     const bool use_order = G.order_nslot > 0 && G.order_ptr == G.slot_loc.p;
     const int norder = use_order ? G.order_nslot : 0;
-    const int* order = use_order ? G.slot_loc.p : nullptr;
-    const int nthr = use_order ? norder : G.n;
     G.order_nslot = 0;
-    hipLaunchKernelGGL(k_fill_int3, dim3(std::max(1, std::min(grid1(G.slot_loc.n, 256), 1024))), dim3(256), 0, s,
-                       G.col_count.p, G.ncol + 1, 0, G.fill.p, G.ncol + 1, 0, G.slot_loc.p,
-                       use_order ? 0 : (int)G.slot_loc.n, -1);
-    if (G.n > 0)
-      hipLaunchKernelGGL(k_bin, dim3(grid1(nthr, 256)), dim3(256), 0, s, G.n, pos_dev, G.off, (const SysArg*)G.sys.p,
-                         (const int*)nullptr, G.info.p, G.key.p, G.col_count.p, c->totals.p + wslot,
-                         c->totals.p + (25 - wslot), order, norder);
-    // atom and cluster starts of the columns; totals[4 + 2 gi], [5 + 2 gi]
-    if ((rc = c->scan_bsum.reserve(2 * (size_t)grid1(std::max(G.ncol, 1), kScanBlock) + 2))) return rc;
-    launch_list_scans(s, G.ncol, nullptr, G.col_count.p, CL, c->scan_bsum.p, G.col_start.p, G.col_cl.p, c->totals.p,
-                      4 + 2 * gi, 5 + 2 * gi);
-    if (G.n > 0) {
-      hipLaunchKernelGGL(k_scatter, dim3(grid1(nthr, 256)), dim3(256), 0, s, G.n, G.info.p, G.col_start.p, G.fill.p,
-                         G.tmp.p, order, norder);
-      hipLaunchKernelGGL(k_rank, dim3(G.ncol), dim3(256), 0, s, G.ncol, G.key.p, G.col_start.p, G.col_cl.p,
-                         G.tmp.p, G.slot_loc.p, G.info.p, pos_dev, G.off, (const SysArg*)G.sys.p,
-                         (const int*)nullptr, G.origin.p, G.bb0.p, G.kr.p, (int*)nullptr, G.cl_col.p, G.p.p, G.bb.p,
-                         pack_scale(c->spec.sw));
+    if (G.zero_count != G.col_count.p || G.zero_fill != G.fill.p) {
+      const int nc = (int)G.col_count.n, nf = (int)G.fill.n;
+      hipLaunchKernelGGL(k_fill_int3, dim3(std::max(1, std::min(grid1(std::max(nc, nf), 256), 1024))), dim3(256), 0, s,
+                         G.col_count.p, nc, 0, G.fill.p, nf, 0, (int*)nullptr, 0, 0);
     }
-    if ((rc = launch_check("rebuild: binning"))) return rc;
+    G.zero_count = G.zero_fill = nullptr;
+    B.s[gi] = BinSide{G.n,     G.off,         norder,          use_order ? G.slot_loc.p : nullptr,
+                      G.sys.p, G.info.p,      G.key.p,         G.col_count.p,
+                      G.col_start.p, G.fill.p, G.tmp.p};
+    nbin[gi] = G.n > 0 ? grid1(use_order ? norder : G.n, 256) : 0;
+    // atom and cluster starts of the columns; totals[4 + 2 gi], [5 + 2 gi]
+    cols[gi] = ScanSide{G.ncol, nullptr, G.col_count.p, G.col_start.p, G.col_cl.p, 4 + 2 * gi, 5 + 2 * gi, bsum[gi]};
+    R.s[gi] = RankSide{G.ncol,   G.off,   G.key.p, G.col_start.p, G.col_cl.p,       G.tmp.p,    G.slot_loc.p,
+                       G.info.p, G.sys.p, G.origin.p, G.bb0.p,    G.kr.p,           nullptr,    G.cl_col.p,
+                       G.p.p,    G.bb.p,  G.col_count.p, G.fill.p};
+    nrank[gi] = G.n > 0 ? G.ncol : 0;
+  }
+  B.n0 = nbin[0];
+  R.n0 = nrank[0];
+  if (nbin[0] + nbin[1] > 0)
+    hipLaunchKernelGGL(k_bin, dim3(nbin[0] + nbin[1]), dim3(256), 0, s, B, pos_dev, (const int*)nullptr,
+                       c->totals.p + wslot, c->totals.p + (25 - wslot));
+  launch_list_scans(s, cols, ngroups, CL, c->totals.p);
+  if (nbin[0] + nbin[1] > 0) {
+    hipLaunchKernelGGL(k_scatter, dim3(nbin[0] + nbin[1]), dim3(256), 0, s, B);
+    hipLaunchKernelGGL(k_rank, dim3(nrank[0] + nrank[1]), dim3(256), 0, s, R, pos_dev, (const int*)nullptr,
+                       pack_scale(c->spec.sw));
+  }
+  if ((rc = launch_check("rebuild: binning"))) return rc;
+  for (int gi = 0; gi < ngroups; gi++) {
+    c->g[gi].zero_count = c->g[gi].col_count.p;
+    c->g[gi].zero_fill = c->g[gi].fill.p;
   }
   // cluster counts stay on the device (totals[5 + 2 g]) until the one host
   // read below; the kernels in between are sized by the cluster capacity
@@ -237,31 +267,46 @@ static int rebuild(p2a_coord* c, const double* box9, const double* pos_dev) {
   int64_t tot_entries = 0;
   const int wpb = 256 / WAVE;
   const int chunk = c->tune.chunk;
-  ListArgs Ls[2];
+  Two<ListSide> T;
+  ScanSide lists[2];
+  std::memset(&T, 0, sizeof(T));
+  int nlist[2] = {0, 0};
   for (int d = 0; d < c->ndir; d++) {
     Dir& D = c->dir[d];
     D.I = (ngroups == 2) ? d : 0;
     D.J = (ngroups == 2) ? 1 - d : 0;
     Group& GI = c->g[D.I];
     Group& GJ = c->g[D.J];
-    ListArgs& L = Ls[d];
+    ListSide& S = T.s[d];
     const int* ncl_dev = c->totals.p + 5 + 2 * D.I;
-    L.nclI = GI.maxcl;
-    L.nclI_dev = ncl_dev;
-    L.mode = (ngroups == 1) ? 0 : (d == 0 ? 1 : 2);
-    L.ent_cap = 0;
-    L.rlist2 = (float)(c->rlist * c->rlist);
-    L.pscale = pack_scale(c->spec.sw);
     if ((rc = D.ecount.reserve(GI.maxcl + 1)) || (rc = D.estart.reserve(GI.maxcl + 1)) ||
-        (rc = D.istart.reserve(GI.maxcl + 1)) || (rc = c->scan_bsum.reserve(2 * (size_t)grid1(GI.maxcl, kScanBlock) + 2)) ||
-        (rc = D.ell.reserve((size_t)GI.maxcl * kEll)))
+        (rc = D.istart.reserve(GI.maxcl + 1)) || (rc = D.ell.reserve((size_t)GI.maxcl * kEll)))
       return rc;
-    hipLaunchKernelGGL(k_list<0>, dim3(grid1(GI.maxcl, wpb)), dim3(256), 0, s, L, GI.cl_col.p, (const int*)nullptr,
-                       (const SysArg*)GI.sys.p, (const SysArg*)GJ.sys.p, GI.bb0.p, GJ.bb0.p, GI.kr.p, GJ.kr.p,
-                       GJ.col_cl.p, GI.origin.p, GJ.origin.p, D.ecount.p, (const int*)nullptr, (Entry*)nullptr, D.ell.p);
-    launch_list_scans(s, GI.maxcl, ncl_dev, D.ecount.p, chunk, c->scan_bsum.p, D.estart.p, D.istart.p, c->totals.p,
-                      8 + 2 * d, 9 + 2 * d);
+    S.L.nclI = GI.maxcl;
+    S.L.nclI_dev = ncl_dev;
+    S.L.mode = (ngroups == 1) ? 0 : (d == 0 ? 1 : 2);
+    S.L.ent_cap = 0;
+    S.L.rlist2 = (float)(c->rlist * c->rlist);
+    S.L.pscale = pack_scale(c->spec.sw);
+    S.cl_colI = GI.cl_col.p;
+    S.sysI = GI.sys.p;
+    S.sysJ = GJ.sys.p;
+    S.bbI = GI.bb0.p;
+    S.bbJ = GJ.bb0.p;
+    S.krI = GI.kr.p;
+    S.krJ = GJ.kr.p;
+    S.col_clJ = GJ.col_cl.p;
+    S.orgI = GI.origin.p;
+    S.orgJ = GJ.origin.p;
+    S.count = D.ecount.p;
+    S.start = D.estart.p;
+    S.ell = D.ell.p;
+    nlist[d] = grid1(GI.maxcl, wpb);
+    lists[d] = ScanSide{GI.maxcl, ncl_dev, D.ecount.p, D.estart.p, D.istart.p, 8 + 2 * d, 9 + 2 * d, bsum[D.I]};
   }
+  T.n0 = nlist[0];
+  hipLaunchKernelGGL(k_list<0>, dim3(nlist[0] + nlist[1]), dim3(256), 0, s, T);
+  launch_list_scans(s, lists, c->ndir, chunk, c->totals.p);
   if ((rc = launch_check("rebuild: list count"))) return rc;
   int* hostT = c->host_ro;
   P2A_HIP(hipMemcpyAsync(hostT, c->totals.p, 16 * sizeof(int), hipMemcpyDeviceToHost, s));
@@ -277,25 +322,31 @@ static int rebuild(p2a_coord* c, const double* box9, const double* pos_dev) {
   for (int d = 0; d < c->ndir; d++) {
     Dir& D = c->dir[d];
     Group& GI = c->g[D.I];
-    Group& GJ = c->g[D.J];
     D.nentries = hostT[8 + 2 * d];
     D.nitems = hostT[9 + 2 * d];
     D.item_offset = c->nitems;
     c->nitems += D.nitems;
     tot_entries += D.nentries;
+    // the schedule of a persistent grid comes with the items
+    const int nw = c->tune.blocks_per_cu > 0 ? pair_grid(c, D.nitems) * (PAIR_BLOCK / WAVE) : 0;
     if ((rc = D.ents.reserve(std::max<int64_t>(D.nentries, 1))) || (rc = D.items.reserve(std::max(D.nitems, 1))) ||
-        (rc = D.fpart.reserve((size_t)CL * 3 * std::max(D.nitems, 1))))
+        (rc = D.fpart.reserve((size_t)CL * 3 * std::max(D.nitems, 1))) || (rc = D.wave_start.reserve((size_t)nw + 1)))
       return rc;
-    Ls[d].ent_cap = (int)D.ents.n;
-    if (GI.ncl > 0) {
-      hipLaunchKernelGGL(k_list<1>, dim3(grid1(GI.ncl, wpb)), dim3(256), 0, s, Ls[d], GI.cl_col.p,
-                         (const int*)nullptr, (const SysArg*)GI.sys.p, (const SysArg*)GJ.sys.p, GI.bb0.p, GJ.bb0.p,
-                         GI.kr.p, GJ.kr.p, GJ.col_cl.p, GI.origin.p, GJ.origin.p, D.ecount.p,
-                         (const int*)D.estart.p, D.ents.p, D.ell.p);
-      hipLaunchKernelGGL(k_items, dim3(grid1(GI.ncl, 256)), dim3(256), 0, s, GI.ncl, (const int*)nullptr,
-                         D.ecount.p, D.estart.p, D.istart.p, D.items.p, chunk, (int)D.items.n);
+    ListSide& S = T.s[d];
+    S.L.ent_cap = (int)D.ents.n;
+    S.L.nclI = GI.ncl;
+    S.L.nclI_dev = nullptr;
+    S.out = D.ents.p;
+    S.M = ItemArgs{D.items.p, D.istart.p, chunk, (int)D.items.n, nw, D.nitems,
+                   (long long)D.nentries + (long long)kItemCost * D.nitems, D.wave_start.p};
+    nlist[d] = D.nitems > 0 ? grid1(GI.ncl, wpb) : 0;
+    if (nw && D.nitems > 0) {
+      D.sched_waves = nw;
+      D.sched_gen = c->rebuilds + 1;
     }
   }
+  T.n0 = nlist[0];
+  if (nlist[0] + nlist[1] > 0) hipLaunchKernelGGL(k_list<1>, dim3(nlist[0] + nlist[1]), dim3(256), 0, s, T);
   c->nentries = tot_entries;
   if (share) {
     for (int gi = 0; gi < 2; gi++) {
@@ -395,27 +446,22 @@ static int reimage(p2a_coord* c, const double* box9) {
 }
 
 // value / virial / pair count from nred rows of c->partial, in one workgroup
-// and a fixed order; with gather_dir >= 0 the same launch also forms that
-// direction's derivatives
+// and a fixed order; the same launch also forms the derivatives of the first
+// ngather directions
 static int reduce_partials(p2a_coord* c, int nred, double* value_dev, double* virial_dev,
-                           int gather_dir = -1, double* deriv_dev = nullptr, bool with_stats = true,
+                           int ngather = 0, double* deriv_dev = nullptr, bool with_stats = true,
                            const int* skip = nullptr) {
   hipStream_t s = c->stream;
-  int ngather = 0, ncl = 0;
-  const float4* gp = nullptr;
-  const int* istart = nullptr;
-  int items_cap = 0;
-  const double* fpart = nullptr;
-  if (gather_dir >= 0) {
-    Dir& D = c->dir[gather_dir];
+  Two<GatherSide> T;
+  std::memset(&T, 0, sizeof(T));
+  int nb[2] = {0, 0};
+  for (int d = 0; d < ngather; d++) {
+    Dir& D = c->dir[d];
     Group& GI = c->g[D.I];
-    ncl = GI.ncl;
-    ngather = grid1((size_t)ncl * CL * 3, 256);
-    gp = GI.p.p;
-    istart = D.istart.p;
-    items_cap = (int)D.items.n;
-    fpart = D.fpart.p;
+    nb[d] = grid1((size_t)GI.ncl * CL * 3, 256);
+    T.s[d] = GatherSide{GI.ncl, nullptr, GI.p.p, D.istart.p, (int)D.items.n, D.fpart.p};
   }
+  T.n0 = nb[0];
   RedArgs R;
   std::memset(&R, 0, sizeof(R));
   R.nred = nred;
@@ -424,8 +470,7 @@ static int reduce_partials(p2a_coord* c, int nred, double* value_dev, double* vi
   R.virial = virial_dev;
   R.stats = with_stats ? c->stats.p : nullptr;
   R.skip = skip;
-  hipLaunchKernelGGL(k_gather_reduce, dim3(ngather + 1), dim3(256), 0, s, ngather, ncl, (const int*)nullptr, gp,
-                     istart, items_cap, fpart, deriv_dev, 1, R);
+  hipLaunchKernelGGL(k_gather_reduce, dim3(nb[0] + nb[1] + 1), dim3(256), 0, s, T, deriv_dev, 1, R);
   return P2A_OK;
 }
 
@@ -436,13 +481,17 @@ static void pack_positions(p2a_coord* c, const double* pos_dev) {
   c->packed_pos = nullptr;
   if (ahead) return;
   const int ngroups = c->spec.nb > 0 ? 2 : 1;
+  Two<PackSide> T;
+  std::memset(&T, 0, sizeof(T));
+  int nb[2] = {0, 0};
   for (int gi = 0; gi < ngroups; gi++) {
     Group& G = c->g[gi];
-    if (G.ncl == 0) continue;
-    hipLaunchKernelGGL(k_pack_bbox, dim3(grid1((size_t)G.ncl * CL, 256)), dim3(256), 0, c->stream, G.ncl * CL,
-                       (const int*)nullptr, G.slot_loc.p, G.info.p, pos_dev, G.off, (const SysArg*)G.sys.p,
-                       (const int*)nullptr, G.origin.p, G.p.p, G.bb.p, pack_scale(c->spec.sw));
+    T.s[gi] = PackSide{G.ncl * CL, G.slot_loc.p, G.info.p, G.off, G.sys.p, G.origin.p, G.p.p, G.bb.p};
+    nb[gi] = G.ncl > 0 ? grid1((size_t)G.ncl * CL, 256) : 0;
   }
+  T.n0 = nb[0];
+  if (nb[0] + nb[1] > 0)
+    hipLaunchKernelGGL(k_pack_bbox, dim3(nb[0] + nb[1]), dim3(256), 0, c->stream, T, pos_dev, pack_scale(c->spec.sw));
 }
 
 // skip: a device flag; when it reads nonzero at run time the pair and
@@ -470,10 +519,8 @@ static int run_pairs(p2a_coord* c, const double* box9, const double* pos_dev, do
   for (int d = 0; d < ndir_run; d++) {
     Dir& D = c->dir[d];
     if (D.nitems == 0) continue;
-    int grid = grid1(D.nitems, PAIR_BLOCK / WAVE);
-    if (c->tune.blocks_per_cu > 0) grid = std::min(grid, c->tune.blocks_per_cu * c->cu_count);
-    grids[d] = grid;
-    nred += grid;
+    grids[d] = pair_grid(c, D.nitems);
+    nred += grids[d];
   }
   if ((rc = c->partial.reserve(8 * (size_t)std::max(nred, 1)))) return rc;
   hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -523,20 +570,8 @@ static int run_pairs(p2a_coord* c, const double* box9, const double* pos_dev, do
     c->pending.emplace_back(e0, e1);
   }
   if ((rc = launch_check("pair kernel"))) return rc;
-  // derivatives of the last direction go with the reduction
-  const int last = value_only ? -1 : c->ndir - 1;
-  for (int d = 0; d < last; d++) {
-    Dir& D = c->dir[d];
-    Group& GI = c->g[D.I];
-    if (GI.ncl == 0) continue;
-    const int ng = grid1((size_t)GI.ncl * CL * 3, 256);
-    RedArgs R;
-    std::memset(&R, 0, sizeof(R));
-    R.skip = skip;
-    hipLaunchKernelGGL(k_gather_reduce, dim3(ng), dim3(256), 0, s, ng, GI.ncl, (const int*)nullptr, GI.p.p,
-                       D.istart.p, (int)D.items.n, D.fpart.p, deriv_dev, 0, R);
-  }
-  if ((rc = reduce_partials(c, nred, value_dev, virial_dev, last, deriv_dev, true, skip))) return rc;
+  // the derivatives go with the reduction
+  if ((rc = reduce_partials(c, nred, value_dev, virial_dev, value_only ? 0 : c->ndir, deriv_dev, true, skip))) return rc;
   return launch_check("finalize");
 }
 
@@ -745,19 +780,8 @@ static int run_rows(p2a_coord* c, const double* box9, const double* pos_dev, dou
   }
   if (!weighted) return launch_check("rows");
   if ((rc = c->out_buf.reserve(16))) return rc;
-  const int last = c->ndir - 1;
-  for (int d = 0; d < last; d++) {
-    Dir& D = c->dir[d];
-    Group& GI = c->g[D.I];
-    if (GI.ncl == 0) continue;
-    const int ng = grid1((size_t)GI.ncl * CL * 3, 256);
-    RedArgs R;
-    std::memset(&R, 0, sizeof(R));
-    hipLaunchKernelGGL(k_gather_reduce, dim3(ng), dim3(256), 0, s, ng, GI.ncl, (const int*)nullptr, GI.p.p,
-                       D.istart.p, (int)D.items.n, D.fpart.p, vjp_dev, 0, R);
-  }
   double* wdev = virial_dev ? virial_dev : c->out_buf.p + 1;
-  if ((rc = reduce_partials(c, nred, c->out_buf.p, wdev, last, vjp_dev, false))) return rc;
+  if ((rc = reduce_partials(c, nred, c->out_buf.p, wdev, c->ndir, vjp_dev, false))) return rc;
   return launch_check("row derivatives");
 }
 

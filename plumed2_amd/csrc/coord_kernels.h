@@ -191,6 +191,19 @@ __device__ __forceinline__ void block_excl_scan2(int& a, int& c, int& ta, int& t
   __syncthreads();
 }
 
+// The arguments of one launch over the two groups (or the two directions) of a
+// list build; workgroups 0 .. n0-1 are the first one's, the others the second's.
+// At the sizes of small groups a build is a row of launches of 2-7 us each, and
+// the two halves of one launch run side by side (2,000 atoms in two groups, list built
+// in the call: 135 us a call, 73 so and with k_items and the schedule in the fill).
+template <class T>
+struct Two {
+  T s[2];
+  int n0;
+  __device__ __forceinline__ int side() const { return (int)blockIdx.x >= n0 ? 1 : 0; }
+  __device__ __forceinline__ int block(int d) const { return (int)blockIdx.x - (d ? n0 : 0); }
+};
+
 __device__ __forceinline__ int nsys_of(const int* idx, int i) { return idx ? idx[i] : 0; }
 
 // Workgroups are dispatched to the 8 XCDs of the chip in turn (workgroup b to
@@ -240,15 +253,25 @@ __device__ __forceinline__ void block_col_range(int col, int* sh, int& lo, int& 
 // order (optional): the atoms in the slot order of the previous build (norder
 // slots, -1 = padding), so that a workgroup's atoms share few columns and its
 // counts stay in LDS; otherwise thread i takes atom i.
-__global__ __launch_bounds__(256) void k_bin(int n, const double* __restrict__ pos, int off,
-                                             const SysArg* __restrict__ sys, const int* __restrict__ atom_sys,
-                                             int4* __restrict__ info, double* __restrict__ key,
-                                             int* __restrict__ col_count, int* __restrict__ mmax = nullptr,
-                                             int* __restrict__ mclear = nullptr, const int* __restrict__ order = nullptr,
-                                             int norder = 0) {
+struct BinSide {
+  int n, off;
+  int norder;
+  const int* order;
+  const SysArg* sys;
+  int4* info;
+  double* key;
+  int* col_count;
+  const int* col_start;
+  int *fill, *tmp;
+};
+__device__ __forceinline__ void bin_atoms(int blk, int n, const double* __restrict__ pos, int off,
+                                          const SysArg* __restrict__ sys, const int* __restrict__ atom_sys,
+                                          int4* __restrict__ info, double* __restrict__ key,
+                                          int* __restrict__ col_count, int* __restrict__ mmax,
+                                          int* __restrict__ mclear, const int* __restrict__ order, int norder) {
   __shared__ int sh[512];
   __shared__ int hist[kBinLds];
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  const int s = blk * blockDim.x + threadIdx.x;
   const int i = order ? (s < norder ? order[s] : -1) : (s < n ? s : -1);
   int col = -1;
   int am = 0;
@@ -292,6 +315,12 @@ __global__ __launch_bounds__(256) void k_bin(int n, const double* __restrict__ p
   for (int j = threadIdx.x; j < range; j += blockDim.x)
     if (hist[j]) atomicAdd(&col_count[lo + j], hist[j]);
 }
+__global__ __launch_bounds__(256) void k_bin(Two<BinSide> T, const double* pos, const int* atom_sys, int* mmax,
+                                             int* mclear) {
+  const int d = T.side();
+  const BinSide& B = T.s[d];
+  bin_atoms(T.block(d), B.n, pos, B.off, B.sys, atom_sys, B.info, B.key, B.col_count, mmax, mclear, B.order, B.norder);
+}
 
 // Two exclusive scans of one count array in one pass over it (out0 of in[i],
 // out1 of ceil(in[i]/chunk)), across many workgroups: per-block sums, a
@@ -304,11 +333,21 @@ constexpr int kScanBlock = 1024;  // elements per workgroup (256 threads x 4)
 // most 8 counts per thread), for counts that one workgroup scans faster than
 // three launches
 constexpr int kScanOneMax = 8192;
-__global__ __launch_bounds__(1024) void k_scan2_one(int n, const int* __restrict__ n_dev, const int* __restrict__ in,
-                                                    int chunk, int* __restrict__ out0, int* __restrict__ out1,
-                                                    int* __restrict__ totals, int slot0, int slot1) {
+struct ScanSide {
+  int n;
+  const int* n_dev;
+  const int* in;
+  int *out0, *out1;
+  int slot0, slot1;
+  int* bsum;
+};
+__global__ __launch_bounds__(1024) void k_scan2_one(Two<ScanSide> A, int chunk, int* __restrict__ totals) {
   __shared__ int sw[32];
-  if (n_dev) n = *n_dev;
+  const ScanSide& S = A.s[blockIdx.x];
+  const int* __restrict__ in = S.in;
+  int* __restrict__ out0 = S.out0;
+  int* __restrict__ out1 = S.out1;
+  const int n = S.n_dev ? *S.n_dev : S.n;
   const int t = threadIdx.x, T = blockDim.x;
   const int per = (n + T - 1) / T;  // <= 8: n <= kScanOneMax
   const int b = min(n, t * per), e = min(n, b + per);
@@ -335,16 +374,18 @@ __global__ __launch_bounds__(1024) void k_scan2_one(int n, const int* __restrict
   if (t == 0) {
     out0[n] = ta;
     out1[n] = tc;
-    totals[slot0] = ta;
-    totals[slot1] = tc;
+    totals[S.slot0] = ta;
+    totals[S.slot1] = tc;
   }
 }
 
-__global__ __launch_bounds__(256) void k_scan2_sums(int n, const int* __restrict__ n_dev, const int* __restrict__ in,
-                                                    int chunk, int* __restrict__ bsum) {
+__global__ __launch_bounds__(256) void k_scan2_sums(Two<ScanSide> A, int chunk) {
   __shared__ int sw[32];
-  if (n_dev) n = *n_dev;
-  const int base = blockIdx.x * kScanBlock + threadIdx.x * 4;
+  const int d = A.side(), blk = A.block(d);
+  const ScanSide& S = A.s[d];
+  const int* __restrict__ in = S.in;
+  const int n = S.n_dev ? *S.n_dev : S.n;
+  const int base = blk * kScanBlock + threadIdx.x * 4;
   int a = 0, c = 0;
   for (int k = 0; k < 4; k++) {
     const int i = base + k;
@@ -356,58 +397,30 @@ __global__ __launch_bounds__(256) void k_scan2_sums(int n, const int* __restrict
   int ta, tc;
   block_excl_scan2(a, c, ta, tc, sw);
   if (threadIdx.x == 0) {
-    bsum[2 * blockIdx.x] = ta;
-    bsum[2 * blockIdx.x + 1] = tc;
+    S.bsum[2 * blk] = ta;
+    S.bsum[2 * blk + 1] = tc;
   }
 }
 
-__global__ __launch_bounds__(1024) void k_scan2_blocks(int nb, int n, const int* __restrict__ n_dev,
-                                                       int* __restrict__ bsum, int* __restrict__ out0,
-                                                       int* __restrict__ out1, int* __restrict__ totals, int slot0,
-                                                       int slot1) {
-  __shared__ int sa[1024], sc[1024];
-  if (n_dev) n = *n_dev;
-  const int t = threadIdx.x, T = blockDim.x;
-  const int per = (nb + T - 1) / T;
-  const int b = t * per, e = min(nb, b + per);
-  int la = 0, lc = 0;
-  for (int i = b; i < e; i++) {
-    la += bsum[2 * i];
-    lc += bsum[2 * i + 1];
-  }
-  sa[t] = la;
-  sc[t] = lc;
-  __syncthreads();
-  for (int o = 1; o < T; o <<= 1) {
-    const int va = (t >= o) ? sa[t - o] : 0, vc = (t >= o) ? sc[t - o] : 0;
-    __syncthreads();
-    sa[t] += va;
-    sc[t] += vc;
-    __syncthreads();
-  }
-  int ra = sa[t] - la, rc = sc[t] - lc;
-  for (int i = b; i < e; i++) {
-    const int xa = bsum[2 * i], xc = bsum[2 * i + 1];
-    bsum[2 * i] = ra;
-    bsum[2 * i + 1] = rc;
-    ra += xa;
-    rc += xc;
-  }
-  if (t == T - 1) {
-    out0[n] = sa[t];
-    out1[n] = sc[t];
-    totals[slot0] = sa[t];
-    totals[slot1] = sc[t];
-  }
-}
-
-__global__ __launch_bounds__(256) void k_scan2_apply(int n, const int* __restrict__ n_dev, const int* __restrict__ in,
-                                                     int chunk, const int* __restrict__ bsum, int* __restrict__ out0,
-                                                     int* __restrict__ out1) {
+// every workgroup adds up the block sums before its own (a scan of them in a
+// launch between took 5 us)
+__global__ __launch_bounds__(256) void k_scan2_apply(Two<ScanSide> A, int chunk, int* __restrict__ totals) {
   __shared__ int sw[32];
-  if (n_dev) n = *n_dev;
-  if (blockIdx.x * kScanBlock >= n) return;  // uniform per workgroup
-  const int base = blockIdx.x * kScanBlock + threadIdx.x * 4;
+  const int d = A.side(), blk = A.block(d);
+  const ScanSide& S = A.s[d];
+  const int* __restrict__ in = S.in;
+  const int* __restrict__ bsum = S.bsum;
+  int* __restrict__ out0 = S.out0;
+  int* __restrict__ out1 = S.out1;
+  const int n = S.n_dev ? *S.n_dev : S.n;
+  if (blk > 0 && blk * kScanBlock >= n) return;  // uniform per workgroup
+  int pa = 0, pc = 0, ba, bc;
+  for (int i = threadIdx.x; i < blk; i += 256) {
+    pa += bsum[2 * i];
+    pc += bsum[2 * i + 1];
+  }
+  block_excl_scan2(pa, pc, ba, bc, sw);
+  const int base = blk * kScanBlock + threadIdx.x * 4;
   int va[4], vc[4], a = 0, c = 0;
   for (int k = 0; k < 4; k++) {
     const int i = base + k;
@@ -418,7 +431,13 @@ __global__ __launch_bounds__(256) void k_scan2_apply(int n, const int* __restric
   }
   int ta, tc;
   block_excl_scan2(a, c, ta, tc, sw);
-  int ra = a + bsum[2 * blockIdx.x], rc = c + bsum[2 * blockIdx.x + 1];
+  int ra = a + ba, rc = c + bc;
+  if (threadIdx.x == 0 && (blk + 1) * kScanBlock >= n) {  // the last one
+    out0[n] = ba + ta;
+    out1[n] = bc + tc;
+    totals[S.slot0] = ba + ta;
+    totals[S.slot1] = bc + tc;
+  }
   for (int k = 0; k < 4; k++) {
     const int i = base + k;
     if (i < n) {
@@ -468,13 +487,12 @@ __global__ void k_fill_double(double* p, size_t n) {
 // atoms listed by column (any order inside a column; k_rank orders them);
 // slots within a column are reserved once per (workgroup, column) as in
 // k_bin, over the same atom order
-__global__ __launch_bounds__(256) void k_scatter(int n, const int4* __restrict__ info,
-                                                 const int* __restrict__ col_start, int* __restrict__ fill,
-                                                 int* __restrict__ tmp, const int* __restrict__ order = nullptr,
-                                                 int norder = 0) {
+__device__ __forceinline__ void scatter_atoms(int blk, int n, const int4* __restrict__ info,
+                                              const int* __restrict__ col_start, int* __restrict__ fill,
+                                              int* __restrict__ tmp, const int* __restrict__ order, int norder) {
   __shared__ int sh[512];
   __shared__ int hist[kBinLds];
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  const int s = blk * blockDim.x + threadIdx.x;
   const int i = order ? (s < norder ? order[s] : -1) : (s < n ? s : -1);
   const int col = (i >= 0) ? info[i].w : -1;
   int lo, hi;
@@ -498,6 +516,11 @@ __global__ __launch_bounds__(256) void k_scatter(int n, const int4* __restrict__
   __syncthreads();
   if (col >= 0) tmp[col_start[col] + hist[col - lo] + local] = i;
 }
+__global__ __launch_bounds__(256) void k_scatter(Two<BinSide> T) {
+  const int d = T.side();
+  const BinSide& B = T.s[d];
+  scatter_atoms(T.block(d), B.n, B.info, B.col_start, B.fill, B.tmp, B.order, B.norder);
+}
 
 // Slots of one column and the bounds of its clusters; one workgroup per column.
 // (1) Rank of each atom inside its column by (key, index): a deterministic
@@ -519,22 +542,37 @@ constexpr int kRankBuckets = 256;  // the workgroup size: one scan
 __device__ __forceinline__ int rank_bucket(double k) {
   return max(0, min((int)(k * kRankBuckets), kRankBuckets - 1));
 }
-__global__ __launch_bounds__(256) void k_rank(int ncol, const double* __restrict__ key,
-                                              const int* __restrict__ col_start, const int* __restrict__ col_cl,
-                                              const int* __restrict__ tmp, int* __restrict__ slot_loc,
-                                              const int4* __restrict__ info, const double* __restrict__ pos, int off,
-                                              const SysArg* __restrict__ sys, const int* __restrict__ atom_sys,
-                                              double4* __restrict__ origin, float4* __restrict__ bb0,
-                                              float2* __restrict__ kr, int* __restrict__ cl_sys,
-                                              int* __restrict__ cl_col, float4* __restrict__ pk,
-                                              float4* __restrict__ pbb, double pscale) {
+// clear0, clear1 (optional): the column's atom count and fill position, zeroed
+// for the next build.
+struct RankSide {
+  int ncol, off;
+  const double* key;
+  const int *col_start, *col_cl, *tmp;
+  int* slot_loc;
+  const int4* info;
+  const SysArg* sys;
+  double4* origin;
+  float4* bb0;
+  float2* kr;
+  int *cl_sys, *cl_col;
+  float4 *pk, *pbb;
+  int *clear0, *clear1;
+};
+__device__ __forceinline__ void rank_column(int col, int ncol, const double* __restrict__ key,
+                                            const int* __restrict__ col_start, const int* __restrict__ col_cl,
+                                            const int* __restrict__ tmp, int* __restrict__ slot_loc,
+                                            const int4* __restrict__ info, const double* __restrict__ pos, int off,
+                                            const SysArg* __restrict__ sys, const int* __restrict__ atom_sys,
+                                            double4* __restrict__ origin, float4* __restrict__ bb0,
+                                            float2* __restrict__ kr, int* __restrict__ cl_sys,
+                                            int* __restrict__ cl_col, float4* __restrict__ pk,
+                                            float4* __restrict__ pbb, double pscale) {
   __shared__ double sk[kRankLds];
   __shared__ int si[kRankLds];
   __shared__ int ss[kRankLds];
   __shared__ int sbk[kRankLds];  // local indices grouped by key bucket
   __shared__ int bcnt[kRankBuckets], bstart[kRankBuckets + 1];
   __shared__ int sw[32];
-  const int col = blockIdx.x;
   if (col >= ncol) return;
   const int b = col_start[col], n = col_start[col + 1] - b;
   const int c0 = col_cl[col], ncl = col_cl[col + 1] - c0;
@@ -671,6 +709,14 @@ __global__ __launch_bounds__(256) void k_rank(int ncol, const double* __restrict
   }
 }
 
+__global__ __launch_bounds__(256) void k_rank(Two<RankSide> T, const double* pos, const int* atom_sys, double pscale) {
+  const int d = T.side(), col = T.block(d);
+  const RankSide& R = T.s[d];
+  if (R.clear0 && threadIdx.x == 0 && col < R.ncol) R.clear0[col] = R.clear1[col] = 0;
+  rank_column(col, R.ncol, R.key, R.col_start, R.col_cl, R.tmp, R.slot_loc, R.info, pos, R.off, R.sys, atom_sys,
+              R.origin, R.bb0, R.kr, R.cl_sys, R.cl_col, R.pk, R.pbb, pscale);
+}
+
 // Two groups that share atoms: for every slot, the requested index of the same
 // atom in the other group (twin, by requested index; negative: not in it), so
 // that the pair kernels leave out an atom's pair with itself
@@ -801,15 +847,53 @@ __device__ __forceinline__ float column_window(const SysArg& S, float rlist2, fl
   return fminf(__builtin_amdgcn_sqrtf(left) * S.invc + 2.0e-6f, S.rb[2]);
 }
 
+// With items, k_list<1> also writes the work items of its cluster ({i cluster,
+// first entry, end entry} of `chunk` entries each) and their place in the pair
+// kernel's schedule (k_wave_sched): two launches less.
+struct ItemArgs {
+  int4* items;
+  const int* istart;
+  int chunk, items_cap;
+  int nwaves;       // 0: no schedule
+  int nitems;
+  long long total;  // cost of all items
+  int* wave_start;
+};
+struct ListSide {
+  ListArgs L;
+  const int *cl_colI, *cl_sysI;
+  const SysArg *sysI, *sysJ;
+  const float4 *bbI, *bbJ;
+  const float2 *krI, *krJ;
+  const int* col_clJ;
+  const double4 *orgI, *orgJ;
+  int* count;
+  const int* start;
+  Entry* out;
+  unsigned* ell;
+  ItemArgs M;
+};
+
+// Balanced static schedule of the pair kernel: the items split into nwaves
+// contiguous ranges of about equal estimated cost, an item costing its
+// entries plus kItemCost (the staging and sums each item pays).  Item i
+// (cost prefix P_i, total C) goes to wave floor(P_i * nwaves / C).
+constexpr int kItemCost = 32;
+__device__ __forceinline__ int sched_wave(long long entry0, int item, long long total, int nwaves) {
+  const long long pre = entry0 + (long long)kItemCost * item;
+  return (int)min((long long)nwaves - 1, pre * nwaves / total);
+}
+
 template <int FILL>
-__global__ __launch_bounds__(256) void k_list(ListArgs L, const int* __restrict__ cl_colI,
+__device__ __forceinline__ void list_clusters(int blk, const ListArgs& L, const int* __restrict__ cl_colI,
                                               const int* __restrict__ cl_sysI, const SysArg* __restrict__ sysI,
                                               const SysArg* __restrict__ sysJ, const float4* __restrict__ bbI,
                                               const float4* __restrict__ bbJ, const float2* __restrict__ krI,
                                               const float2* __restrict__ krJ, const int* __restrict__ col_clJ,
                                               const double4* __restrict__ orgI, const double4* __restrict__ orgJ,
                                               int* __restrict__ count, const int* __restrict__ start,
-                                              Entry* __restrict__ out, unsigned* __restrict__ ell) {
+                                              Entry* __restrict__ out, unsigned* __restrict__ ell,
+                                              const ItemArgs& M) {
   __shared__ unsigned s_cand[4][kCandCap];
   __shared__ float4 s_img[4][27];  // FP32 lattice translation of each image code
   const int lane = threadIdx.x & 63;
@@ -818,7 +902,7 @@ __global__ __launch_bounds__(256) void k_list(ListArgs L, const int* __restrict_
   // FILL=0/1: cluster ci = the wave.  FILL=2: the wave's 64 clusters, of which
   // it searches those whose candidates did not all fit in ell (the others are
   // k_list_stream's), in order.  No workgroup barrier below.
-  int ci = blockIdx.x * (blockDim.x / WAVE) + wv;
+  int ci = blk * (blockDim.x / WAVE) + wv;
   unsigned long long pending = 0ull;
   if (FILL == 2) {
     const int c0 = ci * WAVE;
@@ -870,6 +954,21 @@ __global__ __launch_bounds__(256) void k_list(ListArgs L, const int* __restrict_
   const int base = FILL ? start[ci] : 0;
   if (FILL == 1) {
     const int nc = count[ci];
+    if (M.items) {
+      const int i0 = M.istart[ci], nch = (nc + M.chunk - 1) / M.chunk;
+      for (int k = lane; k < nch; k += WAVE) {
+        const int it = i0 + k, e = base + k * M.chunk, end = base + min(nc, (k + 1) * M.chunk);
+        if (it < M.items_cap) M.items[it] = make_int4(ci, e, end, 0);
+        if (M.nwaves) {
+          // entries are contiguous: item it + 1 starts where this one ends
+          const int w0 = sched_wave(e, it, M.total, M.nwaves);
+          const int w1 = it + 1 < M.nitems ? sched_wave(end, it + 1, M.total, M.nwaves) : M.nwaves;
+          if (it == 0)
+            for (int w = 0; w <= w0; w++) M.wave_start[w] = 0;
+          for (int w = w0 + 1; w <= w1; w++) M.wave_start[w] = it + 1;
+        }
+      }
+    }
     if (nc <= kEll) {
       for (int e = lane; e < nc; e += WAVE) {
         const unsigned pk = ell[(size_t)ci * kEll + e];
@@ -996,6 +1095,14 @@ __global__ __launch_bounds__(256) void k_list(ListArgs L, const int* __restrict_
   }
 }
 
+template <int FILL>
+__global__ __launch_bounds__(256) void k_list(Two<ListSide> T) {
+  const int d = T.side();
+  const ListSide& S = T.s[d];
+  list_clusters<FILL>(T.block(d), S.L, S.cl_colI, S.cl_sysI, S.sysI, S.sysJ, S.bbI, S.bbJ, S.krI, S.krJ, S.col_clJ,
+                      S.orgI, S.orgJ, S.count, S.start, S.out, S.ell, S.M);
+}
+
 // Fill pass of the clusters whose candidates all fit in `ell` (count <=
 // kEll): their entries in the order the count pass kept them, one wave per
 // i cluster, two entries per lane and trip.  The search kernel's registers
@@ -1052,13 +1159,9 @@ __global__ void k_items(int ncl, const int* __restrict__ ncl_dev, const int* __r
   }
 }
 
-// Balanced static schedule of the pair kernel: the items split into nwaves
-// contiguous ranges of about equal estimated cost, an item costing its
-// entries plus kItemCost (the staging and sums each item pays).  Item i
-// (cost prefix P_i, total C) goes to wave floor(P_i * nwaves / C); one
-// thread per item writes the first item of each wave it starts.
-// wave_start has nwaves + 1 entries; nitems = *nitems_dev when given.
-constexpr int kItemCost = 32;
+// the pair kernel's schedule from the items (sched_wave); one thread per item
+// writes the first item of each wave it starts.  wave_start has nwaves + 1
+// entries; nitems = *nitems_dev when given.
 __global__ void k_wave_sched(int nitems, const int* __restrict__ nitems_dev, int items_cap,
                              const int4* __restrict__ items, int nwaves, int* __restrict__ wave_start) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1069,10 +1172,7 @@ __global__ void k_wave_sched(int nitems, const int* __restrict__ nitems_dev, int
   }
   if (i >= nitems) return;
   const long long total = (long long)items[nitems - 1].z + (long long)kItemCost * nitems;
-  auto wave_of = [&](int q) {
-    const long long pre = (long long)items[q].y + (long long)kItemCost * q;
-    return (int)min((long long)nwaves - 1, pre * nwaves / total);
-  };
+  auto wave_of = [&](int q) { return sched_wave(items[q].y, q, total, nwaves); };
   const int wi = wave_of(i);
   const int wp = i == 0 ? -1 : wave_of(i - 1);
   for (int w = wp + 1; w <= wi; w++) wave_start[w] = i;
@@ -1087,14 +1187,20 @@ __global__ void k_wave_sched(int nitems, const int* __restrict__ nitems_dev, int
 // k_pack and k_bbox in one pass: one thread per slot, the 8 slots of a
 // cluster are 8 adjacent lanes, which reduce the cluster's box by shuffles.
 // Positions relative to the cluster origin, times pscale (pack_scale).
-__global__ __launch_bounds__(256) void k_pack_bbox(int nslot, const int* __restrict__ ncl_dev,
-                                                   const int* __restrict__ slot_loc, const int4* __restrict__ info,
-                                                   const double* __restrict__ pos, int off,
-                                                   const SysArg* __restrict__ sys, const int* __restrict__ atom_sys,
-                                                   const double4* __restrict__ origin, float4* __restrict__ out,
-                                                   float4* __restrict__ bb, double pscale) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (ncl_dev) nslot = *ncl_dev * CL;
+struct PackSide {
+  int nslot;
+  const int* slot_loc;
+  const int4* info;
+  int off;
+  const SysArg* sys;
+  const double4* origin;
+  float4 *out, *bb;
+};
+__device__ __forceinline__ void pack_bbox(int blk, int nslot, const int* __restrict__ slot_loc,
+                                          const int4* __restrict__ info, const double* __restrict__ pos, int off,
+                                          const SysArg* __restrict__ sys, const double4* __restrict__ origin,
+                                          float4* __restrict__ out, float4* __restrict__ bb, double pscale) {
+  const int s = blk * blockDim.x + threadIdx.x;
   // whole groups of 8 lanes stay together (nslot is a multiple of 8)
   if (s >= nslot) return;
   const int a = slot_loc[s];
@@ -1106,7 +1212,7 @@ __global__ __launch_bounds__(256) void k_pack_bbox(int nslot, const int* __restr
     lo[0] = lo[1] = lo[2] = FLT_MAX;
     hi[0] = hi[1] = hi[2] = -FLT_MAX;
   } else {
-    const SysArg& S = sys[nsys_of(atom_sys, a)];
+    const SysArg& S = *sys;
     const int4 m = info[a];
     const double4 o = origin[s / CL];
     const double* x = pos + 3 * (size_t)(off + a);
@@ -1130,6 +1236,12 @@ __global__ __launch_bounds__(256) void k_pack_bbox(int nslot, const int* __restr
     bb[2 * c] = make_float4(0.5f * (lo[0] + hi[0]), 0.5f * (lo[1] + hi[1]), 0.5f * (lo[2] + hi[2]), 0.f);
     bb[2 * c + 1] = make_float4(0.5f * (hi[0] - lo[0]), 0.5f * (hi[1] - lo[1]), 0.5f * (hi[2] - lo[2]), 0.f);
   }
+}
+
+__global__ __launch_bounds__(256) void k_pack_bbox(Two<PackSide> T, const double* pos, double pscale) {
+  const int d = T.side();
+  const PackSide& P = T.s[d];
+  pack_bbox(T.block(d), P.nslot, P.slot_loc, P.info, pos, P.off, P.sys, P.origin, P.out, P.bb, pscale);
 }
 
 // The FP64 helpers below take the reference's rounding: no fused
@@ -1996,22 +2108,35 @@ struct RedArgs {
 
 // After the pair kernels, in one launch.  With do_red, workgroup 0 forms the
 // value, virial and pair count from the rows of R in a fixed order (each
-// thread a fixed set of rows, then a fixed tree); the other ngather
+// thread a fixed set of rows, then a fixed tree); the other
 // workgroups form the derivatives of the atoms of every i cluster (fixed-order
 // sums of the cluster's item partials).  The reduction workgroup comes first
 // so that it starts with the first wave of workgroups.
-__global__ __launch_bounds__(256) void k_gather_reduce(int ngather, int ncl, const int* __restrict__ ncl_dev,
-                                                       const float4* __restrict__ p,
-                                                       const int* __restrict__ item_start, int items_cap,
-                                                       const double* __restrict__ fpart, double* __restrict__ deriv,
-                                                       int do_red, RedArgs R) {
+struct GatherSide {
+  int ncl;
+  const int* ncl_dev;
+  const float4* p;
+  const int* item_start;
+  int items_cap;
+  const double* fpart;
+};
+__global__ __launch_bounds__(256) void k_gather_reduce(Two<GatherSide> T, double* __restrict__ deriv, int do_red,
+                                                       RedArgs R) {
   if (R.skip && *R.skip) return;
   const int t = threadIdx.x;
   const int red = do_red ? 1 : 0;
   if ((int)blockIdx.x >= red) {
     if (!deriv) return;
-    const int g = (blockIdx.x - red) * blockDim.x + t;
-    if (ncl_dev) ncl = *ncl_dev;
+    int blk = (int)blockIdx.x - red;
+    const int d = blk >= T.n0 ? 1 : 0;
+    if (d) blk -= T.n0;
+    const GatherSide& G = T.s[d];
+    const float4* __restrict__ p = G.p;
+    const int* __restrict__ item_start = G.item_start;
+    const double* __restrict__ fpart = G.fpart;
+    const int items_cap = G.items_cap;
+    const int ncl = G.ncl_dev ? *G.ncl_dev : G.ncl;
+    const int g = blk * blockDim.x + t;
     if (g >= ncl * CL * 3) return;
     const int c = g / (CL * 3), r = g % (CL * 3);
     // every load that depends only on c goes out before the first wait
@@ -3128,20 +3253,25 @@ inline void launch_pairs(const PairArgs& A, int grid, hipStream_t s, bool value_
 }
 
 // entry starts (out0) and work-item starts (out1, chunks of `chunk`) of the
-// n = *n_dev (or n) i clusters; bsum holds 2 * ceil(ncap / kScanBlock) ints
-inline void launch_list_scans(hipStream_t s, int ncap, const int* n_dev, const int* count, int chunk, int* bsum,
-                              int* out0, int* out1, int* totals, int slot0, int slot1) {
-  if (ncap <= kScanOneMax) {
-    hipLaunchKernelGGL(k_scan2_one, dim3(1), dim3(1024), 0, s, ncap, n_dev, count, chunk, out0, out1, totals, slot0,
-                       slot1);
+// n = *n_dev (or n) i clusters of each side; bsum holds 2 * ceil(n / kScanBlock)
+// ints
+inline void launch_list_scans(hipStream_t s, const ScanSide* sides, int nsides, int chunk, int* totals) {
+  Two<ScanSide> T;
+  bool one = true;
+  int nb[2] = {0, 0};
+  for (int d = 0; d < 2; d++) {
+    T.s[d] = sides[std::min(d, nsides - 1)];
+    if (d >= nsides) continue;
+    one = one && sides[d].n <= kScanOneMax;
+    nb[d] = std::max(1, grid1(sides[d].n, kScanBlock));
+  }
+  T.n0 = nb[0];
+  if (one) {
+    hipLaunchKernelGGL(k_scan2_one, dim3(nsides), dim3(1024), 0, s, T, chunk, totals);
     return;
   }
-  const int nb = std::max(1, grid1(ncap, kScanBlock));
-  hipLaunchKernelGGL(k_scan2_sums, dim3(nb), dim3(256), 0, s, ncap, n_dev, count, chunk, bsum);
-  hipLaunchKernelGGL(k_scan2_blocks, dim3(1), dim3(1024), 0, s, nb, ncap, n_dev, bsum, out0, out1, totals, slot0,
-                     slot1);
-  hipLaunchKernelGGL(k_scan2_apply, dim3(nb), dim3(256), 0, s, ncap, n_dev, count, chunk, (const int*)bsum, out0,
-                     out1);
+  hipLaunchKernelGGL(k_scan2_sums, dim3(nb[0] + nb[1]), dim3(256), 0, s, T, chunk);
+  hipLaunchKernelGGL(k_scan2_apply, dim3(nb[0] + nb[1]), dim3(256), 0, s, T, chunk, totals);
 }
 
 // Scale of the FP32 cluster geometry (packed positions, list offsets,
