@@ -156,28 +156,28 @@ static int batch_step(p2a_batch* b, const double* pos, double* values, double* d
   PairArgs A;
   std::memset(&A, 0, sizeof(A));
   pair_args_switch(b->sw, A);
-  A.nitems = 0;
-  A.nitems_dev = b->totals.p + 3;
-  A.items_cap = b->items_cap;
-  A.ent_cap = b->ent_cap;
   A.pbc = b->pbc.p;
   A.cl_sys = b->cl_sys.p;
   A.pos64 = pos;
   A.item_partials = 1;  // per-system sums need the items' own partials
   A.ipart = b->partial.p;
   int grid = grid1(std::max(b->items_cap, 1), PAIR_BLOCK / WAVE);
-  A.wave_start = nullptr;
+  const int* wave_start = nullptr;
   if (b->tune.blocks_per_cu > 0) grid = std::min(grid, b->tune.blocks_per_cu * b->cu_count);
   const int nw = grid * (PAIR_BLOCK / WAVE);
   // contiguous item ranges of balanced cost per wave of the persistent grid
   // (the first step runs before the list arrays exist: no items, no schedule)
   if (b->tune.blocks_per_cu > 0 && b->items_cap > 0 && b->wave_start.p && b->wave_start.n >= (size_t)nw + 1) {
     hipLaunchKernelGGL(k_wave_sched, dim3(grid1(std::max(b->items_cap, 1), 256)), dim3(256), 0, s, 0,
-                       (const int*)A.nitems_dev, b->items_cap, (const int4*)b->items.p, nw, b->wave_start.p);
-    A.wave_start = b->wave_start.p;
+                       (const int*)b->totals.p + 3, b->items_cap, (const int4*)b->items.p, nw, b->wave_start.p);
+    wave_start = b->wave_start.p;
   }
-  launch_pairs<false>(A, grid, s, false, chunk, b->items.p, b->ents.p, b->p.p, b->p.p, b->bb.p, b->bb.p,
-                      (const int*)nullptr, b->fpart.p, b->partial.p);
+  Two<PairSide> Pt;
+  std::memset(&Pt, 0, sizeof(Pt));
+  Pt.n0 = grid;
+  Pt.s[0] = PairSide{grid,      0,        b->totals.p + 3, b->items_cap, b->ent_cap, wave_start, b->items.p, b->ents.p,
+                     b->p.p,    b->p.p,   b->bb.p,         b->bb.p,      nullptr,    b->fpart.p, b->partial.p};
+  launch_pairs<false>(A, Pt, s, false, chunk);
   if ((rc = launch_check("batch: pair kernel"))) return rc;
   Two<GatherSide> Gt;
   std::memset(&Gt, 0, sizeof(Gt));

@@ -509,7 +509,6 @@ static int run_pairs(p2a_coord* c, const double* box9, const double* pos_dev, do
   if ((rc = upload_pbc(c, box9))) return rc;
   A.pbc = c->pbc_dev.p;
   A.cl_sys = nullptr;
-  A.nitems_dev = nullptr;
   A.pos64 = pos_dev;
   A.skip = skip;
   A.item_partials = 0;  // value / virial / pair count per workgroup
@@ -539,16 +538,16 @@ static int run_pairs(p2a_coord* c, const double* box9, const double* pos_dev, do
     c->ev_pool.pop_back();
     P2A_HIP(hipEventRecord(e0, s));
   }
+  Two<PairSide> T;
+  std::memset(&T, 0, sizeof(T));
+  T.n0 = grids[0];
   int off = 0;
   for (int d = 0; d < ndir_run; d++) {
     Dir& D = c->dir[d];
     if (grids[d] == 0) continue;
     Group& GI = c->g[D.I];
     Group& GJ = c->g[D.J];
-    A.nitems = D.nitems;
-    A.items_cap = (int)D.items.n;
-    A.ent_cap = (int)D.ents.n;
-    A.wave_start = nullptr;
+    const int* wave_start = nullptr;
     if (c->tune.blocks_per_cu > 0) {
       // a persistent grid takes contiguous item ranges of balanced cost
       const int nw = grids[d] * (PAIR_BLOCK / WAVE);
@@ -559,12 +558,14 @@ static int run_pairs(p2a_coord* c, const double* box9, const double* pos_dev, do
         D.sched_waves = nw;
         D.sched_gen = c->rebuilds;
       }
-      A.wave_start = D.wave_start.p;
+      wave_start = D.wave_start.p;
     }
-    launch_pairs<true>(A, grids[d], s, value_only, c->tune.chunk, D.items.p, D.ents.p, GI.p.p, GJ.p.p, GI.bb.p, GJ.bb.p,
-                 GI.twin_slot.p, D.fpart.p, c->partial.p + 8 * (size_t)off);
+    T.s[d] = PairSide{grids[d], D.nitems, nullptr,  (int)D.items.n, (int)D.ents.n, wave_start,       D.items.p, D.ents.p,
+                      GI.p.p,   GJ.p.p,   GI.bb.p,  GJ.bb.p,        GI.twin_slot.p, D.fpart.p,
+                      c->partial.p + 8 * (size_t)off};
     off += grids[d];
   }
+  if (off > 0) launch_pairs<true>(A, T, s, value_only, c->tune.chunk);
   if (rec) {
     P2A_HIP(hipEventRecord(e1, s));
     c->pending.emplace_back(e0, e1);

@@ -211,9 +211,8 @@ __device__ __forceinline__ int nsys_of(const int* idx, int i) { return idx ? idx
 // of one XCD on one contiguous run of indices, so that an XCD takes one
 // contiguous share of the spatially sorted work items and its L2 holds the
 // positions of one region instead of all of them.  A bijection on
-// [0, gridDim.x) for any grid size.
-__device__ __forceinline__ int xcd_block() {
-  const int nb = gridDim.x, b = blockIdx.x;
+// [0, nb) for any grid size.
+__device__ __forceinline__ int xcd_block(int b, int nb) {
   const int q = nb >> 3, r = nb & 7, x = b & 7;
   return x * q + min(x, r) + (b >> 3);
 }
@@ -1424,9 +1423,7 @@ __device__ __forceinline__ float sw_fixed_value(float invr0_2, float r2) {
 constexpr int kBandSlots = 64;
 
 struct PairArgs {
-  int nitems;
-  const int* nitems_dev;  // device item count (null: nitems)
-  int items_cap, ent_cap; // capacities of the item and entry arrays
+  int nitems, items_cap, ent_cap;  // row kernel: items, capacities of the item and entry arrays
   int share;              // the two groups have atoms in common (twinI tells them)
   float dmax2, prune2, band;
   float cut_lo, cut_hi;   // FP32 r^2 at or below cut_lo: inside; in (cut_lo, cut_hi): the band
@@ -1443,9 +1440,6 @@ struct PairArgs {
   // `partial` over all of its items.
   int item_partials;
   double* ipart;
-  // Items of each wave of the grid: [wave_start[g], wave_start[g + 1]) for
-  // wave g = xcd_block() * 4 + wave (k_wave_sched); null: items g, g + waves, ...
-  const int* wave_start;
   // when set and *skip != 0 (written by an earlier kernel on the stream), the
   // launch does nothing: a pass queued on a list that may be stale
   const int* skip;
@@ -1978,8 +1972,9 @@ constexpr int stage_cap() {
 // every listed entry was staged).  Known rational 6-12, 50,000 atoms: 38 us
 // (41 before); EXP, 20,000 atoms: 60 us.
 template <int P, bool GENERIC, bool TWO, bool VO, int CH>
-__global__ __launch_bounds__(PAIR_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void k_pairs(
-    PairArgs A, const int4* __restrict__ items, const Entry* __restrict__ ents, const float4* __restrict__ posI,
+__device__ __forceinline__ void pairs_body(
+    const PairArgs& A, int grid_block, int grid, int nitems, int ent_cap, const int* __restrict__ wave_start,
+    const int4* __restrict__ items, const Entry* __restrict__ ents, const float4* __restrict__ posI,
     const float4* __restrict__ posJ, const float4* __restrict__ bbI, const float4* __restrict__ bbJ,
     const int* __restrict__ twinI, double* __restrict__ fpart, double* __restrict__ partial) {
   constexpr int NW = PAIR_BLOCK / WAVE;
@@ -1987,11 +1982,9 @@ __global__ __launch_bounds__(PAIR_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
   __shared__ float4 sj[NW][CAP];
   __shared__ Entry sent[NW][sent_cap<CH>()];
   __shared__ double stot[NW][8];
-  if (A.skip && *A.skip) return;
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int ii = lane & 7, jj = lane >> 3;
-  const int nitems = A.nitems_dev ? min(*A.nitems_dev, A.items_cap) : A.nitems;
   const WaveLds L = {sj[w], sent[w]};
   PairAcc acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   int ntot = 0;
@@ -2002,12 +1995,12 @@ __global__ __launch_bounds__(PAIR_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
   // computes (a wave handles several items when the grid is persistent)
   // the wave's items: a contiguous range of balanced cost, or every
   // (grid waves)-th item
-  const int blk = xcd_block();
+  const int blk = xcd_block(grid_block, grid);
   const int gw = blk * NW + w;
-  int kfirst = gw, kstride = gridDim.x * NW, kend = nitems;
-  if (A.wave_start) {
-    kfirst = A.wave_start[gw];
-    kend = min(A.wave_start[gw + 1], nitems);
+  int kfirst = gw, kstride = grid * NW, kend = nitems;
+  if (wave_start) {
+    kfirst = wave_start[gw];
+    kend = min(wave_start[gw + 1], nitems);
     kstride = 1;
   }
   int k = kfirst;
@@ -2016,7 +2009,7 @@ __global__ __launch_bounds__(PAIR_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
   if (k < kend) {
     it_n = items[k];
     const int e = it_n.y + lane;
-    if (lane < CH && e < min(it_n.z, A.ent_cap)) my_n = ents[e];
+    if (lane < CH && e < min(it_n.z, ent_cap)) my_n = ents[e];
   }
   for (; k < kend; k += kstride) {
     const int item = k;
@@ -2025,7 +2018,7 @@ __global__ __launch_bounds__(PAIR_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
     const int kn = k + kstride;
     if (kn < kend) it_n = items[kn];
     const int ci = it.x;
-    const int e1 = min(it.z, A.ent_cap);
+    const int e1 = min(it.z, ent_cap);
     const float4 pi = posI[ci * CL + ii];
     const int ai = TWO ? twinI[ci * CL + ii] : 0;
     const float4 ic = bbI[2 * ci], ih = bbI[2 * ci + 1];
@@ -2033,7 +2026,7 @@ __global__ __launch_bounds__(PAIR_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
     stage_item<VO, true, CH>(A, my_e, lane, it.y, e1, ci, ic, ih, posJ, bbJ, L, n0, b1, n1, b2, n2);
     if (kn < kend) {
       const int e = it_n.y + lane;
-      my_n = (lane < CH && e < min(it_n.z, A.ent_cap)) ? ents[e] : Entry{0, 0.f, 0.f, 0.f};
+      my_n = (lane < CH && e < min(it_n.z, ent_cap)) ? ents[e] : Entry{0, 0.f, 0.f, 0.f};
     }
     // group bounds are wave-uniform: scalar loops
     n1 = __builtin_amdgcn_readfirstlane(n1);
@@ -2085,6 +2078,33 @@ __global__ __launch_bounds__(PAIR_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
       partial[(size_t)blk * 8 + lane] = s;
     }
   }
+}
+
+struct PairSide {
+  int grid, nitems;
+  const int* nitems_dev;   // device item count (null: nitems)
+  int items_cap, ent_cap;  // capacities of the item and entry arrays
+  // Items of each wave of the grid: [wave_start[g], wave_start[g + 1]) for
+  // wave g = xcd_block * 4 + wave (sched_wave); null: items g, g + waves, ...
+  const int* wave_start;
+  const int4* items;
+  const Entry* ents;
+  const float4 *posI, *posJ, *bbI, *bbJ;
+  const int* twinI;
+  double *fpart, *partial;
+};
+// both directions of two groups in one launch: the second one's workgroups start
+// as the first one's end (10,000 x 490,000 atoms: 72 us, one after the other 76;
+// 1,000 x 1,000: 10, 19)
+template <int P, bool GENERIC, bool TWO, bool VO, int CH>
+__global__ __launch_bounds__(PAIR_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void k_pairs(PairArgs A,
+                                                                                             Two<PairSide> T) {
+  if (A.skip && *A.skip) return;
+  const int d = T.side();
+  const PairSide& S = T.s[d];
+  const int nitems = S.nitems_dev ? min(*S.nitems_dev, S.items_cap) : S.nitems;
+  pairs_body<P, GENERIC, TWO, VO, CH>(A, T.block(d), S.grid, nitems, S.ent_cap, S.wave_start, S.items, S.ents, S.posI,
+                                      S.posJ, S.bbI, S.bbJ, S.twinI, S.fpart, S.partial);
 }
 
 // virial = -sum dd (x) d (CoordinationBase.cpp:200-206), symmetric
@@ -3036,7 +3056,7 @@ __global__ __launch_bounds__(PAIR_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int ii = lane & 7, jj = lane >> 3;
-  const int nitems = A.nitems_dev ? min(*A.nitems_dev, A.items_cap) : A.nitems;
+  const int nitems = min(A.nitems, A.items_cap);
   const WaveLds L = {sj[w], sent[w]};
   if (lane < 8) stot[w][lane] = 0.0;
   for (int k = blockIdx.x * NW + w; k < nitems; k += gridDim.x * NW) {
@@ -3189,13 +3209,11 @@ inline int switch_known_kind(const p2a_switch& sw) {
 // with derivatives (20,000 atoms with EXP: pair pass 105 -> 62 us); value only and 32 entries
 // an item run the kernel that takes any switch.
 template <bool TWOG>
-inline void launch_pairs(const PairArgs& A, int grid, hipStream_t s, bool value_only, int chunk, const int4* items,
-                         const Entry* ents, const float4* posI, const float4* posJ, const float4* bbI,
-                         const float4* bbJ, const int* twinI, double* fpart, double* partial) {
+inline void launch_pairs(const PairArgs& A, const Two<PairSide>& T, hipStream_t s, bool value_only, int chunk) {
   const p2a_switch& sw = A.sw;
-#define P2A_K(P, GEN, TWO, VO, CH)                                                                                \
-  hipLaunchKernelGGL((k_pairs<P, GEN, TWO, VO, CH>), dim3(grid), dim3(PAIR_BLOCK), 0, s, A, items, ents, posI,      \
-                     posJ, bbI, bbJ, twinI, fpart, partial)
+  const int grid = T.s[0].grid + T.s[1].grid;
+#define P2A_K(P, GEN, TWO, VO, CH) \
+  hipLaunchKernelGGL((k_pairs<P, GEN, TWO, VO, CH>), dim3(grid), dim3(PAIR_BLOCK), 0, s, A, T)
 #define P2A_KCH(P, GEN, TWO, VO)          \
   do {                                    \
     if (chunk == 32) P2A_K(P, GEN, TWO, VO, 32); \
