@@ -262,6 +262,10 @@ class CoordinationNumbers:
         self.env = env
         self.pbc = pbc
         self._idx = None
+        # largest index (reading it back from the device on every call waited for
+        # the stream), and whether the requested atoms are 0, 1, 2, ... once each
+        self._top = max(rows + (env or []))
+        self._in_order = env is None and rows == list(range(len(rows)))
 
     def _req(self, device):
         import torch
@@ -280,9 +284,12 @@ class CoordinationNumbers:
         if not (pos.is_cuda and pos.dtype == torch.float64 and pos.dim() == 2 and pos.shape[1] == 3):
             raise ValueError("positions must be a float64 CUDA tensor [natoms,3]")
         idx = self._req(pos.device)
-        if int(idx.max()) >= pos.shape[0]:
+        if self._top >= pos.shape[0]:
             raise ValueError("atom index outside the positions array")
-        req = pos.index_select(0, idx).contiguous()
+        # all atoms in order are the positions as they are (no gather, and below no
+        # scatter: 30,000 atoms 142 -> 95 us a call with weights)
+        whole = self._in_order and len(idx) == pos.shape[0]
+        req = pos.detach().contiguous() if whole else pos.index_select(0, idx).contiguous()
         b9 = _box9(box if box is not None else np.eye(3))
         self.action.set_stream(torch.cuda.current_stream(pos.device).cuda_stream)
         cn = torch.empty(len(self.rows), dtype=torch.float64, device=pos.device)
@@ -300,6 +307,8 @@ class CoordinationNumbers:
                                               C.c_void_p(req.data_ptr()), C.c_void_p(cn.data_ptr()),
                                               C.c_void_p(w.data_ptr()), C.c_void_p(vjp_req.data_ptr()),
                                               C.c_void_p(vir.data_ptr())))
+        if whole:
+            return cn, vjp_req, vir
         vjp = torch.zeros_like(pos)
         vjp.index_add_(0, idx, vjp_req)
         return cn, vjp, vir

@@ -74,3 +74,25 @@ def test_shared_groups_with_pairs_at_dmax(defn, na, lo, margin):
     assert abs(v - ov) <= TOL * abs(ov)
     close(d, od, F_TOL)
     close(w, ow, F_TOL)
+
+
+@pytest.mark.parametrize("layout", ["plain", "offset", "strided", "grad"])
+def test_all_atoms_in_order_are_not_gathered(layout):
+    """Rows over all atoms in order take the positions as they are, whatever
+    their layout: the same bits as through the gather (the same atoms listed as
+    rows of a longer array whose last atom is left out)."""
+    import torch
+    import plumed2_amd as P
+    x, box = lattice(16)
+    n = len(x)
+    w = np.random.default_rng(17).normal(size=n)
+    y = torch.tensor(np.vstack([x, [[0.5, 0.5, 0.5]]]), dtype=torch.float64, device="cuda:0")
+    t = {"plain": y[:n].clone(), "grad": y[:n].clone().requires_grad_(),
+         "offset": torch.cat([y[:1, 0], y[:n].reshape(-1)])[1:].view(n, 3),
+         "strided": torch.cat([y[:n], y[:n]], 1)[:, 3:]}[layout]
+    cn = P.CoordinationNumbers(SWITCHES[0], species=range(n))
+    a = cn(t, box, weights=w)
+    b = cn(y, box, weights=w)
+    assert a[1].shape == (n, 3) and b[1].shape == (n + 1, 3)
+    assert not any(q.requires_grad for q in a) and torch.all(b[1][n] == 0.0)
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1][:n]) and torch.equal(a[2], b[2])
