@@ -179,13 +179,9 @@ static int batch_step(p2a_batch* b, const double* pos, double* values, double* d
                      b->p.p,    b->p.p,   b->bb.p,         b->bb.p,      nullptr,    b->fpart.p, b->partial.p};
   launch_pairs<false>(A, Pt, s, false, chunk);
   if ((rc = launch_check("batch: pair kernel"))) return rc;
-  Two<GatherSide> Gt;
-  std::memset(&Gt, 0, sizeof(Gt));
-  Gt.n0 = grid1(nslot * 3, 256);
-  Gt.s[0] = GatherSide{clc, ncl_dev, b->p.p, b->istart.p, b->items_cap, b->fpart.p};
-  hipLaunchKernelGGL(k_gather_reduce, dim3(Gt.n0), dim3(256), 0, s, Gt, deriv, 0, RedArgs{});
-  hipLaunchKernelGGL(k_sys_reduce, dim3(b->nsys), dim3(256), 0, s, b->nsys, b->sys_colbase.p, b->col_cl.p,
-                     b->istart.p, b->items_cap, b->partial.p, values, virials, b->npairs.p);
+  const GatherSide G{clc, ncl_dev, b->p.p, b->istart.p, b->items_cap, b->fpart.p};
+  hipLaunchKernelGGL(k_gather_systems, dim3(b->nsys + grid1(nslot * 3, 256)), dim3(256), 0, s, b->nsys,
+                     b->sys_colbase.p, b->col_cl.p, b->partial.p, values, virials, b->npairs.p, G, deriv);
   return launch_check("batch: reductions");
 }
 
