@@ -114,7 +114,7 @@ static int batch_step(p2a_batch* b, const double* pos, double* values, double* d
   R.n0 = ncol;
   R.s[0] = RankSide{ncol,         0,           b->key.p, b->col_start.p, b->col_cl.p, b->tmp.p, b->slot_loc.p,
                     b->info.p,    b->sys.p,    b->origin.p, b->bb0.p, b->kr.p, b->cl_sys.p, b->cl_col.p, b->p.p,
-                    b->bb.p,      nullptr,     nullptr};
+                    b->bb.p,      nullptr,     nullptr,     nullptr};
   hipLaunchKernelGGL(k_rank, dim3(ncol), dim3(256), 0, s, R, pos, (const int*)b->atom_sys.p, pack_scale(b->sw));
   Two<ListSide> T;
   std::memset(&T, 0, sizeof(T));

@@ -48,7 +48,7 @@ struct Group {
   // col_count and fill hold zeros (k_rank leaves them so), at these addresses
   const int *zero_count = nullptr, *zero_fill = nullptr;
   DBuf<SysArg> sys;
-  DBuf<int4> info;
+  DBuf<int4> info, slot_img;
   DBuf<double> key;
   DBuf<int> col_count, col_start, col_cl, fill, tmp, slot_loc, cl_col, twin_slot;
   DBuf<double4> origin;
@@ -189,7 +189,7 @@ static int rebuild(p2a_coord* c, const double* box9, const double* pos_dev) {
         (rc = G.slot_loc.reserve((size_t)maxcl * CL)) || (rc = G.cl_col.reserve(maxcl)) ||
         (rc = G.origin.reserve(maxcl)) || (rc = G.bb0.reserve(2 * (size_t)maxcl)) ||
         (rc = G.bb.reserve(2 * (size_t)maxcl)) || (rc = G.p.reserve((size_t)maxcl * CL)) ||
-        (rc = G.kr.reserve(maxcl)) || (share && (rc = G.twin_slot.reserve((size_t)maxcl * CL))))
+        (rc = G.kr.reserve(maxcl)) || (rc = G.slot_img.reserve((size_t)maxcl * CL)) || (share && (rc = G.twin_slot.reserve((size_t)maxcl * CL))))
       return rc;
     // the descriptor goes to the device in stream order when it changed
     if (!G.S_valid || std::memcmp(&G.S, &G.S_dev, sizeof(SysArg)) != 0) {
@@ -240,7 +240,7 @@ static int rebuild(p2a_coord* c, const double* box9, const double* pos_dev) {
     cols[gi] = ScanSide{G.ncol, nullptr, G.col_count.p, G.col_start.p, G.col_cl.p, 4 + 2 * gi, 5 + 2 * gi, bsum[gi]};
     R.s[gi] = RankSide{G.ncol,   G.off,   G.key.p, G.col_start.p, G.col_cl.p,       G.tmp.p,    G.slot_loc.p,
                        G.info.p, G.sys.p, G.origin.p, G.bb0.p,    G.kr.p,           nullptr,    G.cl_col.p,
-                       G.p.p,    G.bb.p,  G.col_count.p, G.fill.p};
+                       G.p.p,    G.bb.p,  G.col_count.p, G.fill.p, G.slot_img.p};
     nrank[gi] = G.n > 0 ? G.ncol : 0;
   }
   B.n0 = nbin[0];
@@ -486,7 +486,7 @@ static void pack_positions(p2a_coord* c, const double* pos_dev) {
   int nb[2] = {0, 0};
   for (int gi = 0; gi < ngroups; gi++) {
     Group& G = c->g[gi];
-    T.s[gi] = PackSide{G.ncl * CL, G.slot_loc.p, G.info.p, G.off, G.sys.p, G.origin.p, G.p.p, G.bb.p};
+    T.s[gi] = PackSide{G.ncl * CL, G.slot_loc.p, G.slot_img.p, G.off, G.sys.p, G.origin.p, G.p.p, G.bb.p};
     nb[gi] = G.ncl > 0 ? grid1((size_t)G.ncl * CL, 256) : 0;
   }
   T.n0 = nb[0];
