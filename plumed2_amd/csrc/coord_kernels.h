@@ -1301,6 +1301,7 @@ template <int CTRL>
 __device__ __forceinline__ float dpp_f(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
 }
+constexpr int kQuadXor1 = 0xB1, kQuadXor2 = 0x4E;  // quad_perm 1,0,3,2 and 2,3,0,1
 constexpr int kRor1 = 0x121, kRor2 = 0x122, kRor4 = 0x124, kRor8 = 0x128;
 
 // v[l] + v[l ^ 16]: odd 16-lane rows of one copy swap with even rows of the other
@@ -1797,6 +1798,31 @@ __device__ __forceinline__ double item_row(const PairArgs& A, const PairAcc& acc
                    : (lane < 7 ? A.vir_scale * (double)tq : (double)npair);
 }
 
+// The same row entries with one entry per pair of lanes: entry `lane` / 2 in the
+// even lanes below 16 (bit 3 of the lane: bit 2 of the entry, and so on).  The
+// eight sums share their steps: at each of the first three a lane keeps half of
+// its values and adds the partner's (xor 8, 4, 2, then 1, 16, 32: the additions
+// of wave_sum_f, so the same bits) in about half of the instructions.
+__device__ __forceinline__ double item_row_pairs(const PairArgs& A, const PairAcc& acc, int npair, int lane) {
+  const bool b3 = lane & 8, b2 = lane & 4, b1 = lane & 2;
+  const float lo[4] = {acc.sv, acc.vxx, acc.vxy, acc.vxz}, hi[4] = {acc.vyy, acc.vyz, acc.vzz, 0.f};
+  float a[4], b[2];
+#pragma unroll
+  for (int k = 0; k < 4; k++) a[k] = (b3 ? hi[k] : lo[k]) + dpp_f<kRor8>(b3 ? lo[k] : hi[k]);
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    const float give = b2 ? a[k] : a[k + 2];
+    b[k] = (b2 ? a[k + 2] : a[k]) +
+           __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(give), 0x101F));  // lane ^ 4
+  }
+  float v = (b1 ? b[1] : b[0]) + dpp_f<kQuadXor2>(b1 ? b[0] : b[1]);
+  v += dpp_f<kQuadXor1>(v);
+  v = xor32_sum(xor16_sum(v));
+  const int e = (lane >> 1) & 7;
+  return e == 0 ? A.sv_scale * (double)v + A.sv_shift * (double)npair
+                : (e < 7 ? A.vir_scale * (double)v : (double)npair);
+}
+
 // Staging of one work item by one wave (i cluster ci, entries [e0, e1)):
 //  1. lane-parallel pruning of the chunk's entries against the current
 //     bounding boxes (D_MAX); the entries left go to LDS, compacted, counting
@@ -2061,8 +2087,14 @@ __device__ __forceinline__ void pairs_body(
       acc.fx = acc.fy = acc.fz = 0.f;
     }
     if (A.item_partials) {
-      const double o = item_row<VO>(A, acc, npair, lane);
-      if (lane < 8) A.ipart[(size_t)item * 8 + lane] = o + radd;
+      if constexpr (VO) {
+        const double o = item_row<VO>(A, acc, npair, lane);
+        if (lane < 8) A.ipart[(size_t)item * 8 + lane] = o + radd;
+      } else {
+        double o = item_row_pairs(A, acc, npair, lane);
+        if (nrec > 0) o += __shfl(radd, (lane >> 1) & 7, WAVE);
+        if (lane < 16 && !(lane & 1)) A.ipart[(size_t)item * 8 + (lane >> 1)] = o;
+      }
       acc = PairAcc{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     } else {
       // value and virial stay in the lanes' running sums over the wave's items
