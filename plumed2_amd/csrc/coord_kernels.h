@@ -1354,6 +1354,22 @@ __device__ __forceinline__ float sum_over_jj(float v) {
   v += dpp_f<kRor8>(v);
   return xor32_sum(xor16_sum(v));
 }
+// the same sum of three values at once, component jj3_component(lane) in each lane
+// (the lanes keep half of the values at the first step and of those left at the
+// second: the same additions in half of the instructions, and one store of three
+// lanes an atom; 48 systems 730 -> 715 us, 50,000 atoms 38.2 -> 37.3)
+__device__ __forceinline__ float sum_over_jj3(float x, float y, float z, int lane) {
+  const bool b3 = lane & 8;
+  const float u = (b3 ? z : x) + dpp_f<kRor8>(b3 ? x : z);
+  const float v = (b3 ? 0.f : y) + dpp_f<kRor8>(b3 ? y : 0.f);
+  // even 16-lane rows keep u, odd ones v
+  const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(u), __float_as_uint(v), false, false);
+  return xor32_sum(__uint_as_float(p[0]) + __uint_as_float(p[1]));
+}
+// 0, 1, 2 (lanes 0-7, 16-23, 8-15: one of each per atom ii); 3: no component
+__device__ __forceinline__ int jj3_component(int lane) {
+  return lane >= 32 ? 3 : ((lane & 8) ? ((lane & 16) ? 3 : 2) : (lane >> 4));
+}
 // sum over the 64 lanes, in every lane
 __device__ __forceinline__ float wave_sum_f(float v) {
   v += dpp_f<kRor8>(v);
@@ -2077,13 +2093,14 @@ __device__ __forceinline__ void pairs_body(
     if (nrec > 0)
       band_terms<P, GENERIC, TWO, VO>(A, L, ci, posI, posJ, pi, ii, jj, lane, ai, n0, b1, n1, b2, n2, fadd, radd);
     if constexpr (!VO) {
-      const float fx = sum_over_jj(acc.fx), fy = sum_over_jj(acc.fy), fz = sum_over_jj(acc.fz);
-      if (jj == 0) {
-        double* fp = fpart + (size_t)item * (CL * 3) + ii * 3;
-        fp[0] = -A.df_scale * (double)fx + fadd[0];
-        fp[1] = -A.df_scale * (double)fy + fadd[1];
-        fp[2] = -A.df_scale * (double)fz + fadd[2];
+      const float f = sum_over_jj3(acc.fx, acc.fy, acc.fz, lane);
+      const int c = jj3_component(lane);
+      double add = 0.0;
+      if (nrec > 0) {  // uniform, rare
+        const double a0 = __shfl(fadd[0], ii, WAVE), a1 = __shfl(fadd[1], ii, WAVE), a2 = __shfl(fadd[2], ii, WAVE);
+        add = c == 0 ? a0 : (c == 1 ? a1 : a2);
       }
+      if (c < 3) fpart[(size_t)item * (CL * 3) + ii * 3 + c] = -A.df_scale * (double)f + add;
       acc.fx = acc.fy = acc.fz = 0.f;
     }
     if (A.item_partials) {
@@ -3143,13 +3160,9 @@ __global__ __launch_bounds__(PAIR_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
     const float cs = sum_over_jj(acc.sv), cc = sum_over_jj((float)cnt);
     if (jj == 0) rpart[(size_t)item * CL + ii] = A.sv_scale * (double)cs + A.sv_shift * (double)cc;
     if constexpr (WT) {
-      const float fx = sum_over_jj(acc.fx), fy = sum_over_jj(acc.fy), fz = sum_over_jj(acc.fz);
-      if (jj == 0) {
-        double* fp = fpart + (size_t)item * (CL * 3) + ii * 3;
-        fp[0] = -A.df_scale * (double)fx;
-        fp[1] = -A.df_scale * (double)fy;
-        fp[2] = -A.df_scale * (double)fz;
-      }
+      const float f = sum_over_jj3(acc.fx, acc.fy, acc.fz, lane);
+      const int c = jj3_component(lane);
+      if (c < 3) fpart[(size_t)item * (CL * 3) + ii * 3 + c] = -A.df_scale * (double)f;
       float tv[6];
       tv[0] = wave_sum_f(acc.vxx);
       tv[1] = wave_sum_f(acc.vxy);
