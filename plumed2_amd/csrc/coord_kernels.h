@@ -2015,8 +2015,8 @@ constexpr int stage_cap() {
 // sums over all of the wave's items; their wave sums are taken once at the
 // end, converted to FP64 and added to the wave's band sums, and the waves'
 // rows are added in wave order.
-// Bound by VALU issue (16.1 M instructions a launch at 50,000 atoms, 18.1 M when
-// every listed entry was staged).  Known rational 6-12, 50,000 atoms: 38 us
+// Bound by VALU issue (16.5 M instructions a launch at 50,000 atoms, 18.1 M when
+// every listed entry was staged).  Known rational 6-12, 50,000 atoms: 37 us
 // (41 before); EXP, 20,000 atoms: 60 us.
 template <int P, bool GENERIC, bool TWO, bool VO, int CH>
 __device__ __forceinline__ void pairs_body(
