@@ -41,12 +41,12 @@ struct Group {
   int maxcl = 0;   // cluster capacity: n/8 + one partial cluster per column
   int ncol = 1;
   int ncl = 0;  // clusters (device total copied at rebuild)
-  // slot_loc of the last build (order_nslot slots at order_ptr) orders the
+  // slot_loc of the last build (order_nslot slots, `order`) orders the
   // atoms of the next one; 0 = no such order
   int order_nslot = 0;
-  const int* order_ptr = nullptr;
-  // col_count and fill hold zeros (k_rank leaves them so), at these addresses
-  const int *zero_count = nullptr, *zero_fill = nullptr;
+  Held order;
+  // col_count and fill hold zeros over their whole capacity (k_rank leaves them so)
+  Held zero_count, zero_fill;
   DBuf<SysArg> sys;
   DBuf<int4> info, slot_img;
   DBuf<double> key;
@@ -223,15 +223,16 @@ static int rebuild(p2a_coord* c, const double* box9, const double* pos_dev) {
     // still in slot_loc (atoms move little between builds, so a workgroup's
     // column counts stay in LDS); k_rank then writes every slot of the new
     // clusters, padding included
-    const bool use_order = G.order_nslot > 0 && G.order_ptr == G.slot_loc.p;
+    const bool use_order = G.order_nslot > 0 && G.order.of(G.slot_loc);
     const int norder = use_order ? G.order_nslot : 0;
     G.order_nslot = 0;
-    if (G.zero_count != G.col_count.p || G.zero_fill != G.fill.p) {
+    if (!G.zero_count.of(G.col_count) || !G.zero_fill.of(G.fill)) {
       const int nc = (int)G.col_count.n, nf = (int)G.fill.n;
       hipLaunchKernelGGL(k_fill_int3, dim3(std::max(1, std::min(grid1(std::max(nc, nf), 256), 1024))), dim3(256), 0, s,
                          G.col_count.p, nc, 0, G.fill.p, nf, 0, (int*)nullptr, 0, 0);
     }
-    G.zero_count = G.zero_fill = nullptr;
+    G.zero_count.drop();
+    G.zero_fill.drop();
     B.s[gi] = BinSide{G.n,     G.off,         norder,          use_order ? G.slot_loc.p : nullptr,
                       G.sys.p, G.info.p,      G.key.p,         G.col_count.p,
                       G.col_start.p, G.fill.p, G.tmp.p};
@@ -256,8 +257,8 @@ static int rebuild(p2a_coord* c, const double* box9, const double* pos_dev) {
   }
   if ((rc = launch_check("rebuild: binning"))) return rc;
   for (int gi = 0; gi < ngroups; gi++) {
-    c->g[gi].zero_count = c->g[gi].col_count.p;
-    c->g[gi].zero_fill = c->g[gi].fill.p;
+    c->g[gi].zero_count.note(c->g[gi].col_count);
+    c->g[gi].zero_fill.note(c->g[gi].fill);
   }
   // cluster counts stay on the device (totals[5 + 2 g]) until the one host
   // read below; the kernels in between are sized by the cluster capacity
@@ -315,7 +316,7 @@ static int rebuild(p2a_coord* c, const double* box9, const double* pos_dev) {
     Group& G = c->g[gi];
     G.ncl = hostT[5 + 2 * gi];
     G.order_nslot = G.ncl * CL;
-    G.order_ptr = G.slot_loc.p;
+    G.order.note(G.slot_loc);
   }
   c->max_wrap = hostT[wslot];
   c->nitems = 0;

@@ -46,6 +46,7 @@
 #include <cstring>
 #include <string>
 
+#include "dbuf.h"
 #include "fp64_math.h"
 #include "p2a_internal.h"
 #include "switch_eval.h"
@@ -61,33 +62,6 @@ namespace p2a {
 constexpr int CL = 8;           // atoms per cluster
 constexpr int WAVE = 64;
 constexpr int PAIR_BLOCK = 256; // 4 waves per workgroup
-
-template <class T>
-struct DBuf {
-  T* p = nullptr;
-  size_t n = 0;
-  int reserve(size_t m) {
-    if (m <= n && p) return P2A_OK;
-    if (p) (void)hipFree(p);
-    p = nullptr;
-    n = 0;
-    // 1/8 headroom: list sizes drift between rebuilds, and every regrowth
-    // is a hipFree (which waits for the device) plus a hipMalloc
-    size_t want = std::max<size_t>(m + m / 8, 1);
-    if (hipMalloc(&p, want * sizeof(T)) != hipSuccess) {
-      p = nullptr;
-      return fail(P2A_ERR_NOMEM, "hipMalloc of " + std::to_string(want * sizeof(T)) + " bytes failed");
-    }
-    n = want;
-    return P2A_OK;
-  }
-  DBuf() = default;
-  DBuf(const DBuf&) = delete;
-  DBuf& operator=(const DBuf&) = delete;
-  ~DBuf() {
-    if (p) (void)hipFree(p);
-  }
-};
 
 struct Entry {
   int code;
