@@ -332,9 +332,14 @@ int64_t p2a_metad_grid_size(const p2a_metad *ctx);
  * h = HEIGHT*exp(-V(c)/(kbt*(BIASFACTOR-1))) of the grid left by the previous
  * ones (MetaD::update :2377-2470, getHeight :2280-2305, addGaussian
  * :1886-1937).  centers: host [nhills][ncv]; heights: host output (may be NULL)
- * receiving the deposited Gaussian heights.  One device launch. */
+ * receiving the deposited Gaussian heights.  One launch for a few hills, else
+ * two for every 1024 / 2^ncv. */
 int p2a_metad_deposit(p2a_metad *ctx, int64_t nhills, const double *centers, double *heights);
-/* Same with device arrays; asynchronous. */
+/* Same with device arrays; asynchronous.  The first call of more than a few
+ * hills allocates a workspace of a fixed size, kept until p2a_metad_destroy; no
+ * call allocates after that, none while the stream is captured (before the
+ * workspace is there the hills then go one after the other, with the same
+ * result), and a captured call can be replayed as long as the context lives. */
 int p2a_metad_deposit_device(p2a_metad *ctx, int64_t nhills, const double *centers_dev, double *heights_dev);
 /* Add hills of given heights (HILLS restart, MetaD::readGaussians :1807-1829). */
 int p2a_metad_add_hills(p2a_metad *ctx, int64_t nhills, const double *centers, const double *heights);

@@ -534,11 +534,11 @@ __device__ __forceinline__ bool in_support(const GridArg& G, int i, int n, int i
   return d <= G.nneigh[i];
 }
 
-// hills of one epoch: their first index and count, centres and cells
+// hills of one epoch: their first index in the call and count, centres and cells
 struct Epoch {
   long long k0;
   int n;
-  const double* centers;  // of the whole call
+  const double* centers;
   const int* cells;
 };
 
@@ -561,18 +561,17 @@ __global__ __launch_bounds__(kChainThreads) void k_hill_chain(GridArg G, const d
     if (j >= N.n || r / R < j / R) return;
     double e = -1.0;
     if (j < r && r < N.n) {
-      const long long kj = N.k0 + j, kr = N.k0 + r;
       HillDim H[NCV];
       bool in = true;
 #pragma unroll
       for (int i = 0; i < NCV; i++) {
-        int n = N.cells[kr * NCV + i] + ((q >> i) & 1);
+        int n = N.cells[r * NCV + i] + ((q >> i) & 1);
         if (n >= (int)G.nbin[i]) {
           if (G.pbc[i]) n = 0;
           else in = false;
         }
-        in = in && in_support(G, i, n, N.cells[kj * NCV + i]);
-        H[i] = hill_dim<PER>(G, i, N.centers[kj * NCV + i], G.min[i] + (double)n * G.dx[i]);
+        in = in && in_support(G, i, n, N.cells[j * NCV + i]);
+        H[i] = hill_dim<PER>(G, i, N.centers[j * NCV + i], G.min[i] + (double)n * G.dx[i]);
       }
       if (in) e = hill_shape<NCV>(H);
     }
@@ -599,8 +598,8 @@ __global__ __launch_bounds__(kChainThreads) void k_hill_chain(GridArg G, const d
   if (t < E.n) {
     bool ok = true;
     for (int i = 0; i < NCV; i++) {
-      ok = ok && E.cells[(E.k0 + t) * NCV + i] >= 0;
-      sh_c[t][i] = E.centers[(E.k0 + t) * NCV + i];
+      ok = ok && E.cells[t * NCV + i] >= 0;
+      sh_c[t][i] = E.centers[t * NCV + i];
     }
     if (!ok) atomicMin(&sh_bad, t);
   }
@@ -634,7 +633,7 @@ __global__ __launch_bounds__(kChainThreads) void k_hill_chain(GridArg G, const d
 #pragma unroll
       for (int i = 0; i < NCV; i++) {
         c[i] = mine ? sh_c[r][i] : G.min[i];
-        ind[i] = mine ? E.cells[(E.k0 + r) * NCV + i] : 0;
+        ind[i] = mine ? E.cells[r * NCV + i] : 0;
         d[i] = 0.0;
       }
       K = corner_of<NCV>(G, c, ind, q);
@@ -799,8 +798,8 @@ __global__ __launch_bounds__(256) void k_hill_nodes(GridArg G, double* __restric
     hh[p] = hb[h];
 #pragma unroll
     for (int i = 0; i < NCV; i++) {
-      cell[p][i] = E.cells[(E.k0 + h) * NCV + i];
-      x[p][i] = E.centers[(E.k0 + h) * NCV + i];
+      cell[p][i] = E.cells[h * NCV + i];
+      x[p][i] = E.centers[h * NCV + i];
     }
   }
   int l[NCV];
@@ -1080,13 +1079,14 @@ struct p2a_metad {
   int* err = nullptr;
   double* scratch = nullptr;  // staging for host-array entry points
   size_t scratch_n = 0;
-  // workspace of the deposition in epochs: cells of the hills, shapes of two
-  // epochs, heights of two epochs, two epochs' counts
-  int* cells = nullptr;
-  size_t cells_n = 0;
-  double* shapes = nullptr;  // one block: shapes, then hbuf, then state
+  // workspace of the deposition in epochs, one block of a fixed size, kept until
+  // the context goes (a captured deposition holds its address): shapes of two
+  // epochs, heights of two epochs, two epochs' counts, cells of the hills of
+  // kCellEpochs epochs and the next
+  double* shapes = nullptr;
   double* hbuf = nullptr;
   int* state = nullptr;
+  int* cells = nullptr;
   bool first_step = true;
 };
 
@@ -1102,37 +1102,28 @@ static int metad_scratch(p2a_metad* m, size_t n) {
   return P2A_OK;
 }
 
-// The workspace of the deposition in epochs for nhills hills; false when it
-// cannot be had (memory, or a stream under capture, where nothing may be
-// allocated): the hills then go one after the other.
-static bool epoch_workspace(p2a_metad* m, size_t nhills) {
-  const size_t want = nhills * m->G.ncv;
-  const bool ready = m->shapes && m->cells_n >= want;
-  if (ready) return true;
+// The workspace of the deposition in epochs; false when it cannot be had
+// (memory, or a stream under capture, where nothing may be allocated): the
+// hills then go one after the other.
+constexpr int kCellEpochs = 64;
+static bool epoch_workspace(p2a_metad* m) {
+  if (m->shapes) return true;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(m->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
     (void)hipGetLastError();
     return false;
   }
   const size_t eh = kChainThreads >> m->G.ncv;
-  auto get = [](void** p, size_t bytes) {
-    if (*p) return true;
-    if (hipMalloc(p, bytes) == hipSuccess) return true;
-    *p = nullptr;
+  const size_t nshape = 2 * eh * kChainThreads, nheight = 2 * eh;
+  const size_t ncell = (kCellEpochs + 1) * eh * m->G.ncv;
+  if (hipMalloc((void**)&m->shapes, (nshape + nheight) * sizeof(double) + (4 + ncell) * sizeof(int)) != hipSuccess) {
+    m->shapes = nullptr;
     (void)hipGetLastError();
     return false;
-  };
-  if (m->cells_n < want) {
-    if (m->cells) (void)hipFree(m->cells);
-    m->cells = nullptr;
-    m->cells_n = 0;
-    if (!get((void**)&m->cells, want * sizeof(int))) return false;
-    m->cells_n = want;
   }
-  const size_t nshape = 2 * eh * kChainThreads, nheight = 2 * eh;
-  if (!get((void**)&m->shapes, (nshape + nheight) * sizeof(double) + 4 * sizeof(int))) return false;
   m->hbuf = m->shapes + nshape;
   m->state = (int*)(m->hbuf + nheight);
+  m->cells = m->state + 4;
   return true;
 }
 
@@ -1149,13 +1140,23 @@ static void deposit_epochs(p2a_metad* m, int64_t nhills, const double* centers, 
   hipStream_t s = m->stream;
   long long tiles = 1;
   for (int i = 0; i < NCV; i++) tiles *= (G.nbin[i] + tile_dim<NCV>(i) - 1) / tile_dim<NCV>(i);
-  hipLaunchKernelGGL(k_hill_cells<NCV>, dim3((unsigned)((nhills + 255) / 256)), dim3(256), 0, s, G,
-                     (long long)nhills, centers, m->cells);
   const int64_t ne = (nhills + EH - 1) / EH;
+  int64_t e0 = 0;  // the epoch whose cells come first in the workspace
+  auto epoch = [&](int64_t e) {
+    const bool has = e >= 0 && e < ne;
+    return Epoch{has ? e * EH : 0, has ? (int)std::min<int64_t>(EH, nhills - e * EH) : 0,
+                 has ? centers + e * EH * NCV : centers, has ? m->cells + (e - e0) * EH * NCV : m->cells};
+  };
   // launch e finds the heights of epoch e and the shapes of epoch e + 1; e = -1: shapes only
   for (int64_t e = -1; e < ne; e++) {
-    Epoch E = {e < 0 ? 0 : e * EH, e < 0 ? 0 : (int)std::min<int64_t>(EH, nhills - e * EH), centers, m->cells};
-    Epoch N = {(e + 1) * EH, e + 1 < ne ? (int)std::min<int64_t>(EH, nhills - (e + 1) * EH) : 0, centers, m->cells};
+    if (e < 0 || (e > 0 && e % kCellEpochs == 0)) {
+      // the cells of this epoch, the kCellEpochs - 1 after it and the next one
+      e0 = std::max<int64_t>(e, 0);
+      const int64_t nc = std::min<int64_t>((kCellEpochs + 1) * EH, nhills - e0 * EH);
+      hipLaunchKernelGGL(k_hill_cells<NCV>, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, s, G, (long long)nc,
+                         centers + e0 * EH * NCV, m->cells);
+    }
+    const Epoch E = epoch(e), N = epoch(e + 1);
     const int rows = G.welltemp ? N.n : 0;
     if (E.n == 0 && rows == 0) continue;
     const size_t half = (size_t)EH * kChainThreads;
@@ -1267,7 +1268,6 @@ int p2a_metad_destroy(p2a_metad* m) {
   if (m->der) (void)hipFree(m->der);
   if (m->err) (void)hipFree(m->err);
   if (m->scratch) (void)hipFree(m->scratch);
-  if (m->cells) (void)hipFree(m->cells);
   if (m->shapes) (void)hipFree(m->shapes);
   if (m->own_stream) (void)hipStreamDestroy(m->own_stream);
   delete m;
@@ -1293,7 +1293,7 @@ int p2a_metad_deposit_device(p2a_metad* m, int64_t nhills, const double* centers
   // unless a periodic support is wider than the grid (a node would count
   // twice) or the grid's tiles exceed a launch.
   const bool epochs = nhills > kSeqHills && !G.may_alias && m->size < ((size_t)1 << 36) &&
-                      epoch_workspace(m, (size_t)nhills);
+                      epoch_workspace(m);
   bool per = false;
   for (int i = 0; i < G.ncv; i++) per = per || G.pbc[i];
 #define P2A_DEP(N)                                                       \
