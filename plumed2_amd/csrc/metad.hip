@@ -760,9 +760,20 @@ __host__ __device__ constexpr int tile_dim(int i) {
 // to the addition, while the other waves tabulate the next hills.  Bound by
 // wave 0's walk through the hills of the busiest tiles.  Tiles that no hill
 // reaches leave after the list.
+// The workgroups are the tiles of the grid or, where that is fewer, `per` tiles
+// around each hill, of which the first hill that reaches a tile takes it: the
+// launch then follows the supports, not the grid.  A host call with 5 hills on
+// 90^4 nodes: 2,760 us over all tiles, their nodes read at once, now 71 (4 hills
+// one after the other: 450); on 8,000 x 8,000 nodes 1,100 -> 52, with 512 hills
+// 2,320 -> 328.
+struct TileMap {
+  int per;         // 0: the tiles of the grid
+  int early;       // nodes read before it is known whether a hill reaches the tile
+  int n[kMaxCv];   // tiles along each CV that a hill's support can reach
+};
 template <int NCV, bool PER>
 __global__ __launch_bounds__(256) void k_hill_nodes(GridArg G, double* __restrict__ val, double* __restrict__ der,
-                                                    Epoch E, const int* __restrict__ state,
+                                                    Epoch E, TileMap M, const int* __restrict__ state,
                                                     const double* __restrict__ hbuf) {
   constexpr int EH = kChainThreads >> NCV;
   constexpr int ST = NCV == 1 ? 64 : NCV == 2 ? 16 : 12;  // sum of the tile's sides
@@ -771,25 +782,42 @@ __global__ __launch_bounds__(256) void k_hill_nodes(GridArg G, double* __restric
   // the hills that reach the tile, in order: cell, centre, height
   __shared__ int lcell[EH][NCV];
   __shared__ double lx[EH][NCV], lh[EH];
-  __shared__ int wcnt[4];
+  constexpr int HP = (EH + 255) / 256;
+  __shared__ int2 whit[HP][4];  // a wave's hits and the first of them
   __shared__ double2 tsf[2][CH][ST];
   __shared__ double tw[2][CH][ST];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   const int par = (int)((E.k0 / EH) & 1);
   const double* hb = hbuf + (size_t)par * EH;
-  int o[NCV];
-  {
-    long long b = blockIdx.x;
+  const int cnt = state[par];
+  int o[NCV], owner = 0;
+  if (M.per == 0) {
+    unsigned b = blockIdx.x;
 #pragma unroll
     for (int i = 0; i < NCV; i++) {
-      const int nt = ((int)G.nbin[i] + tile_dim<NCV>(i) - 1) / tile_dim<NCV>(i);
+      const unsigned nt = (G.nbin[i] + tile_dim<NCV>(i) - 1) / tile_dim<NCV>(i);
       o[i] = (int)(b % nt) * tile_dim<NCV>(i);
       b /= nt;
     }
+  } else {
+    owner = (int)(blockIdx.x / (unsigned)M.per);
+    if (owner >= cnt) return;  // uniform, as the returns below
+    unsigned b = blockIdx.x % (unsigned)M.per;
+#pragma unroll
+    for (int i = 0; i < NCV; i++) {
+      const int N = (int)G.nbin[i], nt = (int)((G.nbin[i] + tile_dim<NCV>(i) - 1) / tile_dim<NCV>(i));
+      int a = E.cells[owner * NCV + i] - G.nneigh[i];  // the support's first node
+      if (a < 0) a = G.pbc[i] ? a + N : 0;
+      int q = a / tile_dim<NCV>(i) + (int)(b % (unsigned)M.n[i]);
+      if (q >= nt) {
+        if (!G.pbc[i]) return;
+        q -= nt;
+      }
+      o[i] = q * tile_dim<NCV>(i);
+      b /= (unsigned)M.n[i];
+    }
   }
-  // everything the tile may need from memory goes out before the first wait:
-  // the epoch's hills (E.n of them, valid or not), their count, wave 0's node
-  constexpr int HP = (EH + 255) / 256;
+  // the epoch's hills (E.n of them, valid or not)
   int cell[HP][NCV];
   double x[HP][NCV], hh[HP];
 #pragma unroll
@@ -820,19 +848,22 @@ __global__ __launch_bounds__(256) void k_hill_nodes(GridArg G, double* __restric
 #pragma unroll
     for (int i = NCV - 1; i > 0; --i) node = node * G.nbin[i - 1] + n[i - 1];
   }
+  // wave 0's node: on its way while the list is made, or while the tables are formed
   double v = 0.0, d[NCV];
 #pragma unroll
   for (int i = 0; i < NCV; i++) d[i] = 0.0;
-  if (valid) {
+  auto load = [&]() {
+    if (!valid) return;
     v = val[node];
 #pragma unroll
     for (int i = 0; i < NCV; i++) d[i] = der[node * NCV + i];
-  }
-  const int cnt = state[par];
-  int nl = 0;
+  };
+  if (M.early) load();
+  bool hit[HP];
+  int below[HP];  // hits of this wave before this lane's
 #pragma unroll
   for (int p = 0; p < HP; p++) {
-    bool hit = p * 256 + t < cnt;
+    hit[p] = p * 256 + t < cnt;
 #pragma unroll
     for (int i = 0; i < NCV; i++) {
       const int T = min(tile_dim<NCV>(i), (int)G.nbin[i] - o[i]);
@@ -841,31 +872,40 @@ __global__ __launch_bounds__(256) void k_hill_nodes(GridArg G, double* __restric
         const int N = (int)G.nbin[i];
         if (s < 0) s += N;  // |o - cell| < N and the support is no wider than the grid
         else if (s >= N) s -= N;
-        hit = hit && (s <= 2 * G.nneigh[i] || s + T - 1 >= N);
+        hit[p] = hit[p] && (s <= 2 * G.nneigh[i] || s + T - 1 >= N);
       } else {
-        hit = hit && s <= 2 * G.nneigh[i] && s + T - 1 >= 0;
+        hit[p] = hit[p] && s <= 2 * G.nneigh[i] && s + T - 1 >= 0;
       }
     }
-    const unsigned long long m = __ballot(hit);
-    if (lane == 0) wcnt[w] = __popcll(m);
-    __syncthreads();
-    int at = nl;
-    for (int q = 0; q < 4; q++) {
-      if (q < w) at += wcnt[q];
-      nl += wcnt[q];
-    }
-    if (hit) {
-      at += __popcll(m & ((1ull << lane) - 1));
-      lh[at] = hh[p];
-#pragma unroll
-      for (int i = 0; i < NCV; i++) {
-        lcell[at][i] = cell[p][i];
-        lx[at][i] = x[p][i];
-      }
-    }
-    __syncthreads();
+    const unsigned long long m = __ballot(hit[p]);
+    below[p] = __popcll(m & ((1ull << lane) - 1));
+    if (lane == 0) whit[p][w] = make_int2(__popcll(m), m ? p * 256 + w * WAVE_M + __ffsll((long long)m) - 1 : INT_MAX);
   }
-  if (nl == 0) return;
+  __syncthreads();
+  int nl = 0, first = INT_MAX;
+#pragma unroll
+  for (int p = 0; p < HP; p++)
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int2 h = whit[p][q];
+      if (q == w) below[p] += nl;
+      nl += h.x;
+      first = min(first, h.y);
+    }
+  if (nl == 0 || (M.per && first != owner)) return;
+#pragma unroll
+  for (int p = 0; p < HP; p++) {
+    if (!hit[p]) continue;
+    const int at = below[p];
+    lh[at] = hh[p];
+#pragma unroll
+    for (int i = 0; i < NCV; i++) {
+      lcell[at][i] = cell[p][i];
+      lx[at][i] = x[p][i];
+    }
+  }
+  __syncthreads();
+  if (!M.early) load();
   // the tables of the hills [c0, c0 + CH) of the list, by threads q0, q0 + step, ...
   auto tabulate = [&](int c0, int buf, int q0, int step) {
     const int nc = min(CH, nl - c0);
@@ -1133,13 +1173,43 @@ static void deposit_seq(p2a_metad* m, int64_t nhills, const double* centers, dou
                      (long long)nhills, centers, heights, m->err);
 }
 
+// Tiles of the grid, and around a hill (M, per): a run of 2 nneigh + 1 nodes
+// reaches (2 nneigh + T - 1) / T + 1 tiles of T nodes, and one more where it wraps
+// over a last tile that is cut short.
+struct TileCount {
+  int64_t grid = 1, per = 1;
+  TileMap M;
+  // workgroups of an epoch of n hills; work-items have a 32-bit count (kMaxTiles)
+  int64_t launch(int n) const { return by_hill(n) ? per * n : grid; }
+  // a workgroup around a hill costs somewhat more than a tile that no hill
+  // reaches (512 hills on 3,000 x 3,000 periodic nodes: 135,424 around the hills
+  // 690-713 us, 140,625 tiles 607)
+  bool by_hill(int n) const { return per * n * 5 < grid * 4; }
+};
+constexpr int64_t kMaxTiles = (1 << 24) - 1;
+// Up to this many tiles (a few rounds of what the chip holds) the nodes are read
+// early: a round's latency counts, not the bytes (4,000 hills on 513 x 513 nodes,
+// 4,225 tiles: 1,688 us, read late 1,705).
+constexpr int64_t kEarlyTiles = 16384;
+template <int NCV>
+static TileCount count_tiles(const GridArg& G) {
+  TileCount C;
+  std::memset(&C.M, 0, sizeof(C.M));
+  for (int i = 0; i < NCV; i++) {
+    const int64_t T = tile_dim<NCV>(i), nt = (G.nbin[i] + T - 1) / T;
+    C.M.n[i] = (int)std::min(nt, (2 * (int64_t)G.nneigh[i] + T - 1) / T + 1 + (G.pbc[i] && G.nbin[i] % T ? 1 : 0));
+    C.grid *= nt;
+    C.per *= C.M.n[i];
+  }
+  return C;
+}
+
 template <int NCV, bool PER>
-static void deposit_epochs(p2a_metad* m, int64_t nhills, const double* centers, double* heights) {
+static void deposit_epochs(p2a_metad* m, const TileCount& tiles, int64_t nhills, const double* centers,
+                           double* heights) {
   constexpr int EH = kChainThreads >> NCV;
   const GridArg& G = m->G;
   hipStream_t s = m->stream;
-  long long tiles = 1;
-  for (int i = 0; i < NCV; i++) tiles *= (G.nbin[i] + tile_dim<NCV>(i) - 1) / tile_dim<NCV>(i);
   const int64_t ne = (nhills + EH - 1) / EH;
   int64_t e0 = 0;  // the epoch whose cells come first in the workspace
   auto epoch = [&](int64_t e) {
@@ -1163,9 +1233,13 @@ static void deposit_epochs(p2a_metad* m, int64_t nhills, const double* centers, 
     hipLaunchKernelGGL((k_hill_chain<NCV, PER>), dim3(1 + rows), dim3(kChainThreads), 0, s, G, m->val, m->der, E,
                        m->shapes + (e & 1) * half, N, m->shapes + ((e + 1) & 1) * half, e == 0 ? 1 : 0, m->state,
                        m->hbuf, heights, m->err);
-    if (E.n > 0)
-      hipLaunchKernelGGL((k_hill_nodes<NCV, PER>), dim3((unsigned)tiles), dim3(256), 0, s, G, m->val, m->der, E, m->state,
-                         m->hbuf);
+    if (E.n > 0) {
+      TileMap M = tiles.M;
+      M.per = tiles.by_hill(E.n) ? (int)tiles.per : 0;
+      M.early = !M.per && tiles.grid <= kEarlyTiles;
+      hipLaunchKernelGGL((k_hill_nodes<NCV, PER>), dim3((unsigned)tiles.launch(E.n)), dim3(256), 0, s, G, m->val,
+                         m->der, E, M, m->state, m->hbuf);
+    }
   }
 }
 
@@ -1291,16 +1365,18 @@ int p2a_metad_deposit_device(p2a_metad* m, int64_t nhills, const double* centers
   // A few hills: one workgroup, one launch (a host call with 1 / 2 hills takes
   // 41 / 44 us, in epochs 51 us for 3 and 53 us for 8).  More: in epochs,
   // unless a periodic support is wider than the grid (a node would count
-  // twice) or the grid's tiles exceed a launch.
-  const bool epochs = nhills > kSeqHills && !G.may_alias && m->size < ((size_t)1 << 36) &&
-                      epoch_workspace(m);
+  // twice) or the tiles exceed a launch.
+  const bool some = nhills > kSeqHills && !G.may_alias;
   bool per = false;
   for (int i = 0; i < G.ncv; i++) per = per || G.pbc[i];
-#define P2A_DEP(N)                                                       \
-  do {                                                                   \
-    if (epochs && per) deposit_epochs<N, true>(m, nhills, centers_dev, heights_dev); \
-    else if (epochs) deposit_epochs<N, false>(m, nhills, centers_dev, heights_dev);  \
-    else deposit_seq<N>(m, nhills, centers_dev, heights_dev);            \
+#define P2A_DEP(N)                                                                         \
+  do {                                                                                     \
+    const TileCount tiles = count_tiles<N>(G);                                             \
+    const int most = (int)std::min<int64_t>(nhills, kChainThreads >> N);                   \
+    const bool epochs = some && tiles.launch(most) <= kMaxTiles && epoch_workspace(m);     \
+    if (epochs && per) deposit_epochs<N, true>(m, tiles, nhills, centers_dev, heights_dev); \
+    else if (epochs) deposit_epochs<N, false>(m, tiles, nhills, centers_dev, heights_dev); \
+    else deposit_seq<N>(m, nhills, centers_dev, heights_dev);                              \
   } while (0)
   if (G.ncv == 1) P2A_DEP(1);
   else if (G.ncv == 2) P2A_DEP(2);
