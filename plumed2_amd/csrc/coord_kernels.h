@@ -1352,6 +1352,10 @@ __device__ __forceinline__ float wave_sum_f(float v) {
   v += dpp_f<kRor1>(v);
   return xor32_sum(xor16_sum(v));
 }
+// value of lane l (uniform)
+__device__ __forceinline__ float readlane_f(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
 // number of set bits of m in the lanes below this one (v_mbcnt)
 __device__ __forceinline__ int bits_below(unsigned long long m) {
   return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
@@ -1832,12 +1836,21 @@ __device__ __forceinline__ double item_row_pairs(const PairArgs& A, const PairAc
 // a margin over D_MAX) takes one lane per entry, eight loads in flight at once:
 // the same order; 48 systems, list radius 1.2 = D_MAX: 759 us, in rounds 803.
 constexpr int kDenseEntries = 40;
+// TWIN (rounds only): also the staged slot of each i atom's twin, the same atom in
+// the other group, for staged atoms that do not carry their requested index.
 // Returns the group bounds (uniform): n0 (0 or 8), [b1, b1+n1), [b2, b2+n2).
-template <bool VO, bool DENSE, int CH>
+struct Twin {
+  const float4* idxJ;  // packed positions with requested indices
+  int ai;              // requested index of this lane's i atom in the other group, or -2
+  float4 pi;           // its position
+  int slot;            // out: staged slot of its twin, -1: not in the item
+};
+template <bool VO, bool DENSE, int CH, bool TWIN = false>
 __device__ __forceinline__ void stage_item(const PairArgs& A, const Entry& my, int lane, int e0, int e1, int ci,
                                            const float4& ic, const float4& ih, const float4* __restrict__ posJ,
                                            const float4* __restrict__ bbJ, const WaveLds& L, int& n0, int& b1,
-                                           int& n1, int& b2, int& n2) {
+                                           int& n1, int& b2, int& n2, Twin* T = nullptr) {
+  static_assert(!(DENSE && TWIN), "twins are found in the rounds");
   bool pass = false;
   const Entry none = {0, 1.0e5f, 1.0e5f, 1.0e5f};
   L.se[lane] = none;
@@ -1919,7 +1932,17 @@ __device__ __forceinline__ void stage_item(const PairArgs& A, const Entry& my, i
   auto load = [&](const Entry& e) {
     return *(const float4*)((const char*)posJ + (size_t)(((unsigned)e.code << 7) | t16));
   };
-  auto keep_atom = [&](const Entry& e, float4 q) {
+  // the same atom's requested index
+  auto load_idx = [&](const Entry& e) {
+    return *(const int*)((const char*)T->idxJ + (size_t)(((unsigned)e.code << 7) | t16) + 12);
+  };
+  int tw[CL];
+  if constexpr (TWIN) {
+    T->slot = -1;
+#pragma unroll
+    for (int u = 0; u < CL; u++) tw[u] = __builtin_amdgcn_readlane(T->ai, u);
+  }
+  auto keep_atom = [&](const Entry& e, float4 q, int idx) {
     q.x += e.dx;
     q.y += e.dy;
     q.z += e.dz;
@@ -1929,28 +1952,45 @@ __device__ __forceinline__ void stage_item(const PairArgs& A, const Entry& my, i
     const bool keep = fmaf(gz, gz, fmaf(gx, gx, gy * gy)) <= A.prune2;
     const unsigned long long m = __ballot(keep);
     if (keep) L.sj[at + bits_below(m)] = q;
+    if constexpr (TWIN) {
+      bool any = false;
+#pragma unroll
+      for (int u = 0; u < CL; u++) any = any || idx == tw[u];
+      for (unsigned long long f = __ballot(keep && any); f; f &= f - 1) {
+        const int l = __builtin_ctzll(f);
+        const float4 ql = make_float4(readlane_f(q.x, l), readlane_f(q.y, l), readlane_f(q.z, l), 0.f);
+        float dx, dy, dz;
+        // (not one of its images, which lie beyond D_MAX)
+        if (T->ai == __builtin_amdgcn_readlane(idx, l) && pair_d(ql, T->pi, dx, dy, dz) <= A.dmax2)
+          T->slot = at + __popcll(m & ((1ull << l) - 1));
+      }
+    }
     at += __popcll(m);
   };
   if (rounds > 0) {
     Entry ea = se[0], eb = se[CL];
     float4 va = load(ea), vb = load(eb);
+    int xa = 0, xb = 0;
+    if constexpr (TWIN) xa = load_idx(ea), xb = load_idx(eb);
     for (int r = 0; r < rounds; r += 2) {
       const Entry qa = ea, qb = eb;
       const float4 wa = va, wb = vb;
+      const int ja = xa, jb = xb;
       ea = se[(r + 2) * CL];
       eb = se[(r + 3) * CL];
       va = load(ea);
       vb = load(eb);
+      if constexpr (TWIN) xa = load_idx(ea), xb = load_idx(eb);
       if (r == r1) {
         pad();
         n1 = at - b1;
       }
-      keep_atom(qa, wa);
+      keep_atom(qa, wa, ja);
       if (r + 1 == r1) {
         pad();
         n1 = at - b1;
       }
-      keep_atom(qb, wb);
+      keep_atom(qb, wb, jb);
     }
   }
   if (rounds == r1 && (rounds & 1) == 0) {
@@ -2969,7 +3009,11 @@ struct PairTuning {
 // sums.  With weights the staged atoms carry their weight where the others
 // carry their requested index (packed positions pwI / pwJ), which the rare band
 // pair then finds by going through the item's rounds again: a third array in
-// LDS would cost a quarter of the resident waves.
+// LDS would cost a quarter of the resident waves.  In groups that share atoms the
+// staging notes where each i atom's twin went (Twin): one register a lane, and one
+// comparison a pair (3,000 rows in an environment of 30,000 that holds them,
+// D_MAX 1.2: a call with weights 131 us, groups apart 121; with the index looked
+// for at every pair inside D_MAX 1,855).
 // Outputs: rpart[item][8] (row sums of the i atoms), and with WT fpart
 // [item][8][3] and per-workgroup rows (0, six box-derivative products, 0).
 // 30,000 atoms, WT: 33 us (46 with the weights and indices in LDS arrays of their
@@ -3017,6 +3061,7 @@ __device__ int staged_index(const PairArgs& A, const WaveLds& L, int p, int n0, 
 // per-item constants of the row kernel
 struct RowItem {
   int ci, n0, reqi;
+  int twin;            // staged slot of this lane's i atom in the other group (TWO, WT)
   float4 ic, ih;
   const float4* idxJ;  // packed positions with requested indices
   const PbcArg* pbc;
@@ -3030,18 +3075,10 @@ __device__ __forceinline__ void row_term(const PairArgs& A, const RowItem& I, co
   const float r2 = pair_d(pj, pi, dx, dy, dz);
   bool keep = r2 >= A.contact2;
   if constexpr (KIND == 0) keep = keep && jj != ii;
-  if constexpr (TWO && !WT) keep = keep && (__float_as_int(pj.w) != ai);
+  if constexpr (TWO) keep = keep && (WT ? g + jj != I.twin : __float_as_int(pj.w) != ai);
   const float t = r2 - A.dmax2;
   const unsigned long long bm = __ballot(keep && fabsf(t) < A.band);
   bool cut = keep && t <= 0.f;
-  if constexpr (TWO && WT) {
-    // (rare groups that share atoms: the index decides each pair inside)
-    for (unsigned long long m = __ballot(cut) | bm; m; m &= m - 1) {
-      const int l = __builtin_ctzll(m);
-      const int reqj = staged_index<CH>(A, L, g + (l >> 3), I.n0, I.ci, lane, I.ic, I.ih, I.idxJ);
-      if (lane == l && reqj == ai) cut = keep = false;
-    }
-  }
   if (bm != 0ull) {  // uniform, rare
     for (unsigned long long m = bm; m; m &= m - 1) {
       const int l = __builtin_ctzll(m);
@@ -3116,7 +3153,10 @@ __global__ __launch_bounds__(PAIR_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
     Entry my_e = {0, 0.f, 0.f, 0.f};
     if (lane < CH && it.y + lane < e1) my_e = ents[it.y + lane];
     int n0, b1, n1, b2, n2;
-    stage_item<false, false, CH>(A, my_e, lane, it.y, e1, ci, I.ic, I.ih, WT ? pwJ : posJ, bbJ, L, n0, b1, n1, b2, n2);
+    Twin T = {posJ, ai, pi, -1};
+    stage_item<false, false, CH, TWO && WT>(A, my_e, lane, it.y, e1, ci, I.ic, I.ih, WT ? pwJ : posJ, bbJ, L, n0, b1,
+                                            n1, b2, n2, &T);
+    I.twin = T.slot;
     n1 = __builtin_amdgcn_readfirstlane(n1);
     n2 = __builtin_amdgcn_readfirstlane(n2);
     b1 = __builtin_amdgcn_readfirstlane(b1);
