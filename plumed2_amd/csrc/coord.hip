@@ -917,16 +917,15 @@ static void collect_profile(p2a_coord* c) {
 // COORDINATIONNUMBER rows: cn[k] = sum over env atoms j of the contact
 // matrix element of (rows[k], j), ContactMatrix::calculateWeight
 // (src/adjmat/ContactMatrix.h:95-121): nothing when |r|^2 < DBL_EPSILON (the
-// diagonal, or two atoms at one place), s(r) zeroed below DBL_EPSILON.  One
-// wave per row, FP64, the environment over the lanes (a row meets every
-// environment atom, so one thread per row left the chip idle for any but the
-// longest lists).  An index outside [0, natoms) makes that row NaN instead of
-// being read.
+// diagonal, or two atoms at one place), s(r) zeroed below DBL_EPSILON.  FP64,
+// WIDE: a wave per row, the environment over its lanes; else a thread per row.  An
+// index outside [0, natoms) makes that row NaN instead of being read.
+template <bool WIDE>
 __global__ __launch_bounds__(256) void k_cn_rows(int natoms, int nrows, const int* __restrict__ rows, int nenv,
                                                  const int* __restrict__ env, int use_pbc, PbcArg P, p2a_switch sw,
                                                  const double* __restrict__ pos, double* __restrict__ cn) {
-  const int lane = threadIdx.x & 63;
-  const int k = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int lane = WIDE ? threadIdx.x & 63 : 0;
+  const int k = WIDE ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= nrows) return;
   const int i = rows[k];
   if (i < 0 || i >= natoms) {
@@ -935,7 +934,7 @@ __global__ __launch_bounds__(256) void k_cn_rows(int natoms, int nrows, const in
   }
   const double* xi = pos + 3 * (size_t)i;
   double sum = 0.0;
-  for (int q = lane; q < nenv; q += WAVE) {
+  for (int q = lane; q < nenv; q += WIDE ? WAVE : 1) {
     const int j = env[q];
     if (j < 0 || j >= natoms) {
       sum = __builtin_nan("");
@@ -952,8 +951,24 @@ __global__ __launch_bounds__(256) void k_cn_rows(int natoms, int nrows, const in
     if (v < DBL_EPSILON) continue;
     sum += v;
   }
-  sum = wave_sum_d(sum);
+  if constexpr (WIDE) sum = wave_sum_d(sum);
   if (lane == 0) cn[k] = sum;
+}
+
+// A thread per row takes about 0.5 us an environment atom while the rows do not
+// fill the chip, a wave per row about 0.5 us a thousand rows while its lanes hold
+// the environment: a thread per row from 1,000 rows an environment atom on, and
+// for rows that fill the chip as threads (a row's environment is then read by
+// all lanes together).  Thread / wave: 16,000 rows x 16 atoms 12 / 11 us, 100,000 x
+// 64 36 / 51, 500,000 x 1 7 / 266, 500,000 x 256 314 / 542, 4,000 x 256 153 / 8.
+static void launch_cn_rows(hipStream_t s, int natoms, int nrows, const int* rows, int nenv, const int* env,
+                           int use_pbc, const PbcArg& P, const p2a_switch& sw, const double* pos, double* cn) {
+  if (nrows >= (1 << 18) || nrows >= 1000 * (int64_t)nenv)
+    hipLaunchKernelGGL(k_cn_rows<false>, dim3(grid1((size_t)nrows, 256)), dim3(256), 0, s, natoms, nrows, rows, nenv,
+                       env, use_pbc, P, sw, pos, cn);
+  else
+    hipLaunchKernelGGL(k_cn_rows<true>, dim3(grid1((size_t)nrows, 4)), dim3(256), 0, s, natoms, nrows, rows, nenv,
+                       env, use_pbc, P, sw, pos, cn);
 }
 
 // Scratch of the allocation-free entry point: the per-workgroup partials of
@@ -1327,9 +1342,8 @@ int p2a_coord_rows_device(p2a_coord* c, int64_t step, const double* box9, const 
     P2A_HIP(hipMemcpyAsync(c->cn_rows.p, r.data(), na * sizeof(int), hipMemcpyHostToDevice, c->stream));
     P2A_HIP(hipMemcpyAsync(c->cn_env.p, e.data(), nenv * sizeof(int), hipMemcpyHostToDevice, c->stream));
     if ((rc = upload_pbc(c, box9))) return rc;
-    hipLaunchKernelGGL(k_cn_rows, dim3(grid1((size_t)na, 4)), dim3(256), 0, c->stream, c->natoms, na,
-                       (const int*)c->cn_rows.p, nenv, (const int*)c->cn_env.p, c->spec.pbc ? 1 : 0, c->pbc_stage,
-                       c->spec.sw, pos_dev, rows_dev);
+    launch_cn_rows(c->stream, c->natoms, na, c->cn_rows.p, nenv, c->cn_env.p, c->spec.pbc ? 1 : 0, c->pbc_stage,
+                   c->spec.sw, pos_dev, rows_dev);
     // the host vectors are read by the copies above before they return
     P2A_HIP(hipStreamSynchronize(c->stream));
     return launch_check("coordination numbers");
@@ -1355,8 +1369,8 @@ int p2a_coordination_numbers_device(void* stream, const p2a_switch* sw, const do
     pbc_setup(box9, h);
     fill_pbc_arg(h, P);
   }
-  hipLaunchKernelGGL(k_cn_rows, dim3(grid1((size_t)nrows, 4)), dim3(256), 0, (hipStream_t)stream, (int)natoms,
-                     (int)nrows, rows_dev, (int)nenv, env_dev, use_pbc ? 1 : 0, P, *sw, pos_dev, cn_dev);
+  launch_cn_rows((hipStream_t)stream, (int)natoms, (int)nrows, rows_dev, (int)nenv, env_dev, use_pbc ? 1 : 0, P, *sw,
+                 pos_dev, cn_dev);
   return launch_check("coordination numbers");
 }
 
