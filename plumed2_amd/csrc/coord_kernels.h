@@ -3282,8 +3282,9 @@ inline int switch_known_kind(const p2a_switch& sw) {
 // caller may have two groups that share atoms (else the kernels that compare
 // atom indices are not compiled); distinct groups run the kernels of one group.
 // The other switches have a kernel of their own for the default work items
-// with derivatives (20,000 atoms with EXP: pair pass 105 -> 62 us); value only and 32 entries
-// an item run the kernel that takes any switch.
+// (20,000 atoms with EXP: pair pass with derivatives 105 -> 62 us; value only,
+// 400,000 atoms, D_MAX 0.8: EXP 275 -> 137 us, TANH 472 -> 338); 32 entries an item
+// run the kernel that takes any switch.
 template <bool TWOG>
 inline void launch_pairs(const PairArgs& A, const Two<PairSide>& T, hipStream_t s, bool value_only, int chunk) {
   const p2a_switch& sw = A.sw;
@@ -3310,9 +3311,14 @@ inline void launch_pairs(const PairArgs& A, const Two<PairSide>& T, hipStream_t 
 #define P2A_KKN(K)                                              \
   case K:                                                       \
     if constexpr (TWOG) {                                       \
-      if (A.share) { P2A_K(K, true, true, false, 64); break; }  \
+      if (A.share) {                                            \
+        if (value_only) P2A_K(K, true, true, true, 64);         \
+        else P2A_K(K, true, true, false, 64);                   \
+        break;                                                  \
+      }                                                         \
     }                                                           \
-    P2A_K(K, true, false, false, 64);                           \
+    if (value_only) P2A_K(K, true, false, true, 64);            \
+    else P2A_K(K, true, false, false, 64);                      \
     break
   if (sw.type == P2A_SW_RATIONAL_FIXED) {
     switch (sw.nn / 2) {
@@ -3326,7 +3332,7 @@ inline void launch_pairs(const PairArgs& A, const Two<PairSide>& T, hipStream_t 
     }
     return;
   }
-  const int kind = value_only || chunk != 64 ? 0 : switch_known_kind(sw);
+  const int kind = chunk != 64 ? 0 : switch_known_kind(sw);
   switch (kind) {
     P2A_KKN(kSwFastRational);
     P2A_KKN(P2A_SW_RATIONAL);
