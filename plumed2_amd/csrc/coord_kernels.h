@@ -1829,13 +1829,14 @@ __device__ __forceinline__ double item_row_pairs(const PairArgs& A, const PairAc
 //     with far-away atoms, so that every group of 8 has one kind.
 // A list radius above D_MAX leaves about half of the entries: 5-6 rounds,
 // where one lane per listed entry took 8 loads and tests an item, each load 64
-// lines.  The slots of se without an entry hold one that lies far away (atoms of
-// cluster 0, no lane is switched off); rounds go by two, the next two's loads
-// in flight.
+// lines.  The slots of se without an entry hold kNoEntry (their lanes load atoms of
+// cluster 0 and keep none, whatever these hold); rounds go by two, the next two's
+// loads in flight.
 // DENSE: an item of which kDenseEntries entries or more are left (a list without
 // a margin over D_MAX) takes one lane per entry, eight loads in flight at once:
 // the same order; 48 systems, list radius 1.2 = D_MAX: 759 us, in rounds 803.
 constexpr int kDenseEntries = 40;
+constexpr int kNoEntry = INT_MIN;  // "diagonal" of cluster 0, which is never staged in rounds
 // TWIN (rounds only): also the staged slot of each i atom's twin, the same atom in
 // the other group, for staged atoms that do not carry their requested index.
 // Returns the group bounds (uniform): n0 (0 or 8), [b1, b1+n1), [b2, b2+n2).
@@ -1852,7 +1853,7 @@ __device__ __forceinline__ void stage_item(const PairArgs& A, const Entry& my, i
                                            int& n1, int& b2, int& n2, Twin* T = nullptr) {
   static_assert(!(DENSE && TWIN), "twins are found in the rounds");
   bool pass = false;
-  const Entry none = {0, 1.0e5f, 1.0e5f, 1.0e5f};
+  const Entry none = {kNoEntry, 0.f, 0.f, 0.f};
   L.se[lane] = none;
   if (lane < sent_cap<CH>() - WAVE) L.se[WAVE + lane] = none;
   if (lane < CH && e0 + lane < e1 && (!VO || (my.code & kCountBit) || my.code < 0)) {
@@ -1949,7 +1950,7 @@ __device__ __forceinline__ void stage_item(const PairArgs& A, const Entry& my, i
     const float gx = fmaxf(fabsf(q.x - ic.x) - ih.x, 0.f);
     const float gy = fmaxf(fabsf(q.y - ic.y) - ih.y, 0.f);
     const float gz = fmaxf(fabsf(q.z - ic.z) - ih.z, 0.f);
-    const bool keep = fmaf(gz, gz, fmaf(gx, gx, gy * gy)) <= A.prune2;
+    const bool keep = e.code >= 0 && fmaf(gz, gz, fmaf(gx, gx, gy * gy)) <= A.prune2;
     const unsigned long long m = __ballot(keep);
     if (keep) L.sj[at + bits_below(m)] = q;
     if constexpr (TWIN) {
@@ -3033,7 +3034,7 @@ __device__ int staged_index(const PairArgs& A, const WaveLds& L, int p, int n0, 
   for (int r = 0; r < sent_cap<CH>() / CL; r++) {
     const Entry e = L.se[r * CL + (lane >> 3)];
     // the first round of the derivative-only entries starts at a multiple of 8
-    const bool deriv = __ballot((lane & 7) == 0 && e.dx < 1.0e5f && !(e.code & kCountBit)) != 0ull;
+    const bool deriv = __ballot((lane & 7) == 0 && e.code >= 0 && !(e.code & kCountBit)) != 0ull;
     if (deriv && first) {
       at = (at + CL - 1) & ~(CL - 1);
       first = false;
@@ -3046,7 +3047,7 @@ __device__ int staged_index(const PairArgs& A, const WaveLds& L, int p, int n0, 
     const float gx = fmaxf(fabsf(q.x - ic.x) - ih.x, 0.f);
     const float gy = fmaxf(fabsf(q.y - ic.y) - ih.y, 0.f);
     const float gz = fmaxf(fabsf(q.z - ic.z) - ih.z, 0.f);
-    const bool keep = fmaf(gz, gz, fmaf(gx, gx, gy * gy)) <= A.prune2;
+    const bool keep = e.code >= 0 && fmaf(gz, gz, fmaf(gx, gx, gy * gy)) <= A.prune2;
     const unsigned long long m = __ballot(keep);
     const int n = __popcll(m);
     if (p < at + n) {
