@@ -265,7 +265,9 @@ __device__ __forceinline__ void bin_atoms(int blk, int n, const double* __restri
     cy = max(cy, 0);
     col = S.colbase + cx + S.ncx * cy;
     info[i] = make_int4(m[0], m[1], m[2], col);
-    key[i] = sf[2];
+    // a coordinate that is not a number (or infinite) ranks as 0: a NaN key takes no
+    // place of its own in k_rank, and the slot left out would hold any index
+    key[i] = sf[2] >= 0.0 ? sf[2] : 0.0;
     am = max(abs(m[0]), max(abs(m[1]), abs(m[2])));
   }
   if (mmax) {
