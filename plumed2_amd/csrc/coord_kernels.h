@@ -1411,15 +1411,6 @@ __device__ __forceinline__ float sw_fixed_value_x(float x) {
   return __builtin_amdgcn_rcpf(fmaf(xp, x, 1.0f));
 }
 
-template <int P>
-__device__ __forceinline__ float sw_fixed_value(float invr0_2, float r2) {
-  const float x = r2 * invr0_2;
-  float xp = 1.0f;
-#pragma unroll
-  for (int k = 1; k < P; k++) xp *= x;
-  return __builtin_amdgcn_rcpf(fmaf(xp, x, 1.0f));
-}
-
 // band records a wave holds in LDS at once: the band pairs of an item are
 // decided in rounds of this many (one per lane)
 constexpr int kBandSlots = 64;

@@ -149,54 +149,27 @@ __device__ bool spline(const GridArg& G, const double* __restrict__ val, const d
   return true;
 }
 
-// Gaussian of one hill at the node point xx (MetaD.cpp:2244-2275, diagonal),
-// in two parts: the shape (scaled distances dp and exp(-dp^2/2); false
-// beyond the cutoff, where the hill adds nothing), and its value and
-// gradient for the height h.  gaussian() is the two together.
-// NCV > 0: that many CVs, known at compile time (the loops unroll and the
-// small arrays stay in registers); 0: G.ncv.  The arithmetic is the same.
-template <int NCV = 0>
-__device__ __forceinline__ bool gauss_shape(const GridArg& G, const double* xx, const double* c, double* dp,
-                                            double& e) {
-  const int ncv = NCV > 0 ? NCV : G.ncv;
-  double dp2 = 0.0;
+// Value and gradient (d) of one hill of height h at the node point xx
+// (MetaD.cpp:2244-2275, diagonal); 0 beyond the cutoff
+__device__ __forceinline__ double gaussian(const GridArg& G, const double* xx, const double* c, double h,
+                                           double* d) {
+  double dp[kMaxCv], dp2 = 0.0;
 #pragma unroll
-  for (int i = 0; i < (NCV > 0 ? NCV : kMaxCv); i++) {
-    if (i >= ncv) break;
+  for (int i = 0; i < kMaxCv; i++) {
+    if (i >= G.ncv) break;
+    d[i] = 0.0;
     dp[i] = vdiff(G, i, c[i], xx[i]) * G.invsigma[i];
     dp2 += dp[i] * dp[i];
   }
   dp2 *= 0.5;
-  e = 0.0;
-  if (!(dp2 < 6.25)) return false;
-  e = exp(-dp2);
-  return true;
-}
-
-template <int NCV = 0>
-__device__ __forceinline__ double gauss_apply(const GridArg& G, const double* dp, double e, double h, double* d) {
-  const int ncv = NCV > 0 ? NCV : G.ncv;
-  double bias = h * e;
+  if (!(dp2 < 6.25)) return 0.0;
+  const double bias = h * exp(-dp2);
 #pragma unroll
-  for (int i = 0; i < (NCV > 0 ? NCV : kMaxCv); i++) {
-    if (i >= ncv) break;
+  for (int i = 0; i < kMaxCv; i++) {
+    if (i >= G.ncv) break;
     d[i] = -bias * dp[i] * G.invsigma[i] * G.stretchA;
   }
-  bias = G.stretchA * bias + h * G.stretchB;
-  return bias;
-}
-
-template <int NCV = 0>
-__device__ __forceinline__ double gaussian(const GridArg& G, const double* xx, const double* c, double h,
-                                           double* d) {
-  double dp[kMaxCv], e;
-#pragma unroll
-  for (int i = 0; i < (NCV > 0 ? NCV : kMaxCv); i++) {
-    if (i >= (NCV > 0 ? NCV : G.ncv)) break;
-    d[i] = 0.0;
-  }
-  if (!gauss_shape<NCV>(G, xx, c, dp, e)) return 0.0;
-  return gauss_apply<NCV>(G, dp, e, h, d);
+  return G.stretchA * bias + h * G.stretchB;
 }
 
 // node of support offset `s` around the bin `ind` (GridBase::getNeighbors,
