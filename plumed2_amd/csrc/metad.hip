@@ -33,11 +33,14 @@
 #include "fp64_math.h"
 #include "p2a_internal.h"
 
-// The grid arithmetic follows the reference's FP64 operations one rounding at
-// a time: no fused multiply-add contraction.  It also makes every evaluation
-// of a hill's Gaussian round the same way wherever it is inlined, which the
-// run-wise deposition relies on (a corner's value for a height and the node's
-// value on the grid receive bit-identical additions).
+// No fused multiply-add but where fma() stands, so that every evaluation rounds
+// the same way wherever it is inlined: deposition in hill order relies on it (a
+// corner's value for a height and the node's value on the grid receive
+// bit-identical additions).  The spline and the hills of known heights follow the
+// reference's FP64 operations one rounding at a time; hills in order do not (a
+// product of one exponential per CV, fma() into the nodes, an exponential and a
+// reciprocal of their own, HillDim and corner_term): the same formulas in FP64,
+// a few roundings apart.
 #pragma clang fp contract(off)
 
 namespace p2a {
@@ -261,7 +264,8 @@ __device__ void add_hill_block(const GridArg& G, double* __restrict__ val, doubl
 __device__ __forceinline__ double wt_fast(double height0, double inv_wt, double inv_wt2, double vbias,
                                           const ExpK& C) {
   const double n = rint(vbias * -inv_wt2);
-  return exp_part(-vbias * inv_wt, n, C) * ldexp(height0, (int)n);
+  const double h = ldexp(height0, (int)n);
+  return fma(exp_part(-vbias * inv_wt, n, C), h, h);
 }
 // where wt_fast holds: finite heights of any run
 __device__ __forceinline__ bool wt_in_range(double inv_wt, double vbias) { return fabs(vbias * inv_wt) < 700.0; }

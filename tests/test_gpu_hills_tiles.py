@@ -62,3 +62,24 @@ def test_a_grid_of_more_tiles_than_a_launch_holds():
     at = c + rng.normal(0, 1.0e-7, c.shape)
     (b1, d1), (b2, d2) = m1.bias(at), m2.bias(at)
     assert np.any(b1 > 0.0) and np.array_equal(b1, b2) and np.array_equal(d1, d2)
+
+
+def test_the_gaussian_is_good_to_a_rounding(monkeypatch):
+    """One hill of height 1 at a node, arguments of the exponential exact: every
+    node within 1.1 units in the last place of exp (a final rounding of half a unit,
+    and two of a quarter in the reduced argument and the sum before it)."""
+    import plumed2_amd as P
+
+    monkeypatch.setenv("PLUMED_DP2CUTOFF_NOSTRETCH", "1")
+    m = P.MetaD("m: METAD ARG=a SIGMA=1 HEIGHT=1 PACE=1 GRID_MIN=-4 GRID_MAX=4 GRID_BIN=32768")
+    m.deposit(np.zeros((1, 1)))
+    v, d = m.grid()
+    x = -4.0 + np.arange(len(v)) / 4096.0
+    e = np.exp(-0.5 * x.astype(np.longdouble) ** 2)
+    near = 0.5 * x * x < 6.25
+    ulp = np.spacing(e.astype(np.float64))
+    assert not np.any(v[~near]) and np.count_nonzero(near) > 20000
+    assert float(np.max(np.abs((v - e) / ulp)[near])) <= 1.1
+    # the gradient: one rounding of the product more
+    g = -x * e
+    assert float(np.max(np.abs(d[:, 0] - g)[near])) <= 2.5 * np.spacing(1.0)
