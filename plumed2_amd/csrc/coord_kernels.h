@@ -798,8 +798,9 @@ struct ListArgs {
 // nine columns, 520 candidates for 190 entries) searched end after end.
 constexpr int kCandCap = 512;
 
-// t / n and t % n for 0 <= t < 2^31, r = 1/n to a few roundings: the quotient is
-// off by one at most
+// t / n and t % n for t >= 0 and a quotient below 2^22 (sys_columns bounds the
+// columns), r = 1/n to a few roundings: (float)t r is within three roundings of
+// the quotient, which is then off by one at most
 __device__ __forceinline__ int div_by(int t, int n, float r, int& rem) {
   int q = (int)((float)t * r);
   rem = t - q * n;
@@ -1225,7 +1226,8 @@ __global__ __launch_bounds__(256) void k_pack_bbox(Two<PackSide> T, const double
 }
 
 // The FP64 helpers below take the reference's rounding: no fused
-// multiply-add contraction (the reference's host build has none).
+// multiply-add contraction (the reference's host build has none).  (The sums of
+// the FP64 pair loops take fma() where it stands, pair64.)
 #pragma clang fp contract(off)
 
 // Tools::pbc (Tools.h:547-570)
@@ -2424,7 +2426,8 @@ __device__ __forceinline__ double pair64(const PbcArg& P, const p2a_switch& sw, 
   if (SWK > 0 && !(r2 <= sw.dmax_2)) return r2;
   double df;
   const double s = switch64<SWK>(sw, r2, df);
-  // CoordinationBase: deriv[p] -= df*d, deriv[q] += df*d
+  // CoordinationBase: deriv[p] -= df*d, deriv[q] += df*d (one rounding less than
+  // the reference's product and sum, as in the virial below)
   for (int k = 0; k < 3; k++) f[k] = fma(-df, d[k], f[k]);
   if (own) {
     const double g[3] = {df * d[0], df * d[1], df * d[2]};
@@ -2941,8 +2944,9 @@ inline void sys_columns(const double* box9, int n, SysArg& S) {
   double vol = std::fabs(w[0] * w[1] * w[2]);
   double rho = std::max(n, 1) / vol;
   double side = std::cbrt((double)CL / rho);
-  S.ncx = std::max(1, (int)std::floor(w[0] / side));
-  S.ncy = std::max(1, (int)std::floor(w[1] / side));
+  // (div_by: a window holds three times as many)
+  S.ncx = std::max(1, (int)std::min(std::floor(w[0] / side), 1048576.0));
+  S.ncy = std::max(1, (int)std::min(std::floor(w[1] / side), 1048576.0));
   // keep the column count bounded for very dilute groups
   while ((int64_t)S.ncx * S.ncy > 4 * (int64_t)n + 16) {
     S.ncx = std::max(1, S.ncx / 2);

@@ -251,7 +251,7 @@ class MetaD:
         return out
 
     def deposit(self, centers):
-        """Deposit many hills in sequence (one device launch); returns heights."""
+        """Deposit many hills in sequence; returns heights."""
         c = np.ascontiguousarray(np.asarray(centers, dtype=np.float64).reshape(-1, self.ncv))
         h = np.empty(len(c))
         A.check(A.lib().p2a_metad_deposit(self._ctx, len(c), c.ctypes.data, h.ctypes.data))
