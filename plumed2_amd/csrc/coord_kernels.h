@@ -3328,8 +3328,8 @@ inline int switch_known_kind(const p2a_switch& sw) {
 }
 
 // launch of the pair kernel for a switch, group mode and tuning.  TWOG: the
-// caller may have two groups that share atoms (else the kernels that compare
-// atom indices are not compiled); distinct groups run the kernels of one group.
+// caller may have two groups that share atoms, and calls for the value only (else
+// those kernels are not compiled); distinct groups run the kernels of one group.
 // The other switches have a kernel of their own for the default work items
 // (20,000 atoms with EXP: pair pass with derivatives 105 -> 62 us; value only,
 // 400,000 atoms, D_MAX 0.8: EXP 275 -> 137 us, TANH 472 -> 338); 32 entries an item
@@ -3348,26 +3348,24 @@ inline void launch_pairs(const PairArgs& A, const Two<PairSide>& T, hipStream_t 
 #define P2A_KSW(P, GEN)                                     \
   do {                                                      \
     if constexpr (TWOG) {                                   \
-      if (A.share) {                                        \
-        if (value_only) P2A_KCH(P, GEN, true, true);        \
-        else P2A_KCH(P, GEN, true, false);                  \
-        break;                                              \
-      }                                                     \
+      if (A.share && value_only) P2A_KCH(P, GEN, true, true);     \
+      else if (A.share) P2A_KCH(P, GEN, true, false);       \
+      else if (value_only) P2A_KCH(P, GEN, false, true);    \
+      else P2A_KCH(P, GEN, false, false);                   \
+    } else {                                                \
+      P2A_KCH(P, GEN, false, false);                        \
     }                                                       \
-    if (value_only) P2A_KCH(P, GEN, false, true);           \
-    else P2A_KCH(P, GEN, false, false);                     \
   } while (0)
 #define P2A_KKN(K)                                              \
   case K:                                                       \
     if constexpr (TWOG) {                                       \
-      if (A.share) {                                            \
-        if (value_only) P2A_K(K, true, true, true, 64);         \
-        else P2A_K(K, true, true, false, 64);                   \
-        break;                                                  \
-      }                                                         \
+      if (A.share && value_only) P2A_K(K, true, true, true, 64);      \
+      else if (A.share) P2A_K(K, true, true, false, 64);        \
+      else if (value_only) P2A_K(K, true, false, true, 64);     \
+      else P2A_K(K, true, false, false, 64);                    \
+    } else {                                                    \
+      P2A_K(K, true, false, false, 64);                         \
     }                                                           \
-    if (value_only) P2A_K(K, true, false, true, 64);            \
-    else P2A_K(K, true, false, false, 64);                      \
     break
   if (sw.type == P2A_SW_RATIONAL_FIXED) {
     switch (sw.nn / 2) {
