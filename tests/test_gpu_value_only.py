@@ -1,7 +1,8 @@
 """Value-only calls (no derivatives asked for) under every switch, groups apart
 and groups that share atoms, against the FP64 oracle: values to 1e-6 as for the
 calls with derivatives (FP64 terms rounded to FP32, FP64 sums), pair counts
-equal; and such a call takes no longer than one with derivatives."""
+equal; and such a call takes no longer than one with derivatives (5% for the
+clock)."""
 import numpy as np
 import pytest
 
@@ -49,4 +50,4 @@ def test_no_slower_than_with_derivatives(sw):
     act.set_stream(torch.cuda.current_stream().cuda_stream)
     full = _time(lambda: act.calculate_torch(x, box, 0))
     alone = _time(lambda: act.calculate_device(x.data_ptr(), box, 0, v.data_ptr(), 0, 0))
-    assert alone <= full, (alone, full)
+    assert alone <= 1.05 * full, (alone, full)
